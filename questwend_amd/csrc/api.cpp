@@ -125,31 +125,34 @@ qw::MmidArgs mmid_args(int type, const void* as, int64_t K, int64_t N, int64_t n
     return m;
 }
 
-// The exact Q4_K matrix-core form on the f16 matrix cores: an f16 copy of the
-// n_rows activation rows in act_q, in the call's workspace.  Without room for it
-// the int8 form runs (the same bits).
-// QWMOE_MFMA_F16=0 in the environment keeps the int8 form (a test switch).
-int mfma_f16_prep(Arena& ar, qw::MmidArgs& m, int64_t n_rows, hipStream_t st) {
-    if (!qw::mmid_mfma_h_ok(m, n_rows)) return 0;
+// The f16 copy of the n_rows activation rows in act_q that the f16 matrix cores
+// read (the exact Q4_K form, and Q8_0), in the call's workspace: reserved and
+// attached to m, nothing launched (act_h, and for Q8_0 act_hd, go to the launch
+// that quantizes the rows, or to mfma_f16_prep's).  Without room for it the int8
+// matrix cores (Q4_K) or the GEMV (Q8_0) run, with the same bits.
+// QWMOE_MFMA_F16=0 in the environment keeps those (a test switch).
+bool mfma_f16_reserve(Arena& ar, qw::MmidArgs& m, int64_t n_rows) {
+    if (!qw::mmid_mfma_h_ok(m, n_rows)) return false;
     const char* env = getenv("QWMOE_MFMA_F16");
-    if (env && env[0] == '0') return 0;
-    uint16_t* h = ar.take<uint16_t>((size_t) (n_rows * m.K));
-    if (!h) return 0;
-    if (int rc = qw::launch_q8K_to_f16(m.act_q, m.act_row_bytes, m.K, n_rows, h, st)) return rc == -2 ? 0 : rc;
+    if (env && env[0] == '0') return false;
+    const bool q80 = m.type == qw::T_Q8_0;
+    uint16_t* h = ar.take<uint16_t>((size_t) (n_rows * (m.K + (q80 ? m.K / 16 : 0))));   // (K / 32 f32 scales per row)
     m.act_h = h;
-    return 0;
+    m.act_hd = h && q80 ? (const float*) (h + n_rows * m.K) : nullptr;
+    return h != nullptr;
 }
 
-// The same copy, written by the launch that quantizes the rows (the returned
-// buffer goes to launch_quantize_act / launch_swiglu_q8K as h_out): reserved
-// and attached to m, nothing launched; null where the f16 form does not apply.
-uint16_t* mfma_f16_reserve(Arena& ar, qw::MmidArgs& m, int64_t n_rows) {
-    if (!qw::mmid_mfma_h_ok(m, n_rows)) return nullptr;
-    const char* env = getenv("QWMOE_MFMA_F16");
-    if (env && env[0] == '0') return nullptr;
-    uint16_t* h = ar.take<uint16_t>((size_t) (n_rows * m.K));
-    m.act_h = h;
-    return h;
+// The same, and the copy made from the quantized rows by a launch of its own.
+int mfma_f16_prep(Arena& ar, qw::MmidArgs& m, int64_t n_rows, hipStream_t st) {
+    if (!mfma_f16_reserve(ar, m, n_rows)) return 0;
+    const int rc = m.type == qw::T_Q8_0
+                       ? qw::launch_q80_to_f16(m.act_q, m.K, n_rows, (uint16_t*) m.act_h, (float*) m.act_hd, st)
+                       : qw::launch_q8K_to_f16(m.act_q, m.act_row_bytes, m.K, n_rows, (uint16_t*) m.act_h, st);
+    if (rc) {
+        m.act_h = nullptr;
+        m.act_hd = nullptr;
+    }
+    return rc == -2 ? 0 : rc;
 }
 
 // Gate and up reading one activation buffer share its f16 copy.
@@ -158,12 +161,21 @@ int mfma_f16_prep_pair(Arena& ar, qw::MmidArgs& mu, qw::MmidArgs& mg, int64_t n_
     if (mg.act_q == mu.act_q && mg.act_row_bytes == mu.act_row_bytes && mg.K == mu.K &&
         qw::mmid_mfma_h_ok(mg, n_rows)) {
         mg.act_h = mu.act_h;
+        mg.act_hd = mu.act_hd;
         return 0;
     }
     return mfma_f16_prep(ar, mg, n_rows, st);
 }
 
-int mmid_launch(const qw::MmidArgs& m, hipStream_t st) {
+// Q8_0 runs on the matrix cores only with its f16 copy: without it every bin is the GEMV's.
+qw::MmidArgs mfma_bins(const qw::MmidArgs& m) {
+    qw::MmidArgs c = m;
+    if (c.type == qw::T_Q8_0 && !c.act_h) c.mfma_min_rows = 0;
+    return c;
+}
+
+int mmid_launch(const qw::MmidArgs& m_, hipStream_t st) {
+    const qw::MmidArgs m = mfma_bins(m_);
     // with mfma_min_rows == 1 the matrix cores take every bin that holds a row:
     // the GEMV's workgroups would only return
     int rc = m.mfma_min_rows == 1 ? 0 : qw::launch_mmid_gemv(m, st);
@@ -173,7 +185,8 @@ int mmid_launch(const qw::MmidArgs& m, hipStream_t st) {
 
 // Gate and up of a layer (same type, shape and grouping): one GEMV launch and
 // one matrix-core launch for both, else each on its own.
-int mmid_launch_pair(const qw::MmidArgs& mu, const qw::MmidArgs& mg, hipStream_t st) {
+int mmid_launch_pair(const qw::MmidArgs& mu_, const qw::MmidArgs& mg_, hipStream_t st) {
+    const qw::MmidArgs mu = mfma_bins(mu_), mg = mfma_bins(mg_);
     const bool same = mu.type == mg.type && mu.K == mg.K && mu.N == mg.N && mu.mfma_min_rows == mg.mfma_min_rows &&
                       mu.mfma_exact == mg.mfma_exact;
     if (same) {
@@ -529,7 +542,6 @@ int qwmoe_shared_expert_add(void* stream, const qwmoe_shared_expert* se, int64_t
     int32_t* n_active = ar.take<int32_t>(1);
     float* upo = ar.take<float>((size_t) (F * T));
     float* gateo = ar.take<float>((size_t) (F * T));
-    float* act = ar.take<float>((size_t) (F * T));
     float* sh = ar.take<float>((size_t) (H * T));
     const int vg = qw::vec_dot_type(se->type_gate), vu = qw::vec_dot_type(se->type_up);
     const int vd = qw::vec_dot_type(se->type_down);
@@ -537,7 +549,7 @@ int qwmoe_shared_expert_add(void* stream, const qwmoe_shared_expert* se, int64_t
     uint8_t* xg = ar.take<uint8_t>(qg * (size_t) T + 64);
     uint8_t* xu = (vu == vg) ? xg : ar.take<uint8_t>(qu * (size_t) T + 64);
     uint8_t* aq = ar.take<uint8_t>(qd * (size_t) T + 64);
-    if (!rows || !active || !active_off || !n_active || !upo || !gateo || !act || !sh || !xg || !xu || !aq)
+    if (!rows || !active || !active_off || !n_active || !upo || !gateo || !sh || !xg || !xu || !aq)
         return QWMOE_ERR_WORKSPACE;
     if ((rc = qw::launch_group_dense(rows, active, active_off, n_active, T, st))) return rc;
     if ((rc = qw::launch_quantize_act(vg, x, H, 1, T, (size_t) H * 4, (size_t) H * 4, xg, st))) return rc;
@@ -556,15 +568,14 @@ int qwmoe_shared_expert_add(void* stream, const qwmoe_shared_expert* se, int64_t
     md.swiglu_up = upo;
     if (vd == qw::T_Q8_K && qw::mmid_gemv_swiglu_ok(md)) {
         // the down GEMV forms SwiGLU's Q8_K rows itself
-    } else if (vd == qw::T_Q8_K) {
-        md.swiglu_gate = md.swiglu_up = nullptr;
-        if ((rc = qw::launch_swiglu_q8K(gateo, upo, F, T, aq, st))) return rc;
     } else {
         md.swiglu_gate = md.swiglu_up = nullptr;
-        if ((rc = qw::launch_swiglu(gateo, upo, act, T, F, fb, fb, fb, st))) return rc;
-        if ((rc = qw::launch_quantize_act(vd, act, F, 1, T, fb, fb, aq, st))) return rc;
+        mfma_f16_reserve(ar, md, T);
+        uint16_t* ha = (uint16_t*) md.act_h;
+        if ((rc = vd == qw::T_Q8_K ? qw::launch_swiglu_q8K(gateo, upo, F, T, aq, st, ha)
+                                   : qw::launch_swiglu_q80(gateo, upo, F, T, aq, st, ha, (float*) md.act_hd)))
+            return rc;
     }
-    if (!md.swiglu_gate && (rc = mfma_f16_prep(ar, md, T, st))) return rc;
     if ((rc = mmid_launch(md, st))) return rc;
     return qw::launch_shared_gate_add(x, (size_t) H, se->gate_inp, sh, moe_out, resid, out, (size_t) H, H, T, st);
 }
@@ -878,9 +889,8 @@ int qwmoe_ffn_layer(void* stream, const qwmoe_layer* L, const float* x, int64_t 
     float* logits = ar.take<float>((size_t) (E * T));
     float* upo = ar.take<float>((size_t) (F * k * T));
     float* gateo = ar.take<float>((size_t) (F * k * T));
-    float* act = ar.take<float>((size_t) (F * k * T));
     float* ex = ar.take<float>((size_t) (H * k * T));
-    if (!ids || !w || !logits || !upo || !gateo || !act || !ex) return QWMOE_ERR_WORKSPACE;
+    if (!ids || !w || !logits || !upo || !gateo || !ex) return QWMOE_ERR_WORKSPACE;
     // router
     qw::RouterArgs ra{};
     ra.W = L->router;
@@ -928,26 +938,31 @@ int qwmoe_ffn_layer(void* stream, const qwmoe_layer* L, const float* x, int64_t 
     qw::MmidArgs mg = mmid_args(L->type_gate, L->gate, H, F, L->n_slots_gate, L->gate_nb1, L->gate_nb2, xg, 1, qg,
                                       G.rows, G.active, G.active_off, G.n_active, G.max_active, L->slot_gate,
                                       L->slot_gate ? E : 0, gateo, dnb1, dnb2, T, k * T);
-    // x's f16 copy for the exact matrix-core form, written by the quantizing launch
+    const int vd = qw::vec_dot_type(L->type_down);
+    const size_t qd = qwmoe_row_size(vd, F);
+    uint8_t* aq = ar.take<uint8_t>(qd * (size_t) (k * T) + 64);   // (before the copies, which a call can do without)
+    if (!aq) return QWMOE_ERR_WORKSPACE;
+    // x's f16 copy for the matrix-core forms, written by the quantizing launch
     // (gate and up share it when they read one buffer)
     uint16_t* hx = nullptr;
-    if (!xq_fused && xu == xg && vg == qw::T_Q8_K) {
-        hx = mfma_f16_reserve(ar, mu, T);
-        if (hx && qw::mmid_mfma_h_ok(mg, T)) mg.act_h = hx;
-        else if (hx) {
+    float* hxd = nullptr;
+    if (!xq_fused && xu == xg && mfma_f16_reserve(ar, mu, T)) {
+        if (L->type_gate == L->type_up && qw::mmid_mfma_h_ok(mg, T)) {
+            mg.act_h = mu.act_h;
+            mg.act_hd = mu.act_hd;
+            hx = (uint16_t*) mu.act_h;
+            hxd = (float*) mu.act_hd;
+        } else {
             mu.act_h = nullptr;
-            hx = nullptr;
+            mu.act_hd = nullptr;
         }
     }
-    if (!xq_fused && (rc = qw::launch_quantize_act(vg, x, H, 1, T, (size_t) H * 4, (size_t) H * 4, xg, st, hx)))
+    if (!xq_fused &&
+        (rc = qw::launch_quantize_act(vg, x, H, 1, T, (size_t) H * 4, (size_t) H * 4, xg, st, hx, hxd)))
         return rc;
     if (xu != xg && (rc = qw::launch_quantize_act(vu, x, H, 1, T, (size_t) H * 4, (size_t) H * 4, xu, st))) return rc;
     if (!hx && (rc = mfma_f16_prep_pair(ar, mu, mg, T, st))) return rc;
     if ((rc = mmid_launch_pair(mu, mg, st))) return rc;   // gate and up in one launch each
-    const int vd = qw::vec_dot_type(L->type_down);
-    const size_t qd = qwmoe_row_size(vd, F);
-    uint8_t* aq = ar.take<uint8_t>(qd * (size_t) (k * T) + 64);
-    if (!aq) return QWMOE_ERR_WORKSPACE;
     qw::MmidArgs md = mmid_args(L->type_down, L->down, F, H, L->n_slots_down, L->down_nb1, L->down_nb2, aq, k, qd,
                                 G.rows, G.active, G.active_off, G.n_active, G.max_active, L->slot_down,
                                 L->slot_down ? E : 0, ex, (size_t) H * 4, (size_t) H * 4 * (size_t) k, T, k * T, true);
@@ -955,18 +970,14 @@ int qwmoe_ffn_layer(void* stream, const qwmoe_layer* L, const float* x, int64_t 
     md.swiglu_up = upo;
     if (vd == qw::T_Q8_K && qw::mmid_gemv_swiglu_ok(md)) {
         // small bins: the down GEMV forms SwiGLU's Q8_K rows itself
-    } else if (vd == qw::T_Q8_K) {   // SwiGLU straight into Q8_K (and the f16 copy the matrix cores read)
+    } else {   // SwiGLU straight into the quantized rows (and the f16 copy the matrix cores read)
         md.swiglu_gate = md.swiglu_up = nullptr;
-        uint16_t* ha = mfma_f16_reserve(ar, md, k * T);
-        if ((rc = qw::launch_swiglu_q8K(gateo, upo, F, k * T, aq, st, ha))) return rc;
-    } else {
-        md.swiglu_gate = md.swiglu_up = nullptr;
-        if ((rc = qw::launch_swiglu(gateo, upo, act, k * T, F, (size_t) F * 4, (size_t) F * 4, (size_t) F * 4, st)))
-            return rc;
-        if ((rc = qw::launch_quantize_act(vd, act, F, k, k * T, (size_t) F * 4, (size_t) F * 4 * (size_t) k, aq, st)))
+        mfma_f16_reserve(ar, md, k * T);
+        uint16_t* ha = (uint16_t*) md.act_h;
+        if ((rc = vd == qw::T_Q8_K ? qw::launch_swiglu_q8K(gateo, upo, F, k * T, aq, st, ha)
+                                   : qw::launch_swiglu_q80(gateo, upo, F, k * T, aq, st, ha, (float*) md.act_hd)))
             return rc;
     }
-    if (!md.swiglu_gate && !md.act_h && (rc = mfma_f16_prep(ar, md, k * T, st))) return rc;
     if ((rc = mmid_launch(md, st))) return rc;
     if (rms_eps >= 0.0f && H <= 16384) {
         if ((rc = qw::launch_weighted_sum_rms(ex, w, out, x_next, H, k, T, rms_eps, st))) return rc;

@@ -807,6 +807,8 @@ static int launch_gemv(const MmidPair& pr, int nz, hipStream_t stream) {
         if (!mmid_gemv_swiglu_ok(m) || (nz == 2 && !mmid_gemv_swiglu_ok(pr.m[1]))) return -2;
     }
     if (const size_t bp = gemv_bp_lds(m, gemv_bp_direct(pr, nz))) return launch_gemv_bp(pr, nz, bp, stream);
+    if (m.type == T_Q8_0)
+        if (const int rc = launch_gemv_q80(pr.m, nz, stream); rc != -2) return rc;
     const size_t row_bytes = (size_t) (m.K / block_elems(m.type)) * block_bytes(m.type);
     size_t lds_bytes = (size_t) mmid_slot_bytes(row_bytes) * MMID_ROWS +
                        (size_t) mmid_stage_rows(m.max_rows) * (((m.act_row_bytes + 3) / 4) * 4 + 16);

@@ -27,16 +27,12 @@
 // v_mfma_i32_16x16x64_i8 over the 64 positions of sub-blocks 2m and 2m+1 with
 // every A byte equal to that sub-block's min.  20 MFMAs per 16 x 16 tile and
 // super-block.
-#include "qw_kernels.hpp"
+#include "qw_mfma.hpp"
 
 #include <type_traits>
 
 namespace qw {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4m __attribute__((ext_vector_type(4)));
-
-constexpr int MF_M = 64;          // weight rows per workgroup (4 waves x 16)
 constexpr uint32_t MF_WS = 144;   // LDS stride of a staged Q4_K block (9 x 16 B)
 constexpr uint32_t MF_AS = 276;   // LDS stride of a staged Q8_K block (69 dwords): d at 0, qs at 16
                                   // (an odd dword stride: 16 or 32 lanes reading one offset of their
@@ -49,43 +45,6 @@ constexpr int MF_NB_B = 4;        // block-sum form
 __device__ __forceinline__ v4i lds_v4i(const uint8_t* p) {
     const uint32_t* q = (const uint32_t*) p;
     return v4i{(int) q[0], (int) q[1], (int) q[2], (int) q[3]};
-}
-
-// Waits until at most N of this wave's vector memory operations are in flight.
-template <int N>
-__device__ __forceinline__ void vm_wait() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// Buffer resource words over [base, base + bytes) (the layout
-// __builtin_amdgcn_make_buffer_rsrc builds; loads past the end return zeros).
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ i32x4 rsrc_words(const void* base, uint32_t bytes) {
-    const uint64_t a = (uint64_t) base;
-    return i32x4{(int) (uint32_t) a, (int) ((uint32_t) (a >> 32) & 0xffffu), (int) bytes, 0x00020000};
-}
-
-// Buffer loads straight into LDS: lane l's 16 (4) bytes from voff + soff land at
-// LDS byte lds_base + 16 l (4 l).  Written as instructions, not through the
-// compiler's builtin: the compiler then inserts no wait of its own before the
-// LDS reads (it would wait for every copy in flight, the prefetched stages
-// included); the kernel waits with vm_wait and orders waves with a barrier.
-// M0 holds the LDS base for the instruction and is restored after it.
-__device__ __forceinline__ void dma_b128(i32x4 rsrc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
-    uint32_t keep;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff)
-        : "memory");
-}
-__device__ __forceinline__ void dma_b32(i32x4 rsrc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
-    uint32_t keep;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dword %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff)
-        : "memory");
 }
 
 __device__ __forceinline__ long pack2(uint32_t lo, uint32_t hi) { return (long) (((uint64_t) hi << 32) | lo); }
@@ -103,63 +62,6 @@ __device__ __forceinline__ uint32_t mul_bytes(uint32_t b, uint32_t s) {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short) 0, (int) bytes, 0x00020000);
 }
-
-// Work items: the routed rows of each heavy expert (at least mfma_min_rows)
-// cut into chunks of R rows; item i is chunk c of active expert g, items in
-// expert order.  Wave 0 scans the active experts' chunk counts 64 at a time and
-// leaves (g, c) in s_item, g = -1 past the last item.  Splitting an expert's
-// rows over workgroups keeps the longest workgroup at R rows whatever the skew
-// of the routing (one expert can hold every token of the batch).
-__device__ __forceinline__ void mf_item(const MmidArgs& m, int item, int R, int wave, int lane, int* s_item) {
-    if (wave == 0) {
-        const int n = *m.n_active;
-        int run = 0, fg = -1, fc = 0;
-        for (int base = 0; base < n; base += 64) {
-            const int j = base + lane;
-            int ch = 0;
-            if (j < n) {
-                const int cnt = m.active_off[j + 1] - m.active_off[j];
-                ch = cnt >= m.mfma_min_rows ? (cnt + R - 1) / R : 0;
-            }
-            int incl = ch;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(incl, o);
-                if (lane >= o) incl += v;
-            }
-            const int excl = incl - ch;
-            const uint64_t hit = __ballot(item >= run + excl && item < run + incl);
-            if (hit) {   // uniform
-                const int src = __ffsll((unsigned long long) hit) - 1;
-                fg = base + src;
-                fc = item - run - __shfl(excl, src);
-                break;
-            }
-            run += __shfl(incl, 63);
-        }
-        if (lane == 0) {
-            s_item[0] = fg;
-            s_item[1] = fc;
-        }
-    }
-    __syncthreads();
-}
-
-// Upper bound on the items of a launch: at most min(max_active, n_pairs /
-// mfma_min_rows) heavy experts, each with at most one partial chunk.
-inline int64_t mf_max_items(const MmidArgs& m, int R) {
-    const int64_t heavy = std::min<int64_t>(m.max_active, m.n_pairs / std::max(m.mfma_min_rows, 1));
-    return heavy + m.n_pairs / R;
-}
-
-// One launch runs the matrix-core part of one mul_mat_id, or of two of the same
-// type, shape and grouping (gate and up of an FFN): workgroups [0, groups) take
-// m[0], [groups, 2 groups) m[1], so the second matrix's workgroups fill the CUs
-// the first one's last round leaves idle.
-struct MfLaunch {
-    MmidArgs m[2];
-    uint32_t groups;   // workgroups per matrix
-};
 
 // Workgroup b = (work item, row tile): weight rows r0 .. r0 + 63 of the expert's
 // matrix against one pass of 16 NB routed activation rows (the item).  Items
@@ -1597,9 +1499,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
 }
 
 // Whether a matrix-core kernel can take (type, form, shape, strides): Q4_K rows
-// of 16-byte aligned super-blocks, or Q6_K rows on 4-byte aligned tensors;
+// of 16-byte aligned super-blocks, Q6_K rows on 4-byte aligned tensors, or Q8_0
+// rows of 16-byte aligned groups of eight blocks (and the f16 copy: act_h);
 // 64-row tiles, 16-byte aligned output rows.
 bool mmid_mfma_supported(const MmidArgs& m) {
+    if (m.type == T_Q8_0) return mf_q80_supported(m);
     const bool q4 = m.type == T_Q4_K && m.nb1 % 16 == 0 && m.nb2 % 16 == 0 && ((uintptr_t) m.w & 15) == 0;
     const bool q6 = m.type == T_Q6_K && m.nb1 % 2 == 0 && m.nb2 % 4 == 0 && ((uintptr_t) m.w & 3) == 0 &&
                     (uint64_t) M6_M * m.nb1 + 64ull * m.nb1 < (1ull << 31);
@@ -1607,9 +1511,12 @@ bool mmid_mfma_supported(const MmidArgs& m) {
            ((uintptr_t) m.dst & 15) == 0 && m.act_row_bytes % 4 == 0 && ((uintptr_t) m.act_q & 3) == 0;
 }
 
-// Whether the exact Q4_K form can run on the f16 matrix cores (act_h set from
-// launch_q8K_to_f16 over all n_rows activation rows).
+// Whether the exact Q4_K form can run on the f16 matrix cores, or the Q8_0 form at
+// all (act_h set from an f16 copy of all n_rows activation rows).
 bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows) {
+    if (m.type == T_Q8_0)
+        return m.mfma_min_rows > 0 && mmid_mfma_supported(m) && n_rows > 0 &&
+               (uint64_t) n_rows * (uint64_t) m.K * 2u + 512u < (1ull << 31);
     return m.type == T_Q4_K && m.mfma_exact && m.mfma_min_rows > 0 && mmid_mfma_supported(m) && n_rows > 0 &&
            (uint64_t) n_rows * (uint64_t) m.K * 2u + 512u < (1ull << 31);
 }
@@ -1650,6 +1557,7 @@ static unsigned mp_grid() {
 static int launch_mf(const MfLaunch& lp, int nz, hipStream_t stream) {
     const MmidArgs& m = lp.m[0];
     if (lp.groups == 0) return 0;
+    if (m.type == T_Q8_0) return launch_mf_q80(lp, nz, stream);
     if (mp_ok(lp, nz)) {
         // at most (items of 32 rows) x tiles x nz units: no more workgroups than that
         const int64_t units = mf_max_items(m, MP_NR) * (m.N / MF_M) * nz;
@@ -1670,6 +1578,7 @@ static int launch_mf(const MfLaunch& lp, int nz, hipStream_t stream) {
 
 // Workgroups of one matrix: (work item, row tile) pairs.
 static int64_t mf_groups(const MmidArgs& m) {
+    if (m.type == T_Q8_0) return mf_q80_groups(m);
     const bool q6b = m.type == T_Q6_K && !m.mfma_exact;
     const int rows = q6b ? M6_N
                          : 16 * (m.type == T_Q6_K ? MX_NB : !m.mfma_exact ? MF_NB_B : m.act_h ? MH_NB : MF_NB_X);

@@ -60,19 +60,10 @@ int launch_swiglu_q8K(const float* gate, const float* up, int64_t F, int64_t n_r
 }
 
 // Activation Q8_0 (x86 AVX2 branch): one 32-value block per 8 lanes, 4 per lane.
-__global__ void __launch_bounds__(256) k_quant_q8_0_act(const float* __restrict__ src, int64_t K, int64_t ne1,
-                                                        int64_t nrows, size_t nb1, size_t nb2,
-                                                        BlockQ8_0* __restrict__ dst) {
-    const int64_t nb = K / QK8_0;
-    const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t blk = gid >> 3;
-    const int sub = threadIdx.x & 7;
-    const bool valid = blk < nb * nrows;
-    const int64_t b = valid ? blk : 0;
-    const int64_t row = b / nb, ib = b % nb;
-    const int64_t i1 = row % ne1, i2 = row / ne1;
-    const float* x = (const float*) ((const char*) src + i1 * nb1 + i2 * nb2) + ib * QK8_0;
-    float4 q = *(const float4*) (x + 4 * sub);
+// With h set, each lane also writes its four quants as f16 and the block's d as
+// f32 in launch_q80_to_f16's layout.
+__device__ __forceinline__ void quant_q80_lane8(const float4 q, bool valid, int64_t blk, int sub, BlockQ8_0* dst,
+                                                _Float16* h, float* hd) {
     float m = fmaxf(fmaxf(__builtin_fabsf(q.x), __builtin_fabsf(q.y)), fmaxf(__builtin_fabsf(q.z), __builtin_fabsf(q.w)));
     m = fmaxf(m, __shfl_xor(m, 1));
     m = fmaxf(m, __shfl_xor(m, 2));
@@ -89,12 +80,61 @@ __global__ void __launch_bounds__(256) k_quant_q8_0_act(const float* __restrict_
     uint16_t* qs16 = (uint16_t*) ((char*) y + 2 + 4 * sub);
     qs16[0] = (uint16_t) (packed & 0xffff);
     qs16[1] = (uint16_t) (packed >> 16);
-    if (sub == 0) y->d = f2h(d);
+    const uint16_t dh = f2h(d);
+    if (sub == 0) y->d = dh;
+    if (h) {
+        typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+        auto b = [&](int k) { return (_Float16) (float) (int8_t) (packed >> (8 * k)); };
+        *(h4v*) (h + 32 * (size_t) blk + 8 * (sub & 3) + 4 * (sub >> 2)) = h4v{b(0), b(1), b(2), b(3)};
+        if (sub == 0) hd[blk] = h2f(dh);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_quant_q8_0_act(const float* __restrict__ src, int64_t K, int64_t ne1,
+                                                        int64_t nrows, size_t nb1, size_t nb2,
+                                                        BlockQ8_0* __restrict__ dst, _Float16* __restrict__ h,
+                                                        float* __restrict__ hd) {
+    const int64_t nb = K / QK8_0;
+    const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t blk = gid >> 3;
+    const int sub = threadIdx.x & 7;
+    const bool valid = blk < nb * nrows;
+    const int64_t b = valid ? blk : 0;
+    const int64_t row = b / nb, ib = b % nb;
+    const int64_t i1 = row % ne1, i2 = row / ne1;
+    const float* x = (const float*) ((const char*) src + i1 * nb1 + i2 * nb2) + ib * QK8_0;
+    quant_q80_lane8(*(const float4*) (x + 4 * sub), valid, blk, sub, dst, h, hd);
+}
+
+// SwiGLU of dense rows straight into Q8_0 (k_swiglu's values, k_quant_q8_0_act's
+// quantizer), without the fp32 round trip and its launch.
+__global__ void __launch_bounds__(256) k_swiglu_q80(const float* __restrict__ gate, const float* __restrict__ up,
+                                                    int64_t nblk, BlockQ8_0* __restrict__ dst,
+                                                    _Float16* __restrict__ h, float* __restrict__ hd) {
+    const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t blk = gid >> 3;
+    const int sub = threadIdx.x & 7;
+    const bool valid = blk < nblk;
+    const int64_t off = QK8_0 * (valid ? blk : 0) + 4 * sub;
+    const float4 g = *(const float4*) (gate + off);
+    const float4 u = *(const float4*) (up + off);
+    quant_q80_lane8(float4{v_silu(g.x) * u.x, v_silu(g.y) * u.y, v_silu(g.z) * u.z, v_silu(g.w) * u.w}, valid, blk, sub,
+                    dst, h, hd);
+}
+
+int launch_swiglu_q80(const float* gate, const float* up, int64_t F, int64_t n_rows, void* dst, hipStream_t stream,
+                      uint16_t* h_out, float* hd_out) {
+    if (F % QK8_0 || (((uintptr_t) gate | (uintptr_t) up) & 15) || !h_out != !hd_out) return -2;
+    const int64_t nblk = (F / QK8_0) * n_rows;
+    if (nblk == 0) return 0;
+    hipLaunchKernelGGL(k_swiglu_q80, dim3((unsigned) ((8 * nblk + 255) / 256)), dim3(256), 0, stream, gate, up, nblk,
+                       (BlockQ8_0*) dst, (_Float16*) h_out, hd_out);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 int launch_quantize_act(int vdt, const float* src, int64_t K, int64_t ne1, int64_t nrows, size_t nb1, size_t nb2,
-                        void* dst, hipStream_t stream, uint16_t* h_out) {
-    if (h_out && vdt != T_Q8_K) return -2;
+                        void* dst, hipStream_t stream, uint16_t* h_out, float* hd_out) {
+    if (h_out && vdt == T_Q8_0 && !hd_out) return -2;
     if (vdt == T_Q8_K) {
         const int64_t nblk = (K / QK_K) * nrows;
         if (nblk == 0) return 0;
@@ -104,7 +144,7 @@ int launch_quantize_act(int vdt, const float* src, int64_t K, int64_t ne1, int64
         const int64_t nthr = (K / QK8_0) * nrows * 8;
         if (nthr == 0) return 0;
         hipLaunchKernelGGL(k_quant_q8_0_act, dim3((unsigned) ((nthr + 255) / 256)), dim3(256), 0, stream, src, K, ne1,
-                           nrows, nb1, nb2, (BlockQ8_0*) dst);
+                           nrows, nb1, nb2, (BlockQ8_0*) dst, (_Float16*) h_out, hd_out);
     } else {
         return -1;
     }

@@ -8,10 +8,10 @@
 namespace qw {
 
 // quantize.hip
-// h_out (optional, Q8_K only): the f16 copy the exact Q4_K matrix-core form reads
-// (launch_q8K_to_f16's layout), written by the same launch
+// h_out (optional): the f16 copy the matrix-core forms read, written by the same
+// launch: Q8_K launch_q8K_to_f16's layout; Q8_0 launch_q80_to_f16's, with hd_out
 int launch_quantize_act(int vdt, const float* src, int64_t K, int64_t ne1, int64_t nrows, size_t nb1, size_t nb2,
-                        void* dst, hipStream_t stream, uint16_t* h_out = nullptr);
+                        void* dst, hipStream_t stream, uint16_t* h_out = nullptr, float* hd_out = nullptr);
 int launch_quantize_weights(int type, const float* src, int64_t n, void* dst, hipStream_t stream);
 int launch_dequantize(int type, const void* x, float* y, int64_t n, hipStream_t stream);
 int launch_randn(float* y, int64_t n, uint64_t seed, float mean, float stddev, hipStream_t stream);
@@ -91,9 +91,15 @@ struct MmidArgs {
     const float* swiglu_up;
     // optional (exact Q4_K matrix-core form): the f16 copy of act_q's quants made by
     // launch_q8K_to_f16; with it the exact form runs on the f16 matrix cores (the same bits)
+    // (Q8_0: the copy of launch_quantize_act / launch_swiglu_q80 / launch_q80_to_f16, which
+    // the Q8_0 matrix-core form needs, and act_hd the row blocks' d as f32 [row][K / 32])
     const uint16_t* act_h;
+    const float* act_hd;
 };
 int launch_mmid_gemv(const MmidArgs& m, hipStream_t stream);
+// mmid_q80.hip: one or two Q8_0 GEMVs on the kernel that copies whole rows straight
+// into LDS; -2 where it does not apply (launch_mmid_gemv then runs k_mmid_gemv)
+int launch_gemv_q80(const MmidArgs* m, int nz, hipStream_t stream);
 // whether launch_mmid_gemv forms the activations itself for these arguments with
 // swiglu_gate / swiglu_up set (small bins on the block-parallel kernel)
 bool mmid_gemv_swiglu_ok(const MmidArgs& m);
@@ -111,6 +117,11 @@ int launch_mmid_mfma2(const MmidArgs& a, const MmidArgs& b, hipStream_t stream);
 int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t n_rows, uint16_t* out, hipStream_t stream);
 // whether m (with act_q holding n_rows rows) can take such a copy as act_h
 bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows);
+
+// The f16 copy the Q8_0 matrix-core form reads, of n_rows dense Q8_0 rows of K
+// values: per 32-value block four 16-byte chunks, chunk c the quants of elements
+// 4 c .. + 3 and 16 + 4 c .. + 3; hd: the blocks' d as f32.
+int launch_q80_to_f16(const uint8_t* q, int64_t K, int64_t n_rows, uint16_t* h, float* hd, hipStream_t stream);
 
 // ffn.hip
 int launch_swiglu(const float* gate, const float* up, float* out, int64_t n_rows, int64_t n, size_t g_stride,
@@ -132,6 +143,10 @@ int launch_weighted_sum_rms(const float* experts, const float* weights, float* o
 // reads (launch_q8K_to_f16's layout), written by the same launch
 int launch_swiglu_q8K(const float* gate, const float* up, int64_t F, int64_t n_rows, void* dst, hipStream_t stream,
                       uint16_t* h_out = nullptr);
+// k_swiglu then k_quant_q8_0_act of its output, in one launch (F % 32 == 0; rows
+// dense and 16-byte aligned); h_out / hd_out as launch_quantize_act's
+int launch_swiglu_q80(const float* gate, const float* up, int64_t F, int64_t n_rows, void* dst, hipStream_t stream,
+                      uint16_t* h_out = nullptr, float* hd_out = nullptr);
 
 // Static device scratch of the allocation-free entry point (scratch.hip):
 // kScratchBytes per GPU.  scratch_setup(device), with that device current,
