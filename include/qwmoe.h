@@ -72,7 +72,10 @@ const char * qwmoe_strerror(int status);
 /* Experts that receive at least `rows` rows in one mul_mat_id (prefill and
  * large verify batches) are computed on the matrix cores when the weight type
  * is Q4_K, Q6_K or Q8_0; lighter experts, and every expert when rows == 0, use the
- * GEMV kernels, which are bit-identical to ggml.  Default 8.  The exact Q4_K form and Q8_0 run on the f16 matrix cores with an f16 copy
+ * GEMV kernels, which are bit-identical to ggml.  Default 8.  Where the matrix
+ * cores give the same bits (Q8_0, and the exact forms below), a batch of at least
+ * `rows` tokens that is dense in pairs per expert sends its lighter experts there
+ * too.  The exact Q4_K form and Q8_0 run on the f16 matrix cores with an f16 copy
  * of the activation quants (2 K bytes per activation row, Q8_0 K / 8 more, taken
  * from the workspace; without room for it the int8 matrix cores run for Q4_K, the
  * GEMV for Q8_0, with the same bits).  No reference counterpart: ggml's CPU

@@ -167,10 +167,27 @@ int mfma_f16_prep_pair(Arena& ar, qw::MmidArgs& mu, qw::MmidArgs& mg, int64_t n_
     return mfma_f16_prep(ar, mg, n_rows, st);
 }
 
-// Q8_0 runs on the matrix cores only with its f16 copy: without it every bin is the GEMV's.
+// Which bins the matrix cores take, once the f16 copy is known to be there or not.
+//  - Q8_0 runs on them only with its copy: without it every bin is the GEMV's.
+//  - Where every form gives ggml's bits (all but the block sums), a batch dense
+//    enough sends its light bins there too, in one launch in place of two: a
+//    16-row tile costs about what reading its weights does, the GEMV a pass per
+//    few rows.  The line is pairs per bin (128 experts, 8 per token, us per layer,
+//    light bins on the GEMV / everything on the matrix cores): Q4_K at the 30B
+//    shape 86.7 / 93.3 at T = 10, 119.5 / 113.4 at T = 16 (1 pair per bin),
+//    181.6 / 146.1 at T = 33, 312.5 / 267.4 at T = 512; Q8_0 123.9 / 125.1,
+//    161.9 / 156.4, 242.0 / 207.3, 466.7 / 418.7.  The exact Q6_K form does more
+//    work per tile: 216.1 / 261.3 at T = 33, 255.6 / 263.3 at T = 64,
+//    315.9 / 309.7 at T = 128 (8 pairs per bin), 502.4 / 459.4 at T = 512.
 qw::MmidArgs mfma_bins(const qw::MmidArgs& m) {
     qw::MmidArgs c = m;
     if (c.type == qw::T_Q8_0 && !c.act_h) c.mfma_min_rows = 0;
+    if (c.mfma_min_rows <= 1) return c;
+    const int64_t bins = c.slot_of ? c.n_slot_of : c.n_as;
+    const bool all = c.type == qw::T_Q8_0 ? c.n_pairs >= bins
+                                          : c.mfma_exact && (c.type == qw::T_Q6_K ? c.n_pairs >= 8 * bins
+                                                                                  : c.act_h && c.n_pairs >= bins);
+    if (all) c.mfma_min_rows = 1;
     return c;
 }
 
