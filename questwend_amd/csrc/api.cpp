@@ -57,6 +57,7 @@ struct Arena {
         off += count * sizeof(T) + 64;  // + slack: kernels may read a few bytes past a row end
         return p;
     }
+    size_t left() const { return cap > off ? cap - off : 0; }
     ~Arena() {
         if (track && off > g_lib.high_water) g_lib.high_water = off;
     }
@@ -627,27 +628,17 @@ int qwmoe_attn_seg(void* stream, const qwmoe_attn_layer* L, const float* h, int6
     if (T == 0) return QWMOE_OK;
     hipStream_t st = S(stream);
     Arena ar(kReserved);
-    const int64_t n_kv = n_past + T, split = qw::attn_split(T, nk, n_kv), n_split = (n_kv + split - 1) / split;
+    const int64_t n_kv = n_past + T;
     int32_t* rows = ar.take<int32_t>((size_t) (2 * T + 2));
     int32_t* active = ar.take<int32_t>(2);
     int32_t* active_off = ar.take<int32_t>(3);
     int32_t* n_active = ar.take<int32_t>(1);
-    float* cur = ar.take<float>((size_t) (H * T));
     float* q = ar.take<float>((size_t) (NQ * T));
     float* k = ar.take<float>((size_t) (NK * T));
     float* v = ar.take<float>((size_t) (NK * T));
-    float* qr = ar.take<float>((size_t) (NQ * T));
-    // the score rows and P.V partials exist only on the split path (fewer than 64
-    // query rows per kv head); the matrix-core path recomputes scores beside P.V
-    const bool mf_path = T * (nq / nk) >= 64;
-    float* sc = mf_path ? nullptr : ar.take<float>((size_t) (nq * T * n_kv));
-    float* part = mf_path ? nullptr : ar.take<float>((size_t) (n_split * T * NQ));
-    float* stat = ar.take<float>((size_t) (qw::attn_stat_blocks(T, nk, n_kv) * T * nq * 2));
-    float* att = ar.take<float>((size_t) (NQ * T));
+    uint16_t* qr = ar.take<uint16_t>((size_t) (NQ * T));
     float* proj = ar.take<float>((size_t) (H * T));
-    if (!rows || !active || !active_off || !n_active || !cur || !q || !k || !v || !qr || (!mf_path && (!sc || !part)) ||
-        !stat || !att || !proj)
-        return QWMOE_ERR_WORKSPACE;
+    if (!rows || !active || !active_off || !n_active || !q || !k || !v || !qr || !proj) return QWMOE_ERR_WORKSPACE;
     // quantized activations, one per vec_dot type in use
     const int vqt = qw::vec_dot_type(L->type_q), vkt = qw::vec_dot_type(L->type_k), vvt = qw::vec_dot_type(L->type_v);
     const int vot = qw::vec_dot_type(L->type_o);
@@ -658,40 +649,83 @@ int qwmoe_attn_seg(void* stream, const qwmoe_attn_layer* L, const float* h, int6
     uint8_t* xv = vvt == vqt ? xq : vvt == vkt ? xk : ar.take<uint8_t>(rv * (size_t) T + 64);
     uint8_t* aq = ar.take<uint8_t>(ro * (size_t) T + 64);
     if (!xq || !xk || !xv || !aq) return QWMOE_ERR_WORKSPACE;
+    // the norm's f32 rows, unless it writes Q8_K for all three projections
+    const bool all_q8K = vqt == qw::T_Q8_K && xk == xq && xv == xq && H % 256 == 0 && !((uintptr_t) L->attn_norm & 15);
+    float* cur = all_q8K ? nullptr : ar.take<float>((size_t) (H * T));
+    if (!all_q8K && !cur) return QWMOE_ERR_WORKSPACE;
+    // PV splits: as many of the statistics' splits as the workspace holds beside the
+    // f16 copies (f32 att too where the output projection reads Q8_0 and there is
+    // more than one), the others merged
+    const int64_t split = qw::attn_split(T, nq, nk, n_kv), n_split = (n_kv + split - 1) / split;
+    float* stat = ar.take<float>((size_t) (n_split * T * nq * 2));
+    const size_t per_pv = (size_t) (T * NQ * 4);
+    const size_t beside = (size_t) (T * (H + NQ) * 2) + (size_t) (T * (H + NQ) / 8) + (vot == qw::T_Q8_K ? 0 : per_pv) + 8192;
+    const int64_t fit = ar.left() > beside + per_pv ? (int64_t) ((ar.left() - beside) / per_pv) : 1;
+    int64_t merge = (n_split + std::min(fit, n_split) - 1) / std::min(fit, n_split);
+    if (merge * split * nk * 256 >= (int64_t(1) << 31)) return QWMOE_ERR_WORKSPACE;
+    const int64_t n_pv = (n_split + merge - 1) / merge;
+    float* part = ar.take<float>((size_t) (n_pv * T * NQ));
+    float* att = vot == qw::T_Q8_K ? nullptr : n_pv == 1 ? part : ar.take<float>((size_t) (NQ * T));
+    if (!part || !stat || (vot != qw::T_Q8_K && !att)) return QWMOE_ERR_WORKSPACE;
+    auto proj_args = [&](int type, const void* w, size_t nb1, int64_t K, int64_t N, const uint8_t* xb, size_t xrow,
+                         float* dst) {
+        const size_t ob = (size_t) N * 4;
+        return mmid_args(type, w, K, N, 1, nb1, nb1 * (size_t) N, xb, 1, xrow, rows, active, active_off, n_active, 1,
+                         nullptr, 0, dst, ob, ob, T, T);
+    };
+    qw::MmidArgs mq = proj_args(L->type_q, L->wq, L->wq_nb1, H, NQ, xq, rq, q);
+    qw::MmidArgs mk = proj_args(L->type_k, L->wk, L->wk_nb1, H, NK, xk, rk, k);
+    qw::MmidArgs mv = proj_args(L->type_v, L->wv, L->wv_nb1, H, NK, xv, rv, v);
+    qw::MmidArgs mo = proj_args(L->type_o, L->wo, L->wo_nb1, NQ, H, aq, ro, proj);
+    // the f16 copies the matrix cores read: one per quantized buffer, written by the
+    // launch that quantizes it
+    qw::MmidArgs* in[3] = {&mq, &mk, &mv};
+    for (int i = 0; i < 3; ++i) {
+        for (int j = 0; j < i && !in[i]->act_h; ++j)
+            if (in[j]->act_q == in[i]->act_q && in[j]->act_h && qw::mmid_mfma_h_ok(*in[i], T)) {
+                in[i]->act_h = in[j]->act_h;
+                in[i]->act_hd = in[j]->act_hd;
+            }
+        if (!in[i]->act_h) mfma_f16_reserve(ar, *in[i], T);
+    }
+    auto copy_of = [&](const uint8_t* x, uint16_t*& h, float*& hd) {
+        h = nullptr;
+        hd = nullptr;
+        for (const qw::MmidArgs* m : in)
+            if (m->act_q == x && m->act_h) {
+                h = (uint16_t*) m->act_h;
+                hd = (float*) m->act_hd;
+            }
+    };
+    mfma_f16_reserve(ar, mo, T);
     if ((rc = qw::launch_group_dense(rows, active, active_off, n_active, T, st))) return rc;
     const size_t hb = (size_t) H * 4;
     // attn_norm, then the projections' input quantized: one launch when every
     // projection reads Q8_K (the K-quants), the same bits as the two steps
-    const bool fused_norm = vqt == qw::T_Q8_K && xk == xq && xv == xq &&
-                            qw::launch_rms_norm_q8K(h, H, T, rms_eps, L->attn_norm, xq, st) == 0;
-    if (!fused_norm) {
+    uint16_t* hx;
+    float* hxd;
+    if (all_q8K) {
+        copy_of(xq, hx, hxd);
+        if ((rc = qw::launch_rms_norm_q8K(h, H, T, rms_eps, L->attn_norm, xq, st, hx))) return rc;
+    } else {
         if ((rc = qw::launch_rms_norm(h, cur, H, T, rms_eps, st, L->attn_norm))) return rc;
-        if ((rc = qw::launch_quantize_act(vqt, cur, H, 1, T, hb, hb, xq, st))) return rc;
-        if (xk != xq && (rc = qw::launch_quantize_act(vkt, cur, H, 1, T, hb, hb, xk, st))) return rc;
-        if (xv != xq && xv != xk && (rc = qw::launch_quantize_act(vvt, cur, H, 1, T, hb, hb, xv, st))) return rc;
-    }
-    auto proj_launch = [&](int type, const void* w, size_t nb1, int64_t K, int64_t N, const uint8_t* xb, size_t xrow,
-                           float* dst) {
-        const size_t ob = (size_t) N * 4;
-        const qw::MmidArgs m = mmid_args(type, w, K, N, 1, nb1, nb1 * (size_t) N, xb, 1, xrow, rows, active,
-                                         active_off, n_active, 1, nullptr, 0, dst, ob, ob, T, T);
-        return mmid_launch(m, st);
-    };
-    {   // Q and K in one GEMV launch when they share a type and neither takes the matrix cores
-        const qw::MmidArgs mq = mmid_args(L->type_q, L->wq, H, NQ, 1, L->wq_nb1, L->wq_nb1 * (size_t) NQ, xq, 1, rq,
-                                          rows, active, active_off, n_active, 1, nullptr, 0, q, (size_t) NQ * 4,
-                                          (size_t) NQ * 4, T, T);
-        const qw::MmidArgs mk = mmid_args(L->type_k, L->wk, H, NK, 1, L->wk_nb1, L->wk_nb1 * (size_t) NK, xk, 1, rk,
-                                          rows, active, active_off, n_active, 1, nullptr, 0, k, (size_t) NK * 4,
-                                          (size_t) NK * 4, T, T);
-        const bool pair = mq.type == mk.type && mq.mfma_min_rows == 0 && mk.mfma_min_rows == 0 && NQ >= NK &&
-                          qw::launch_mmid_gemv2(mq, mk, st) == 0;
-        if (!pair) {
-            if ((rc = mmid_launch(mq, st))) return rc;
-            if ((rc = mmid_launch(mk, st))) return rc;
+        const int vt[3] = {vqt, vkt, vvt};
+        uint8_t* xb[3] = {xq, xk, xv};
+        for (int i = 0; i < 3; ++i) {
+            bool done = false;
+            for (int j = 0; j < i; ++j) done = done || xb[j] == xb[i];
+            copy_of(xb[i], hx, hxd);
+            if (!done && (rc = qw::launch_quantize_act(vt[i], cur, H, 1, T, hb, hb, xb[i], st, hx, hxd))) return rc;
         }
     }
-    if ((rc = proj_launch(L->type_v, L->wv, L->wv_nb1, H, NK, xv, rv, v))) return rc;
+    // Q and K in one GEMV launch when they share a type and neither takes the matrix cores
+    const bool pair = mq.type == mk.type && mq.mfma_min_rows == 0 && mk.mfma_min_rows == 0 && NQ >= NK &&
+                      qw::launch_mmid_gemv2(mq, mk, st) == 0;
+    if (!pair) {
+        if ((rc = mmid_launch(mq, st))) return rc;
+        if ((rc = mmid_launch(mk, st))) return rc;
+    }
+    if ((rc = mmid_launch(mv, st))) return rc;
     qw::AttnArgs a{};
     a.T = (int) T;
     a.n_head = (int) nq;
@@ -709,16 +743,19 @@ int qwmoe_attn_seg(void* stream, const qwmoe_attn_layer* L, const float* h, int6
     a.qr = qr;
     a.kc = L->k_cache;
     a.vc = L->v_cache;
-    a.s = sc;
     a.split = split;
+    a.merge = (int) merge;
     a.part = part;
     a.stat = stat;
     a.att = att;
-    a.att_q8K = vot == qw::T_Q8_K ? aq : nullptr;   // the split path quantizes att as it sums it
+    a.att_q8K = vot == qw::T_Q8_K ? aq : nullptr;   // quantized as the splits are summed
+    a.att_h = vot == qw::T_Q8_K ? (uint16_t*) mo.act_h : nullptr;
     if ((rc = qw::launch_attn_core(a, st))) return rc;
     const size_t qb = (size_t) NQ * 4;
-    if (!qw::attn_writes_q8K(a) && (rc = qw::launch_quantize_act(vot, att, NQ, 1, T, qb, qb, aq, st))) return rc;
-    if ((rc = proj_launch(L->type_o, L->wo, L->wo_nb1, NQ, H, aq, ro, proj))) return rc;
+    if (vot != qw::T_Q8_K && (rc = qw::launch_quantize_act(vot, att, NQ, 1, T, qb, qb, aq, st, (uint16_t*) mo.act_h,
+                                                           (float*) mo.act_hd)))
+        return rc;
+    if ((rc = mmid_launch(mo, st))) return rc;
     return qw::launch_add_rms_norm_mul(proj, h, attn_resid, ffn_in, H, T, rms_eps, L->ffn_norm, st);
 }
 

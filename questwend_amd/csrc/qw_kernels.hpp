@@ -158,15 +158,19 @@ void* scratch_ptr(int device);
 // attn.hip: the attention half of Seg A (per-head norms, NEOX RoPE, f16 KV cache,
 // GQA scores, softmax, P.V), head dimension 128
 constexpr int ATT_RMAX = 16;      // query heads per kv head, at most
-constexpr int ATT_MF_SK = 512;   // keys per block of the matrix-core scores (and of their softmax statistics)
-// Keys per split of the split-softmax path (fewer than 64 query rows): a
-// multiple of 64 that gives the (kv head, token, split) workgroups about 512 in
-// all (64 keys at the 30B decode shape up to 8 k keys of context).
-inline int64_t attn_split(int64_t T, int64_t n_head_kv, int64_t n_kv) {
-    const int64_t pairs = T * n_head_kv > 0 ? T * n_head_kv : 1;
-    const int64_t want = 512 / pairs > 1 ? 512 / pairs : 1;   // splits per (kv head, token)
+// Waves per workgroup of the attention kernel, 32 query rows each.
+inline int attn_waves(int64_t rows) { return rows <= 32 ? 1 : rows <= 64 ? 2 : 4; }
+// Keys per split of the softmax statistics: a multiple of 64 that gives the (kv
+// head, row block, split) workgroups about 512 in all (two per CU; 64 keys at the
+// 30B decode shape up to 8 k keys of context).
+inline int64_t attn_split(int64_t T, int64_t n_head, int64_t n_head_kv, int64_t n_kv) {
+    const int64_t rows = T * (n_head / n_head_kv), per = 32 * attn_waves(rows);
+    const int64_t groups = n_head_kv * ((rows + per - 1) / per);
+    int64_t want = groups < 512 ? 512 / groups : 1;
+    const int64_t need = n_kv * n_head_kv * 256 / (int64_t(1) << 30) + 1;   // a split's rows are addressed in 31 bits
+    if (want < need) want = need;
     const int64_t keys = (n_kv + want - 1) / want;
-    return 64 * ((keys + 63) / 64 > 0 ? (keys + 63) / 64 : 1);
+    return 64 * ((keys + 63) / 64);
 }
 struct AttnArgs {
     int T, n_head, n_head_kv;
@@ -177,31 +181,22 @@ struct AttnArgs {
     const float* v;               // [T][n_head_kv][128]
     const float* q_norm;          // [128]
     const float* k_norm;          // [128]
-    float* qr;                    // [T][n_head][128] Q after norm and RoPE
+    uint16_t* qr;                 // f16 [T][n_head][128] Q after norm and RoPE
     uint16_t* kc;                 // f16 caches [n_ctx][n_head_kv * 128], 16-byte aligned
     uint16_t* vc;
-    float* s;                     // [T][n_head][n_kv] scores, then probabilities
-    int64_t split;                // keys per split (attn_split; fewer than 64 query rows)
-    float* part;                  // [ceil(n_kv / split)][T][n_head][128] partial products
-    float* stat;                  // [blocks][T][n_head][2]: each key split's / 512-key block's max and sum
-                                  // (attn_stat_blocks blocks)
-    float* att;                   // [T][n_head * 128]
-    void* att_q8K;                // optional: Q8_K rows of att (the split path writes these instead of att)
+    int64_t split;                // keys per split of the statistics (attn_split)
+    int merge;                    // statistics splits per PV split
+    float* part;                  // [PV splits][T][n_head][128] each PV split's sums
+    float* stat;                  // [splits][T][n_head][2] each split's maximum (log2 units) and sum
+    float* att;                   // [T][n_head * 128] (without att_q8K; may be part when there is one split)
+    void* att_q8K;                // optional: Q8_K rows of att, written in its place (n_head * 128 a multiple of 256)
+    uint16_t* att_h;              // optional, with att_q8K: its f16 copy (launch_q8K_to_f16's layout)
 };
-// blocks of softmax statistics launch_attn_core writes: one per key split (fewer
-// than 64 query rows) or per 512-key block of the matrix-core scores
-inline int64_t attn_stat_blocks(int64_t T, int64_t n_head_kv, int64_t n_kv) {
-    const int64_t sp = attn_split(T, n_head_kv, n_kv), ns = (n_kv + sp - 1) / sp, nb = (n_kv + ATT_MF_SK - 1) / ATT_MF_SK;
-    return ns > nb ? ns : nb;
-}
 int launch_attn_core(const AttnArgs& a, hipStream_t stream);
-// whether launch_attn_core writes a.att_q8K (and not att) for these arguments
-inline bool attn_writes_q8K(const AttnArgs& a) {
-    return a.att_q8K && (int64_t) a.T * (a.n_head / a.n_head_kv) < 64;
-}
-// attn_norm and its Q8_K quantisation in one launch (n % 256 == 0, x and w 16-byte aligned)
+// attn_norm and its Q8_K quantisation in one launch (n % 256 == 0, x and w 16-byte aligned);
+// h_out (optional): the rows' f16 copy (launch_q8K_to_f16's layout)
 int launch_rms_norm_q8K(const float* x, int64_t n, int64_t rows, float eps, const float* w, void* dst,
-                        hipStream_t stream);
+                        hipStream_t stream, uint16_t* h_out = nullptr);
 // resid = x + y; out = rms_norm(resid) * w (rows of n, dense), out may be null
 int launch_add_rms_norm_mul(const float* x, const float* y, float* resid, float* out, int64_t n, int64_t rows,
                             float eps, const float* w, hipStream_t stream);
