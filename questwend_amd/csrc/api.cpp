@@ -136,10 +136,9 @@ bool mfma_f16_reserve(Arena& ar, qw::MmidArgs& m, int64_t n_rows) {
     if (!qw::mmid_mfma_h_ok(m, n_rows)) return false;
     const char* env = getenv("QWMOE_MFMA_F16");
     if (env && env[0] == '0') return false;
-    const bool q80 = m.type == qw::T_Q8_0;
-    uint16_t* h = ar.take<uint16_t>((size_t) (n_rows * (m.K + (q80 ? m.K / 16 : 0))));   // (K / 32 f32 scales per row)
+    uint16_t* h = ar.take<uint16_t>((size_t) (n_rows * (m.K + m.K / 16)));   // (a row's f32 scales or f16 bsums behind)
     m.act_h = h;
-    m.act_hd = h && q80 ? (const float*) (h + n_rows * m.K) : nullptr;
+    m.act_hd = h ? h + n_rows * m.K : nullptr;
     return h != nullptr;
 }
 

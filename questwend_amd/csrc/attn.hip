@@ -396,7 +396,9 @@ __global__ void __launch_bounds__(256) k_attn_combine(AttnArgs a, int n_split) {
     if (blk * 256 >= n) return;
     if (a.att_q8K) {   // (n is a multiple of 256)
         const float vv[4] = {acc.x, acc.y, acc.z, acc.w};
-        quant_q8K_wave(vv, lane, (BlockQ8_K*) a.att_q8K + blk, a.att_h ? (_Float16*) a.att_h + (size_t) blk * QK_K : nullptr);
+        _Float16* hh = (_Float16*) a.att_h;
+        quant_q8K_wave(vv, lane, (BlockQ8_K*) a.att_q8K + blk, hh ? hh + (size_t) blk * QK_K : nullptr,
+                       hh ? hh + (size_t) n + (size_t) blk * 16 : nullptr);
     } else if (i0 < n) {
         *(float4*) (a.att + i0) = acc;
     }
@@ -452,7 +454,8 @@ __global__ void __launch_bounds__(256) k_rms_norm_q8K(const float* __restrict__ 
         const float4 ww = *(const float4*) (w + ib * QK_K + 4 * lane);
         const float v[4] = {(q.x * scale) * ww.x, (q.y * scale) * ww.y, (q.z * scale) * ww.z, (q.w * scale) * ww.w};
         const int64_t blk = (int64_t) blockIdx.x * nb + ib;
-        quant_q8K_wave(v, lane, dst + blk, hout ? hout + (size_t) blk * QK_K : nullptr);
+        quant_q8K_wave(v, lane, dst + blk, hout ? hout + (size_t) blk * QK_K : nullptr,
+                       hout ? hout + (size_t) (nb * gridDim.x) * QK_K + (size_t) blk * 16 : nullptr);
     }
 }
 

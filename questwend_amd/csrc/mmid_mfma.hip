@@ -381,6 +381,8 @@ k_mmid_mfma_q4k(MfLaunch lp) {
 // from the Q8_K rows.  ~52 KB of LDS: three workgroups per CU.
 typedef _Float16 h8m __attribute__((ext_vector_type(8)));
 typedef _Float16 h2m __attribute__((ext_vector_type(2)));
+typedef _Float16 h4m __attribute__((ext_vector_type(4)));
+typedef float f16m __attribute__((ext_vector_type(16)));
 typedef float f4m __attribute__((ext_vector_type(4)));
 constexpr int MH_NB = 1;   // 16-row activation tiles per pass of the f16 form (two measured slower, 78 KB
                            // of LDS and two workgroups per CU, and failed the bit-exact test: not used)
@@ -610,6 +612,10 @@ __global__ void k_q8K_to_h(const uint8_t* __restrict__ q, size_t row_bytes, int6
     const uint32_t u0 = *(const uint32_t*) src, u1 = *(const uint32_t*) (src + 32);
     auto b = [](uint32_t u, int k) { return (_Float16) (float) (int8_t) (u >> (8 * k)); };
     *(h8m*) (out + (size_t) r * K + 8 * ci) = h8m{b(u0, 0), b(u0, 2), b(u0, 1), b(u0, 3), b(u1, 0), b(u1, 2), b(u1, 1), b(u1, 3)};
+    if (c < 16) {
+        const int16_t s = *(const int16_t*) (q + (size_t) r * row_bytes + 292 * (size_t) bb + 260 + 2 * c);
+        out[(size_t) (rows * K) + ((size_t) (r * (K / QK_K) + bb)) * 16 + c] = (_Float16) (float) s;
+    }
 }
 
 int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t rows, uint16_t* out, hipStream_t stream) {
@@ -629,10 +635,10 @@ int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t row
 //    matrices; an item is up to 32 routed rows of one heavy expert.  Each
 //    workgroup builds the item table (first item of each active expert) once in
 //    LDS; a unit's expert is a count over that table.
-//  - the three-stage copy pipeline runs on across units: while the last
-//    super-blocks of a unit are computed, the first ones of the next unit are
-//    being copied.  The next unit's (e, t) pairs are copied into LDS by the same
-//    DMA path one super-block ahead, so they are counted by the same waits.
+//  - the copy pipeline (two stage buffers, one super-block ahead) runs on across
+//    units: while the last super-block of a unit is computed, the first one of the
+//    next unit is being copied.  The next unit's (e, t) pairs are copied into LDS by
+//    the same DMA path two super-blocks ahead.
 //  - two 16-row activation tiles per item: each A operand (sc * q4 of 16 weight
 //    rows) serves 32 activation rows.  A last item of at most 16 rows computes
 //    one tile; those items are numbered after all others, so a workgroup runs
@@ -644,16 +650,22 @@ int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t row
 //    per pair apart (16 bytes of pad): the 16 rows a tile reads at one chunk
 //    offset fall on distinct LDS banks, and every B read is the lane's base plus
 //    a constant.
-// ~81 KB of LDS: two workgroups per CU.  Needs K >= 768 (three super-blocks: the
-// next unit's pairs land one super-block before they are used) and at most
-// MP_MAXG active bins.  Measured at configs[2] (T = 512, Zipf-skewed routing):
-// gate + up 170 us, down 104 us per launch against 174 / 114 us for
-// k_mmid_mfma_q4k_h; counters put it at ~56 % VALU-busy and ~16 % MFMA-busy,
-// with waves waiting a third of their cycles (two waves per SIMD).
+//  - the min lanes from the Q8_K blocks' bsums (an f16 copy behind the quants' one):
+//    prod_m is mins 2m, 2m, 2m + 1, 2m + 1 against bsums 4m .. 4m + 3, so one
+//    v_mfma_f32_16x16x4_4b_f16 forms all four min lanes of a tile from 8 bytes per
+//    lane, in place of eight 32-deep products over the quants read from LDS a
+//    second time (half of the kernel's LDS reads).
+// ~57 KB of LDS, 248 VGPRs: two workgroups per CU.  Needs K >= 768 (three
+// super-blocks: the next unit's pairs land before they are used) and at most
+// MP_MAXG active bins.  Bound: VALU issue (about 258 instructions per wave and
+// super-block, 96 of them ggml's own fma) with two waves per SIMD to hide each
+// other's LDS and barrier waits.  us per launch: T = 1024 at H = 4096, gate + up
+// 894 (min lanes over the quants) -> 723; T = 512 at the 30B shape, Zipf-skewed,
+// mean of gate + up and down 129 -> 120.
 constexpr int MP_NR = 32;             // activation rows per item (two 16-row tiles)
 constexpr uint32_t MP_HS = 1040;      // LDS bytes per activation DMA instruction (rows i, i + 16, pad)
 constexpr int MP_MAXG = 128;          // active bins the item table holds
-constexpr int MP_VM = 6;              // fewest DMA instructions a wave issues per stage (waves 1, 2: 2 + 4)
+constexpr int MP_ST = 2;              // stage buffers
 
 struct MpUnit {
     int z, ntok, ok, p0;
@@ -663,9 +675,10 @@ struct MpUnit {
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
-    __shared__ __align__(16) uint8_t s_w[3][MF_M * MF_WS];
-    __shared__ __align__(16) uint8_t s_h[3][16 * MP_HS];
-    __shared__ __align__(16) float s_d[3][MP_NR];
+    __shared__ __align__(16) uint8_t s_w[MP_ST][MF_M * MF_WS];
+    __shared__ __align__(16) uint8_t s_h[MP_ST][16 * MP_HS];
+    __shared__ __align__(16) uint8_t s_b[MP_ST][MP_NR * 32];   // bsums (f16)
+    __shared__ __align__(16) float s_d[MP_ST][MP_NR];
     __shared__ __align__(16) int32_t s_meta[2][2 * MP_NR];   // (e, t) of a unit's 32 rows
     __shared__ int32_t s_if[MP_MAXG + 1], s_if1[MP_MAXG + 1], s_aoff[MP_MAXG + 1], s_mat[2][MP_MAXG];
     const MmidArgs& m0 = lp.m[0];
@@ -729,6 +742,7 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
     const int64_t b_ne1 = m0.b_ne1;
     const i32x4 hrsrc = rsrc_words(m0.act_h, 0x7fffffffu);
     const i32x4 arsrc = rsrc_words(m0.act_q, 0x7fffffffu);
+    const i32x4 brsrc = rsrc_words(m0.act_hd, 0x7fffffffu);
     const i32x4 prsrc = rsrc_words(m0.rows, (uint32_t) (8 * m0.n_pairs));
     // unit u: its matrix, rows and weight tile (uniform).  Units [0, U2) are the
     // two-tile items' (matrix, item, tile), then the one-tile items'.  (Units
@@ -776,25 +790,28 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
         const uint32_t er = bn == 1u ? 0u : e < bn ? e : e % bn;
         return er + t * bn;
     };
-    auto lane_offs = [&](int mb, int ntok, uint32_t (&ho)[4], uint32_t& dof) __attribute__((always_inline)) {
+    auto lane_offs = [&](int mb, int ntok, uint32_t (&ho)[4], uint32_t& dof, uint32_t& bof) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int nrow = wave + 4 * k + 16 * (lane >> 5);
             ho[k] = arow(mb, nrow < ntok ? nrow : 0) * (uint32_t) (2 * m0.K) + 16u * (uint32_t) (lane & 31);
         }
         dof = arow(mb, lane < ntok && lane < MP_NR ? lane : 0) * (uint32_t) m0.act_row_bytes;
+        bof = arow(mb, (lane >> 1) < ntok ? lane >> 1 : 0) * (uint32_t) (m0.K / 8) + 16u * (uint32_t) (lane & 1);
     };
     // copies of super-block i of a unit into stage buffer sb
-    auto issue = [&](int sb, const MpUnit& U, const uint32_t (&ho)[4], uint32_t dof, int i) __attribute__((always_inline)) {
+    auto issue = [&](int sb, const MpUnit& U, const uint32_t (&ho)[4], uint32_t dof, uint32_t bof, int i)
+        __attribute__((always_inline)) {
         uint32_t lw = (uint32_t) (uintptr_t) s_w[sb], lh = (uint32_t) (uintptr_t) s_h[sb];
-        uint32_t ld = (uint32_t) (uintptr_t) s_d[sb];
-        asm volatile("" : "+s"(lw), "+s"(lh), "+s"(ld));
+        uint32_t ld = (uint32_t) (uintptr_t) s_d[sb], lb = (uint32_t) (uintptr_t) s_b[sb];
+        asm volatile("" : "+s"(lw), "+s"(lh), "+s"(ld), "+s"(lb));
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             if (wv + 4 * k < 9) dma_b128(U.wrsrc, lw + 1024u * (uint32_t) (wv + 4 * k), woff[k], 144u * (uint32_t) i);
 #pragma unroll
         for (int k = 0; k < 4; ++k) dma_b128(hrsrc, lh + MP_HS * (uint32_t) (wv + 4 * k), ho[k], 512u * (uint32_t) i);
         if (wv == 3 && lane < MP_NR) dma_b32(arsrc, ld, dof, 292u * (uint32_t) i);
+        if (wv == 2) dma_b128(brsrc, lb, bof, 32u * (uint32_t) i);   // row lane / 2, half lane % 2
     };
 
     float acc[2][4][8], accm[2][4][4];
@@ -830,6 +847,9 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
         uint32_t hx2 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 2) * MF_WS);
         uint32_t hx3 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 3) * MF_WS);
         float dy0 = sd[lr], dy1 = NBT > 1 ? sd[16 + lr] : 0.0f;
+        h4m bs[NBT];
+#pragma unroll
+        for (int t = 0; t < NBT; ++t) bs[t] = *(const h4m*) (s_b[sb] + (16 * t + lr) * 32 + 8 * gq);
         const u32x4m hdr = *(const u32x4m*) (sw + arow_l * MF_WS);
         uint32_t s0 = hdr.y, s1 = hdr.z, s2 = hdr.w, sx = hdr.x;
         // and the 8 quant words of its 32-byte group gq (one per AVX lane)
@@ -865,6 +885,20 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
                 dmin[t][r] = -dy * xdm[r];
             }
         }
+        // the min lanes: product p of one four-product instruction (16 x 16 x 4 each) is
+        // min lane p, mins 2p, 2p, 2p + 1, 2p + 1 against bsums 4p .. 4p + 3
+        const uint32_t mnw = ((gq < 2 ? mn_lo : mn_hi) >> (16 * (gq & 1))) & 0xffffu;
+        const h2m mn0 = h2_bits(__builtin_amdgcn_perm(0u, mnw, 0x0c000c00u) | 0x64006400u) - h2m{1024, 1024};
+        const h2m mn1 = h2_bits(__builtin_amdgcn_perm(0u, mnw, 0x0c010c01u) | 0x64006400u) - h2m{1024, 1024};
+        const h4m Am = {mn0.x, mn0.y, mn1.x, mn1.y};
+        f16m Dm[NBT];
+#pragma unroll
+        for (int t = 0; t < NBT; ++t) {
+            f16m z;
+#pragma unroll
+            for (int k = 0; k < 16; ++k) z[k] = 0.0f;
+            Dm[t] = __builtin_amdgcn_mfma_f32_16x16x4f16(Am, bs[t], z, 0, 0, 0);
+        }
         // software-pipelined over the AVX lanes: lane L's matrix-core products are
         // issued before lane L - 1's fp32 steps, so each result is read an
         // iteration after its instruction (the same operations per accumulator)
@@ -879,7 +913,7 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
             h8m Bn[NBT];
 #pragma unroll
             for (int t = 0; t < NBT; ++t)
-                Bn[t] = *(const h8m*) (sh + 512 * t + 16 * (L < 7 ? 8 * gq + L + 1 : gq));
+                Bn[t] = L < 7 ? *(const h8m*) (sh + 512 * t + 16 * (8 * gq + L + 1)) : Bc[t];
             __builtin_amdgcn_sched_barrier(0);   // (keeps those reads issued here, a step ahead)
             const uint32_t v = w >> 8;
             const h2m a0 = __builtin_elementwise_fma(h2_bits((w & 0x000F000Fu) | hmag), S_lo, C_lo);
@@ -900,7 +934,7 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
 #pragma unroll
             for (int t = 0; t < NBT; ++t) {
                 Dp[t] = Dc[t];
-                Bc[t] = Bn[t];   // (after lane 7: min lane 0's first operand, chunk gq)
+                Bc[t] = Bn[t];
             }
         }
 #pragma unroll
@@ -908,46 +942,11 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[t][r][7] = __builtin_fmaf(d[t][r], Dp[t][r], acc[t][r][7]);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t mnw = q < 2 ? mn_lo : mn_hi;
-            const uint32_t b0 = (uint32_t) (2 * (q & 1)), b1 = b0 + 1;
-            const h2m mm0 = h2_bits(__builtin_amdgcn_perm(0u, mnw, 0x0c000c00u | b0 | (b0 << 16)) | 0x64006400u) -
-                            h2m{1024, 1024};
-            const h2m mm1 = h2_bits(__builtin_amdgcn_perm(0u, mnw, 0x0c000c00u | b1 | (b1 << 16)) | 0x64006400u) -
-                            h2m{1024, 1024};
-            const h8m Am = __builtin_bit_cast(h8m, u32x4m{h2_u32(mm0), h2_u32(mm0), h2_u32(mm1), h2_u32(mm1)});
-            // Bc holds chunk 8 q + gq of each tile (read a step ahead); chunk 8 q + 4 + gq
-            // is read here, and the next min lane's first chunk for the step after
-            h8m B1[NBT], Bn[NBT];
-#pragma unroll
-            for (int t = 0; t < NBT; ++t) {
-                B1[t] = *(const h8m*) (sh + 512 * t + 16 * (8 * q + 4 + gq));
-                Bn[t] = *(const h8m*) (sh + 512 * t + 16 * (q < 3 ? 8 * (q + 1) + gq : gq));
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            f4m Dc[NBT];
-#pragma unroll
-            for (int t = 0; t < NBT; ++t) {
-                Dc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Am, Bc[t], f4m{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                Dc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Am, B1[t], Dc[t], 0, 0, 0);
-            }
-            if (q > 0) {   // (min lane q - 1's fp32 steps, pipelined as above)
-#pragma unroll
-                for (int t = 0; t < NBT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        accm[t][r][q - 1] = __builtin_fmaf(dmin[t][r], Dp[t][r], accm[t][r][q - 1]);
-            }
-#pragma unroll
-            for (int t = 0; t < NBT; ++t) {
-                Dp[t] = Dc[t];
-                Bc[t] = Bn[t];
-            }
-        }
-#pragma unroll
         for (int t = 0; t < NBT; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) accm[t][r][3] = __builtin_fmaf(dmin[t][r], Dp[t][r], accm[t][r][3]);
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) accm[t][r][q] = __builtin_fmaf(dmin[t][r], Dm[t][4 * q + r], accm[t][r][q]);
     };
     // hsum_float_8(acc) + ((m0 + m2) + (m1 + m3)) of a finished unit; weight rows
     // r0 + 16 wave + 4 gq .. +3, activation rows lr and 16 + lr
@@ -983,20 +982,18 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
     if (wv == 0) dma_b32(prsrc, (uint32_t) (uintptr_t) s_meta[0], 4u * (uint32_t) lane, 8u * (uint32_t) cur.p0);
     vm_wait<0>();
     lds_barrier();
-    uint32_t ho[4], dof, hn[4], dn = 0;
-    lane_offs(0, cur.ntok, ho, dof);
+    uint32_t ho[4], dof, bof, hn[4], dn = 0, bn = 0;
+    lane_offs(0, cur.ntok, ho, dof, bof);
 #pragma unroll
     for (int k = 0; k < 4; ++k) hn[k] = ho[k];
     zero();
-    issue(0, cur, ho, dof, 0);
-    issue(1, cur, ho, dof, 1);
+    issue(0, cur, ho, dof, bof, 0);
     const int S = my_units * nb;
     int i = 0, j = 0, sb = 0, s = 0;
     // one step: super-block i of unit j.  The unit's tile count is a template
     // argument: a workgroup meets its two-tile units first, then its one-tile ones.
     auto step = [&](auto nbt_c) __attribute__((always_inline)) {
-        if (s + 1 < S) vm_wait<MP_VM>();   // super-block s + 1's copies may stay in flight
-        else vm_wait<0>();
+        vm_wait<0>();
         lds_barrier();
         const bool more = j + 1 < my_units;
         if (i == 0 && more) {   // the next unit's pairs: copied before this step's super-block copies
@@ -1004,13 +1001,16 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
             if (wv == 0)
                 dma_b32(prsrc, (uint32_t) (uintptr_t) s_meta[(j + 1) & 1], 4u * (uint32_t) lane, 8u * (uint32_t) nxt.p0);
         }
-        if (i == 1 && more) lane_offs((j + 1) & 1, nxt.ntok, hn, dn);   // (landed: waited for above)
-        if (s + 2 < S) {
-            const int i2 = i + 2, sb2 = sb == 0 ? 2 : sb - 1;
-            if (i2 < nb) issue(sb2, cur, ho, dof, i2);
-            else issue(sb2, nxt, hn, dn, i2 - nb);
+        if (i == 1 && more) lane_offs((j + 1) & 1, nxt.ntok, hn, dn, bn);   // (landed: waited for above)
+        if (s + 1 < S) {
+            if (i + 1 < nb) issue(sb ^ 1, cur, ho, dof, bof, i + 1);
+            else issue(sb ^ 1, nxt, hn, dn, bn, 0);
         }
+        // (a wave in its products goes before the other workgroup's wave on the SIMD that
+        // is between steps: 740 -> 723 us and 125 -> 119 us per launch, see above)
+        __builtin_amdgcn_s_setprio(1);
         compute(sb, nbt_c);
+        __builtin_amdgcn_s_setprio(0);
         if (++i == nb) {
             finish(cur, j & 1, nbt_c);
             zero();
@@ -1018,10 +1018,11 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) ho[k] = hn[k];
             dof = dn;
+            bof = bn;
             i = 0;
             ++j;
         }
-        sb = sb == 2 ? 0 : sb + 1;
+        sb ^= 1;
         ++s;
     };
     while (s < S && cur.ntok > 16) step(std::integral_constant<int, 2>{});
@@ -1527,13 +1528,13 @@ bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows) {
 // the environment keeps k_mmid_mfma_q4k_h (a test switch).
 static bool mp_ok(const MfLaunch& lp, int nz) {
     const MmidArgs& a = lp.m[0];
-    if (a.type != T_Q4_K || !a.mfma_exact || !a.act_h || a.K < 3 * QK_K || a.max_active > MP_MAXG ||
+    if (a.type != T_Q4_K || !a.mfma_exact || !a.act_h || !a.act_hd || a.K < 3 * QK_K || a.max_active > MP_MAXG ||
         a.n_pairs <= 0 || 8 * a.n_pairs >= (int64_t(1) << 31) || a.b_ne1 < 1 || a.b_ne1 > 65535)
         return false;
     if (nz == 2) {
         const MmidArgs& b = lp.m[1];
         if (b.rows != a.rows || b.active != a.active || b.active_off != a.active_off || b.n_active != a.n_active ||
-            b.act_h != a.act_h || b.act_q != a.act_q || b.b_ne1 != a.b_ne1 || b.act_row_bytes != a.act_row_bytes ||
+            b.act_h != a.act_h || b.act_hd != a.act_hd || b.act_q != a.act_q || b.b_ne1 != a.b_ne1 || b.act_row_bytes != a.act_row_bytes ||
             b.mfma_min_rows != a.mfma_min_rows || b.nb1 != a.nb1 || b.K != a.K || b.N != a.N)
             return false;
     }

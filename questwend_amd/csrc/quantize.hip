@@ -28,7 +28,8 @@ __global__ void __launch_bounds__(256) k_quant_q8K(const float* __restrict__ src
     const float* x = (const float*) ((const char*) src + i1 * nb1 + i2 * nb2) + ib * QK_K;
     const float4 q = *(const float4*) (x + 4 * lane);
     const float v[4] = {q.x, q.y, q.z, q.w};
-    quant_q8K_wave(v, lane, dst + blk, hout ? hout + (size_t) blk * QK_K : nullptr);
+    quant_q8K_wave(v, lane, dst + blk, hout ? hout + (size_t) blk * QK_K : nullptr,
+                   hout ? hout + (size_t) (nb * nrows) * QK_K + (size_t) blk * 16 : nullptr);
 }
 
 // SwiGLU (ggml_swiglu_split: silu(gate) * up, ops.cpp:3182-3238) of n_rows dense
@@ -46,7 +47,8 @@ __global__ void __launch_bounds__(256) k_swiglu_q8K(const float* __restrict__ ga
     const float4 g = *(const float4*) (gate + off);
     const float4 u = *(const float4*) (up + off);
     const float v[4] = {v_silu(g.x) * u.x, v_silu(g.y) * u.y, v_silu(g.z) * u.z, v_silu(g.w) * u.w};
-    quant_q8K_wave(v, lane, dst + blk, hout ? hout + (size_t) blk * QK_K : nullptr);
+    quant_q8K_wave(v, lane, dst + blk, hout ? hout + (size_t) blk * QK_K : nullptr,
+                   hout ? hout + (size_t) (nb * n_rows) * QK_K + (size_t) blk * 16 : nullptr);
 }
 
 int launch_swiglu_q8K(const float* gate, const float* up, int64_t F, int64_t n_rows, void* dst, hipStream_t stream,

@@ -92,9 +92,10 @@ struct MmidArgs {
     // optional (exact Q4_K matrix-core form): the f16 copy of act_q's quants made by
     // launch_q8K_to_f16; with it the exact form runs on the f16 matrix cores (the same bits)
     // (Q8_0: the copy of launch_quantize_act / launch_swiglu_q80 / launch_q80_to_f16, which
-    // the Q8_0 matrix-core form needs, and act_hd the row blocks' d as f32 [row][K / 32])
+    // the Q8_0 matrix-core form needs).  act_hd: behind the rows' quants, for Q4_K the
+    // blocks' bsums as f16 [row][K / 256][16], for Q8_0 their d as f32 [row][K / 32]
     const uint16_t* act_h;
-    const float* act_hd;
+    const void* act_hd;
 };
 int launch_mmid_gemv(const MmidArgs& m, hipStream_t stream);
 // mmid_q80.hip: one or two Q8_0 GEMVs on the kernel that copies whole rows straight
@@ -113,7 +114,8 @@ int launch_mmid_mfma(const MmidArgs& m, hipStream_t stream);
 int launch_mmid_mfma2(const MmidArgs& a, const MmidArgs& b, hipStream_t stream);
 // f16 copy of n_rows Q8_K activation rows (row_bytes apart, K values each) for
 // the exact Q4_K form on the f16 matrix cores: row r at out + r * K, every group
-// of four quants in the order 0, 2, 1, 3
+// of four quants in the order 0, 2, 1, 3; then the rows' bsums, 16 per block
+// (out holds n_rows * (K + K / 16) values)
 int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t n_rows, uint16_t* out, hipStream_t stream);
 // whether m (with act_q holding n_rows rows) can take such a copy as act_h
 bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows);
