@@ -75,10 +75,10 @@ const char * qwmoe_strerror(int status);
  * GEMV kernels, which are bit-identical to ggml.  Default 8.  Where the matrix
  * cores give the same bits (Q8_0, and the exact forms below), a batch of at least
  * `rows` tokens that is dense in pairs per expert sends its lighter experts there
- * too.  The exact Q4_K form and Q8_0 run on the f16 matrix cores with an f16 copy
- * of the activation quants (2 K bytes per activation row, Q8_0 K / 8 more, taken
- * from the workspace; without room for it the int8 matrix cores run for Q4_K, the
- * GEMV for Q8_0, with the same bits).  No reference counterpart: ggml's CPU
+ * too.  The exact forms and Q8_0 run on the f16 matrix cores with an f16 copy
+ * of the activation quants (2 K + K / 8 bytes per activation row, taken from
+ * the workspace; without room for it the int8 matrix cores run for the K-quants,
+ * the GEMV for Q8_0, with the same bits).  No reference counterpart: ggml's CPU
  * backend has one dot product per type (ggml-cpu.c:1463-1524); this only
  * selects the GPU kernel. */
 int qwmoe_set_mfma_min_rows(int rows);

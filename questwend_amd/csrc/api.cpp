@@ -127,10 +127,10 @@ qw::MmidArgs mmid_args(int type, const void* as, int64_t K, int64_t N, int64_t n
 }
 
 // The f16 copy of the n_rows activation rows in act_q that the f16 matrix cores
-// read (the exact Q4_K form, and Q8_0), in the call's workspace: reserved and
+// read (the exact Q4_K and Q6_K forms, and Q8_0), in the call's workspace: reserved and
 // attached to m, nothing launched (act_h, and for Q8_0 act_hd, go to the launch
 // that quantizes the rows, or to mfma_f16_prep's).  Without room for it the int8
-// matrix cores (Q4_K) or the GEMV (Q8_0) run, with the same bits.
+// matrix cores (Q4_K, Q6_K) or the GEMV (Q8_0) run, with the same bits.
 // QWMOE_MFMA_F16=0 in the environment keeps those (a test switch).
 bool mfma_f16_reserve(Arena& ar, qw::MmidArgs& m, int64_t n_rows) {
     if (!qw::mmid_mfma_h_ok(m, n_rows)) return false;
@@ -176,16 +176,17 @@ int mfma_f16_prep_pair(Arena& ar, qw::MmidArgs& mu, qw::MmidArgs& mg, int64_t n_
 //    light bins on the GEMV / everything on the matrix cores): Q4_K at the 30B
 //    shape 86.7 / 93.3 at T = 10, 119.5 / 113.4 at T = 16 (1 pair per bin),
 //    181.6 / 146.1 at T = 33, 312.5 / 267.4 at T = 512; Q8_0 123.9 / 125.1,
-//    161.9 / 156.4, 242.0 / 207.3, 466.7 / 418.7.  The exact Q6_K form does more
-//    work per tile: 216.1 / 261.3 at T = 33, 255.6 / 263.3 at T = 64,
-//    315.9 / 309.7 at T = 128 (8 pairs per bin), 502.4 / 459.4 at T = 512.
+//    161.9 / 156.4, 242.0 / 207.3, 466.7 / 418.7.  Q6_K forms more integers per tile:
+//    142.0 / 157.6 at T = 16, 214.5 / 203.9 at T = 33, 230.7 / 205.3 at T = 64 (4 pairs
+//    per bin), but as the down projection at H = 4096 459.7 / 510.6 at T = 33,
+//    490.8 / 508.1 at T = 64, 539.5 / 551.2 at T = 128.
 qw::MmidArgs mfma_bins(const qw::MmidArgs& m) {
     qw::MmidArgs c = m;
     if (c.type == qw::T_Q8_0 && !c.act_h) c.mfma_min_rows = 0;
     if (c.mfma_min_rows <= 1) return c;
     const int64_t bins = c.slot_of ? c.n_slot_of : c.n_as;
     const bool all = c.type == qw::T_Q8_0 ? c.n_pairs >= bins
-                                          : c.mfma_exact && (c.type == qw::T_Q6_K ? c.n_pairs >= 8 * bins
+                                          : c.mfma_exact && (c.type == qw::T_Q6_K ? c.act_h && c.n_pairs >= 4 * bins
                                                                                   : c.act_h && c.n_pairs >= bins);
     if (all) c.mfma_min_rows = 1;
     return c;

@@ -627,7 +627,7 @@ int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t row
 }
 
 // ---- exact Q4_K on the f16 matrix cores, persistent -------------------------
-// k_mmid_mfma_q4k_hp computes what k_mmid_mfma_q4k_h computes -- the same A and
+// k_mmid_mfma_hp computes what k_mmid_mfma_q4k_h computes -- the same A and
 // B operands, one v_mfma_f32_16x16x32_f16 per AVX lane and tile, the same fp32
 // steps in the same order, so the same bits -- with another schedule:
 //  - a grid of two workgroups per CU walks the work units u = b, b + grid, ...
@@ -662,6 +662,21 @@ int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t row
 // other's LDS and barrier waits.  us per launch: T = 1024 at H = 4096, gate + up
 // 894 (min lanes over the quants) -> 723; T = 512 at the 30B shape, Zipf-skewed,
 // mean of gate + up and down 129 -> 120.
+//
+// Q6_K (TYPE) runs the same pipeline.  Its integers (see k_mmid_mfma_q6k_x) are, per
+// AVX lane L, sum sc q6 q8 over the lane's 32 elements, less 32 (sc bsum) of
+// sub-blocks 2 L and 2 L + 1.  sc q6 does not fit an f16's 11 bits, so sc = 16 hi + lo
+// (hi in [-8, 7], lo in [0, 15]): A_lo = lo q6 <= 945, A_hi = hi q6, each exact, one
+// v_mfma_f32_16x16x32_f16 each over the Q4_K form's B chunks (the same elements lie in
+// the same lanes); the bsum term in units of 16, -2 sc bsum, is a product over the
+// 16 bsums in A_hi's accumulator.  Every sum is an integer below 2^23, and
+// fma(16, D_hi, D_lo) is the rounding of the exact integer that the reference's
+// conversion makes.  (In one accumulator the sum could pass 2^24.)  470 VALU
+// instructions per wave and super-block against about 640 of the int8 form, which
+// makes base-64 digits of sc q6 and converts.  The loop reads B one AVX lane ahead
+// behind a scheduling barrier: with the reads hoisted, eight spilled registers
+// made every super-block wait for the copies in flight (869 against 711 us).
+// T = 1024 at H = 4096, K = 1536, N = 4096: 889 (k_mmid_mfma_q6k_x) -> 711 us.
 constexpr int MP_NR = 32;             // activation rows per item (two 16-row tiles)
 constexpr uint32_t MP_HS = 1040;      // LDS bytes per activation DMA instruction (rows i, i + 16, pad)
 constexpr int MP_MAXG = 128;          // active bins the item table holds
@@ -673,9 +688,18 @@ struct MpUnit {
     i32x4 wrsrc;
 };
 
+template <int TYPE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
-    __shared__ __align__(16) uint8_t s_w[MP_ST][MF_M * MF_WS];
+k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
+    constexpr bool Q6 = TYPE == T_Q6_K;
+    // 16-byte chunks of a staged weight row: Q4_K the block's nine; Q6_K the 212 bytes
+    // from the dword at or below the block's start (210-byte blocks start 2 bytes past
+    // a dword in every other row or super-block) as chunks 0 .. 12, chunk 13 bytes
+    // 196 .. 211 (the last dword, holding d, and no byte past it), one of padding
+    constexpr int WCH = Q6 ? 15 : 9;
+    constexpr uint32_t WST = 16u * WCH;                   // LDS stride of a staged row
+    constexpr int WDMA = MF_M * WCH / 64, WDW = (WDMA + 3) / 4;   // copy instructions per stage, per wave
+    __shared__ __align__(16) uint8_t s_w[MP_ST][MF_M * WST];
     __shared__ __align__(16) uint8_t s_h[MP_ST][16 * MP_HS];
     __shared__ __align__(16) uint8_t s_b[MP_ST][MP_NR * 32];   // bsums (f16)
     __shared__ __align__(16) float s_d[MP_ST][MP_NR];
@@ -702,8 +726,8 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
                 const int cnt = m0.active_off[j + 1] - m0.active_off[j];
                 if (cnt >= m0.mfma_min_rows) {
                     const int rem = cnt % MP_NR;
-                    ch = cnt / MP_NR + (rem > 16 ? 1 : 0);
-                    c1 = rem > 0 && rem <= 16 ? 1 : 0;
+                    ch = one_tile ? 0 : cnt / MP_NR + (rem > 16 ? 1 : 0);
+                    c1 = one_tile ? (cnt + 15) / 16 : rem > 0 && rem <= 16 ? 1 : 0;
                 }
             }
             int incl = ch, incl1 = c1;
@@ -761,26 +785,34 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
         }
         g = __builtin_amdgcn_readfirstlane(g);
         const int a0 = s_aoff[g], a1 = s_aoff[g + 1];
-        r.p0 = __builtin_amdgcn_readfirstlane(one ? a0 + MP_NR * ((a1 - a0) / MP_NR) : a0 + MP_NR * (item - s_if[g]));
-        const int ntok = a1 - r.p0;
-        r.ntok = __builtin_amdgcn_readfirstlane(ntok < MP_NR ? ntok : MP_NR);
+        r.p0 = __builtin_amdgcn_readfirstlane(one_tile ? a0 + 16 * (item - s_if1[g])
+                                              : one    ? a0 + MP_NR * ((a1 - a0) / MP_NR)
+                                                       : a0 + MP_NR * (item - s_if[g]));
+        const int ntok = a1 - r.p0, most = one ? 16 : MP_NR;
+        r.ntok = __builtin_amdgcn_readfirstlane(ntok < most ? ntok : most);
         const int mat = __builtin_amdgcn_readfirstlane(s_mat[r.z][g]);
         r.ok = mat >= 0;
         r.r0 = (uint32_t) tile * MF_M;
         const MmidArgs& mz = lp.m[r.z];
         const uint8_t* wt = mz.w + (size_t) (mat >= 0 ? mat : 0) * mz.nb2 + (size_t) r.r0 * mz.nb1;
-        const i32x4 w4 = rsrc_words(wt, (uint32_t) (MF_M * mz.nb1));
+        // (Q6_K: to the end of the last row's last dword)
+        const i32x4 w4 = rsrc_words(wt, ((uint32_t) (MF_M * mz.nb1) + 3u) & ~3u);
         r.wrsrc = i32x4{__builtin_amdgcn_readfirstlane(w4.x), __builtin_amdgcn_readfirstlane(w4.y),
                         __builtin_amdgcn_readfirstlane(w4.z), __builtin_amdgcn_readfirstlane(w4.w)};
         return r;
     };
     // this lane's copy offsets for a unit whose (e, t) pairs are in s_meta[mb]
-    uint32_t woff[3];
+    uint32_t woff[WDW], wrow[Q6 ? WDW : 1];   // Q6_K: wrow the row, woff the chunk's offset
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
+    for (int k = 0; k < WDW; ++k) {
         const int q = 64 * (wave + 4 * k) + lane;
-        const int qc = q < MF_M * 9 ? q : 0;
-        woff[k] = (uint32_t) (qc / 9) * (uint32_t) m0.nb1 + 16u * (uint32_t) (qc % 9);
+        const int qc = q < MF_M * WCH ? q : 0, c = qc % WCH;
+        if constexpr (Q6) {
+            wrow[k] = (uint32_t) (qc / WCH) * (uint32_t) m0.nb1;
+            woff[k] = c < 13 ? 16u * (uint32_t) c : c == 13 ? 196u : 0x40000000u;   // (padding: past the buffer's end)
+        } else {
+            woff[k] = (uint32_t) (qc / WCH) * (uint32_t) m0.nb1 + 16u * (uint32_t) c;
+        }
     }
     auto arow = [&](int mb, int nn) __attribute__((always_inline)) {
         // (32-bit: slot e >= 0 and 1 <= b_ne1 <= 65535 -- mp_ok -- give e % b_ne1 without
@@ -806,15 +838,21 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
         uint32_t ld = (uint32_t) (uintptr_t) s_d[sb], lb = (uint32_t) (uintptr_t) s_b[sb];
         asm volatile("" : "+s"(lw), "+s"(lh), "+s"(ld), "+s"(lb));
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (wv + 4 * k < 9) dma_b128(U.wrsrc, lw + 1024u * (uint32_t) (wv + 4 * k), woff[k], 144u * (uint32_t) i);
+        for (int k = 0; k < WDW; ++k)
+            if (wv + 4 * k < WDMA) {
+                if constexpr (Q6)
+                    dma_b128(U.wrsrc, lw + 1024u * (uint32_t) (wv + 4 * k),
+                             ((wrow[k] + 210u * (uint32_t) i) & ~3u) + woff[k], 0u);
+                else
+                    dma_b128(U.wrsrc, lw + 1024u * (uint32_t) (wv + 4 * k), woff[k], 144u * (uint32_t) i);
+            }
 #pragma unroll
         for (int k = 0; k < 4; ++k) dma_b128(hrsrc, lh + MP_HS * (uint32_t) (wv + 4 * k), ho[k], 512u * (uint32_t) i);
         if (wv == 3 && lane < MP_NR) dma_b32(arsrc, ld, dof, 292u * (uint32_t) i);
         if (wv == 2) dma_b128(brsrc, lb, bof, 32u * (uint32_t) i);   // row lane / 2, half lane % 2
     };
 
-    float acc[2][4][8], accm[2][4][4];
+    float acc[2][4][8], accm[Q6 ? 1 : 2][4][4];
     auto zero = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -823,7 +861,7 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
 #pragma unroll
                 for (int L = 0; L < 8; ++L) acc[t][r][L] = 0.0f;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) accm[t][r][q] = 0.0f;
+                for (int q = 0; q < 4 && !Q6; ++q) accm[t][r][q] = 0.0f;
             }
     };
     uint32_t hmag = 0x64006400u;
@@ -834,7 +872,7 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
     // count tested inside the unrolled loops, the compiler put its wait states for
     // the matrix-core result only on the path that computes the second tile; the
     // branch around it read the first tile's result too early.)
-    auto compute = [&](int sb, auto nbt_c) __attribute__((always_inline)) {
+    auto compute_q4k = [&](int sb, auto nbt_c) __attribute__((always_inline)) {
         constexpr int NBT = decltype(nbt_c)::value;
         const uint8_t* sw = s_w[sb];
         const uint8_t* sh = s_h[sb] + MP_HS * (uint32_t) lr;   // this lane's rows: lr (tile 0), lr + 16 (tile 1)
@@ -842,19 +880,19 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
         // this lane's A row: the 6-bit scales and mins of the 8 sub-blocks (quants.c:2067-2072);
         // the fp16 d / dmin of the four rows of its D registers; the activation rows' d.
         // All read before any is used (one LDS wait: the empty asm takes them all).
-        uint32_t hx0 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 0) * MF_WS);
-        uint32_t hx1 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 1) * MF_WS);
-        uint32_t hx2 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 2) * MF_WS);
-        uint32_t hx3 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 3) * MF_WS);
+        uint32_t hx0 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 0) * WST);
+        uint32_t hx1 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 1) * WST);
+        uint32_t hx2 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 2) * WST);
+        uint32_t hx3 = *(const uint32_t*) (sw + (16 * wave + 4 * gq + 3) * WST);
         float dy0 = sd[lr], dy1 = NBT > 1 ? sd[16 + lr] : 0.0f;
         h4m bs[NBT];
 #pragma unroll
         for (int t = 0; t < NBT; ++t) bs[t] = *(const h4m*) (s_b[sb] + (16 * t + lr) * 32 + 8 * gq);
-        const u32x4m hdr = *(const u32x4m*) (sw + arow_l * MF_WS);
+        const u32x4m hdr = *(const u32x4m*) (sw + arow_l * WST);
         uint32_t s0 = hdr.y, s1 = hdr.z, s2 = hdr.w, sx = hdr.x;
         // and the 8 quant words of its 32-byte group gq (one per AVX lane)
-        u32x4m wq0 = *(const u32x4m*) (sw + arow_l * MF_WS + 16 + 32 * gq);
-        u32x4m wq1 = *(const u32x4m*) (sw + arow_l * MF_WS + 32 + 32 * gq);
+        u32x4m wq0 = *(const u32x4m*) (sw + arow_l * WST + 16 + 32 * gq);
+        u32x4m wq1 = *(const u32x4m*) (sw + arow_l * WST + 32 + 32 * gq);
         asm volatile("" : "+v"(sx), "+v"(s0), "+v"(s1), "+v"(s2), "+v"(hx0), "+v"(hx1), "+v"(hx2), "+v"(hx3), "+v"(dy0),
                      "+v"(dy1), "+v"(wq0), "+v"(wq1));
         const uint32_t wl[8] = {wq0.x, wq0.y, wq0.z, wq0.w, wq1.x, wq1.y, wq1.z, wq1.w};
@@ -948,6 +986,114 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) accm[t][r][q] = __builtin_fmaf(dmin[t][r], Dm[t][4 * q + r], accm[t][r][q]);
     };
+    // Q6_K (see above): super-block i of the unit
+    auto compute_q6k = [&](int sb, int i, auto nbt_c) __attribute__((always_inline)) {
+        constexpr int NBT = decltype(nbt_c)::value;
+        const uint8_t* sh = s_h[sb] + MP_HS * (uint32_t) lr;
+        const float* sd = s_d[sb];
+        const uint32_t nb1 = (uint32_t) m0.nb1, si = 2u * ((uint32_t) i & 1u);
+        const uint32_t off = (((uint32_t) arow_l * nb1) & 2u) ^ si;   // the block's byte offset in its window
+        const uint32_t* wr = (const uint32_t*) (s_w[sb] + arow_l * WST);
+        const int nh = gq >> 1, nib = gq & 1;   // half of this lane's elements, their ql nibble
+        // the block's dword j of half 0, or the one `half` dwords on of half 1 (all below dword 49)
+        auto stream = [&](int j, int half) __attribute__((always_inline)) {
+            const uint32_t* p = wr + half * nh;
+            return __builtin_amdgcn_alignbyte(p[j + 1], p[j], off);
+        };
+        // scales 4 gq .. 4 gq + 3 (this lane's sub-blocks) as f16 digits sc = 16 hi + lo
+        uint32_t scm;
+        {
+            const uint32_t w0 = wr[48 + gq], w1 = wr[gq < 3 ? 49 + gq : 55];
+            scm = __builtin_amdgcn_alignbyte(w1, w0, off);
+        }
+        h2m S_lo[4], S_hi[4], C_lo[4], C_hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t x = __builtin_amdgcn_perm(0u, scm, 0x0c000c00u | (uint32_t) k | ((uint32_t) k << 16));
+            S_lo[k] = h2_bits((x & 0x000F000Fu) | 0x64006400u) - h2m{1024, 1024};
+            S_hi[k] = h2_bits((((x >> 4) & 0x000F000Fu) ^ 0x00080008u) | 0x64006400u) - h2m{1032, 1032};
+            C_lo[k] = S_lo[k] * h2m{-1024, -1024};
+            C_hi[k] = S_hi[k] * h2m{-1024, -1024};
+        }
+        // the bsum term in units of 16: k-slot s of a 32-deep product is bsum s (slots 16
+        // and up hold nothing), so AVX lane L's operand is its two scales times -2 in slots
+        // 2 L, 2 L + 1: word L % 4 of lane group L / 4
+        uint32_t bp[4];
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+            const int j = 48 + 2 * (gq & 1) + (k >> 1);   // scales 8 gq + 2 k .. + 3
+            const uint32_t w = __builtin_amdgcn_alignbyte(wr[j + 1 < 52 ? j + 1 : 55], wr[j], off) ^ 0x80808080u;
+            bp[k] = h2_u32((h2_bits(__builtin_amdgcn_perm(0u, w, 0x0c010c00u) | 0x64006400u) - h2m{1152, 1152}) * h2m{-2, -2});
+            bp[k + 1] = h2_u32((h2_bits(__builtin_amdgcn_perm(0u, w, 0x0c030c02u) | 0x64006400u) - h2m{1152, 1152}) * h2m{-2, -2});
+        }
+        h8m Bb[NBT];
+#pragma unroll
+        for (int t = 0; t < NBT; ++t) {
+            const u32x4m v = *(const u32x4m*) (s_b[sb] + (16 * t + lr) * 32 + 16 * (gq & 1));
+            Bb[t] = __builtin_bit_cast(h8m, gq < 2 ? v : u32x4m{0u, 0u, 0u, 0u});
+        }
+        float d[2][4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t row = (uint32_t) (16 * wave + 4 * gq + r);
+            const uint32_t w = ((const uint32_t*) (s_w[sb] + row * WST))[55];
+            const float xd = h2f((uint16_t) (w >> (8u * (((row * nb1) & 2u) ^ si))));
+#pragma unroll
+            for (int t = 0; t < NBT; ++t) d[t][r] = sd[16 * t + lr] * xd;
+        }
+        f4m Plo[NBT], Phi[NBT];
+        h8m Bc[NBT];
+#pragma unroll
+        for (int t = 0; t < NBT; ++t) Bc[t] = *(const h8m*) (sh + 512 * t + 16 * (8 * gq));
+        auto step = [&](int t, int L) __attribute__((always_inline)) {   // lane L's fp32 steps: (float) (16 hi + lo) is one rounding
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                acc[t][r][L] = __builtin_fmaf(d[t][r], __builtin_fmaf(16.0f, Phi[t][r], Plo[t][r]), acc[t][r][L]);
+        };
+#pragma unroll
+        for (int L = 0; L < 8; ++L) {
+            const uint32_t t0 = stream(128 / 4 + L, 8) << (4 * (1 - nib));
+            const uint32_t q0 = ((stream(L, 16) >> (4 * nib)) & 0x0F0F0F0Fu) | (t0 & 0x30303030u);
+            const uint32_t q1 = ((stream(8 + L, 16) >> (4 * nib)) & 0x0F0F0F0Fu) | ((t0 >> 2) & 0x30303030u);
+            const int k0 = L >> 2, k1 = 2 + (L >> 2);
+            const h2m x0 = h2_bits((q0 & 0x00FF00FFu) | hmag), x1 = h2_bits(((q0 >> 8) & 0x00FF00FFu) | hmag);
+            const h2m x2 = h2_bits((q1 & 0x00FF00FFu) | hmag), x3 = h2_bits(((q1 >> 8) & 0x00FF00FFu) | hmag);
+            auto four = [&](const h2m* S, const h2m* C) __attribute__((always_inline)) {
+                return __builtin_bit_cast(
+                    h8m, u32x4m{h2_u32(__builtin_elementwise_fma(x0, S[k0], C[k0])), h2_u32(__builtin_elementwise_fma(x1, S[k0], C[k0])),
+                                h2_u32(__builtin_elementwise_fma(x2, S[k1], C[k1])), h2_u32(__builtin_elementwise_fma(x3, S[k1], C[k1]))});
+            };
+            const h8m Alo = four(S_lo, C_lo), Ahi = four(S_hi, C_hi);
+            h8m Bn[NBT];
+#pragma unroll
+            for (int t = 0; t < NBT; ++t) Bn[t] = L < 7 ? *(const h8m*) (sh + 512 * t + 16 * (8 * gq + L + 1)) : Bc[t];
+            __builtin_amdgcn_sched_barrier(0);
+            u32x4m ab = {0u, 0u, 0u, 0u};
+            ab[L & 3] = gq == L >> 2 ? bp[L & 3] : 0u;
+            const h8m Abs = __builtin_bit_cast(h8m, ab);
+            f4m Dlo[NBT], Dhi[NBT];
+#pragma unroll
+            for (int t = 0; t < NBT; ++t) Dhi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Abs, Bb[t], f4m{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < NBT; ++t) {
+                Dlo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Alo, Bc[t], f4m{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                Dhi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ahi, Bc[t], Dhi[t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < NBT; ++t) {
+                if (L > 0) step(t, L - 1);
+                Plo[t] = Dlo[t];
+                Phi[t] = Dhi[t];
+                Bc[t] = Bn[t];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < NBT; ++t) step(t, 7);
+    };
+    auto compute = [&](int sb, int i, auto nbt_c) __attribute__((always_inline)) {
+        if constexpr (Q6) compute_q6k(sb, i, nbt_c);
+        else compute_q4k(sb, nbt_c);
+    };
     // hsum_float_8(acc) + ((m0 + m2) + (m1 + m3)) of a finished unit; weight rows
     // r0 + 16 wave + 4 gq .. +3, activation rows lr and 16 + lr
     auto finish = [&](const MpUnit& U, int mb, auto nbt_c) __attribute__((always_inline)) {
@@ -965,8 +1111,12 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
             for (int r = 0; r < 4; ++r) {
                 const float* a = acc[t][r];
                 const float hs = ((a[4] + a[0]) + (a[6] + a[2])) + ((a[5] + a[1]) + (a[7] + a[3]));
-                const float* mm = accm[t][r];
-                o[r] = hs + ((mm[0] + mm[2]) + (mm[1] + mm[3]));
+                if constexpr (Q6) {
+                    o[r] = hs;
+                } else {
+                    const float* mm = accm[t][r];
+                    o[r] = hs + ((mm[0] + mm[2]) + (mm[1] + mm[3]));
+                }
             }
             if (row < U.ntok) {
                 const int e = s_meta[mb][2 * row], tt = s_meta[mb][2 * row + 1];
@@ -1009,7 +1159,7 @@ k_mmid_mfma_q4k_hp(MfLaunch lp, uint32_t nz) {
         // (a wave in its products goes before the other workgroup's wave on the SIMD that
         // is between steps: 740 -> 723 us and 125 -> 119 us per launch, see above)
         __builtin_amdgcn_s_setprio(1);
-        compute(sb, nbt_c);
+        compute(sb, i, nbt_c);
         __builtin_amdgcn_s_setprio(0);
         if (++i == nb) {
             finish(cur, j & 1, nbt_c);
@@ -1512,13 +1662,13 @@ bool mmid_mfma_supported(const MmidArgs& m) {
            ((uintptr_t) m.dst & 15) == 0 && m.act_row_bytes % 4 == 0 && ((uintptr_t) m.act_q & 3) == 0;
 }
 
-// Whether the exact Q4_K form can run on the f16 matrix cores, or the Q8_0 form at
+// Whether the exact Q4_K or Q6_K form can run on the f16 matrix cores, or the Q8_0 form at
 // all (act_h set from an f16 copy of all n_rows activation rows).
 bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows) {
     if (m.type == T_Q8_0)
         return m.mfma_min_rows > 0 && mmid_mfma_supported(m) && n_rows > 0 &&
                (uint64_t) n_rows * (uint64_t) m.K * 2u + 512u < (1ull << 31);
-    return m.type == T_Q4_K && m.mfma_exact && m.mfma_min_rows > 0 && mmid_mfma_supported(m) && n_rows > 0 &&
+    return (m.type == T_Q4_K || m.type == T_Q6_K) && m.mfma_exact && m.mfma_min_rows > 0 && mmid_mfma_supported(m) && n_rows > 0 &&
            (uint64_t) n_rows * (uint64_t) m.K * 2u + 512u < (1ull << 31);
 }
 
@@ -1528,7 +1678,7 @@ bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows) {
 // the environment keeps k_mmid_mfma_q4k_h (a test switch).
 static bool mp_ok(const MfLaunch& lp, int nz) {
     const MmidArgs& a = lp.m[0];
-    if (a.type != T_Q4_K || !a.mfma_exact || !a.act_h || !a.act_hd || a.K < 3 * QK_K || a.max_active > MP_MAXG ||
+    if ((a.type != T_Q4_K && a.type != T_Q6_K) || !a.mfma_exact || !a.act_h || !a.act_hd || a.K < 3 * QK_K || a.max_active > MP_MAXG ||
         a.n_pairs <= 0 || 8 * a.n_pairs >= (int64_t(1) << 31) || a.b_ne1 < 1 || a.b_ne1 > 65535)
         return false;
     if (nz == 2) {
@@ -1560,11 +1710,19 @@ static int launch_mf(const MfLaunch& lp, int nz, hipStream_t stream) {
     if (lp.groups == 0) return 0;
     if (m.type == T_Q8_0) return launch_mf_q80(lp, nz, stream);
     if (mp_ok(lp, nz)) {
-        // at most (items of 32 rows) x tiles x nz units: no more workgroups than that
-        const int64_t units = mf_max_items(m, MP_NR) * (m.N / MF_M) * nz;
+        // at most (items of 32 rows) x tiles x nz units: no more workgroups than that.
+        // Units for half of the workgroups or fewer: items of 16 rows (one tile), twice
+        // the workgroups with half the work each (a 512-row Q6_K projection of 512
+        // tokens: 23.3 -> 17.9 us with the bsum form below 256 registers)
+        int64_t units = mf_max_items(m, MP_NR) * (m.N / MF_M) * nz;
+        const uint32_t one = 2 * units <= (int64_t) mp_grid() ? 1u : 0u;
+        if (one) units = mf_max_items(m, 16) * (m.N / MF_M) * nz;
         const unsigned grid = (unsigned) std::min<int64_t>(units, (int64_t) mp_grid());
         if (grid == 0) return 0;
-        hipLaunchKernelGGL(k_mmid_mfma_q4k_hp, dim3(grid), dim3(256), 0, stream, lp, (uint32_t) nz);
+        if (m.type == T_Q6_K)
+            hipLaunchKernelGGL(k_mmid_mfma_hp<T_Q6_K>, dim3(grid), dim3(256), 0, stream, lp, (uint32_t) nz, one);
+        else
+            hipLaunchKernelGGL(k_mmid_mfma_hp<T_Q4_K>, dim3(grid), dim3(256), 0, stream, lp, (uint32_t) nz, one);
         return hipGetLastError() == hipSuccess ? 0 : -3;
     }
     const unsigned grid = lp.groups * (unsigned) nz;

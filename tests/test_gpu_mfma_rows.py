@@ -1,0 +1,67 @@
+"""GPU parity of the persistent matrix-core kernel (k_mmid_mfma_hp) on block bytes
+of the whole range -- every quant, every 6-bit or int8 scale, extreme activations
+-- bit for bit against the CPU oracle: Q4_K and Q6_K, row lengths whose Q6_K rows
+start on and off a dword, one- and two-tile items of every remainder, launches small
+enough for 16-row items and large enough for 32-row ones, all bins on the matrix
+cores and only those of eight rows or more."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from questwend_amd import ops  # noqa: E402
+from oracle_lib import Oracle, Q4_K, Q6_K  # noqa: E402
+from test_gpu_parity import bits, dev, host  # noqa: E402
+
+
+@pytest.fixture(scope="module", autouse=True)
+def lib_init():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    ops.init(0, 512 << 20)
+
+
+@pytest.fixture(scope="module")
+def orc():
+    return Oracle()
+
+
+def raw_blocks(rng, t, rows, K):
+    nb = K // 256
+    size, d_at = (144, 0) if t == Q4_K else (210, 208)
+    w = rng.integers(0, 256, (rows, nb, size)).astype(np.uint8)
+    d = (rng.standard_normal((rows, nb, 2 if t == Q4_K else 1)) * 1e-3).astype(np.float16)
+    w[..., d_at:d_at + 2 * d.shape[-1]] = d.view(np.uint8).reshape(rows, nb, -1)
+    if t == Q6_K:
+        w[0, :, 192:208] = 0x80          # scales all -128 ...
+        w[0, :, 0:192] = 0xff            # ... times quants all 63
+        w[1, :, 192:208] = 0x7f
+    else:
+        w[0, :, 4:] = 0xff
+    return w.reshape(-1)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("K,N", [(768, 64), (1024, 192), (2048, 64), (2816, 128)])
+@pytest.mark.parametrize("min_rows", [1, 8])
+@pytest.mark.parametrize("many", [False, True])
+def test_raw_blocks(orc, t, K, N, min_rows, many):
+    rng = np.random.default_rng(K + N + min_rows)
+    counts = [1, 8, 15, 16, 17, 31, 32, 33, 48, 49, 7, 64]
+    if many:   # enough units for 32-row items: every expert again, four times over
+        counts = counts * (4 if N > 64 else 8)
+    n_as = len(counts)
+    w = raw_blocks(rng, t, n_as * N, K)
+    ids = rng.permutation(np.repeat(np.arange(n_as), counts)).astype(np.int32).reshape(-1, 1)
+    b = rng.standard_normal((ids.shape[0], 1, K)).astype(np.float32)
+    b[0] = np.float32(3.0)               # a row of equal values: quants all -127
+    b[1, 0, 256:512] = 0.0
+    prev = ops.set_mfma_min_rows(min_rows)
+    try:
+        got = host(ops.mul_mat_id(t, dev(w), K, N, n_as, dev(b), dev(ids)))
+    finally:
+        ops.set_mfma_min_rows(prev)
+    assert np.array_equal(bits(got), bits(orc.mul_mat_id(t, K, N, n_as, w, b, ids)))
