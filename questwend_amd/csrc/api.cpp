@@ -698,7 +698,11 @@ int qwmoe_attn_seg(void* stream, const qwmoe_attn_layer* L, const float* h, int6
             }
     };
     mfma_f16_reserve(ar, mo, T);
-    if ((rc = qw::launch_group_dense(rows, active, active_off, n_active, T, st))) return rc;
+    qw::RowGroups grp{};
+    grp.rows = rows;
+    grp.active = active;
+    grp.active_off = active_off;
+    grp.n_active = n_active;
     const size_t hb = (size_t) H * 4;
     // attn_norm, then the projections' input quantized: one launch when every
     // projection reads Q8_K (the K-quants), the same bits as the two steps
@@ -706,8 +710,9 @@ int qwmoe_attn_seg(void* stream, const qwmoe_attn_layer* L, const float* h, int6
     float* hxd;
     if (all_q8K) {
         copy_of(xq, hx, hxd);
-        if ((rc = qw::launch_rms_norm_q8K(h, H, T, rms_eps, L->attn_norm, xq, st, hx))) return rc;
+        if ((rc = qw::launch_rms_norm_q8K(h, H, T, rms_eps, L->attn_norm, xq, st, hx, nullptr, &grp))) return rc;
     } else {
+        if ((rc = qw::launch_row_groups(grp, T, st))) return rc;
         if ((rc = qw::launch_rms_norm(h, cur, H, T, rms_eps, st, L->attn_norm))) return rc;
         const int vt[3] = {vqt, vkt, vvt};
         uint8_t* xb[3] = {xq, xk, xv};
@@ -806,7 +811,7 @@ int qwmoe_gdn_seg(void* stream, const qwmoe_gdn_layer* L, const float* h, int64_
     float* o = ar.take<float>((size_t) (d_inner * T));
     float* y = ar.take<float>((size_t) (d_inner * T));
     float* proj = ar.take<float>((size_t) (H * T));
-    // one bin per token for the H_v-row projections (beta, alpha)
+    // bins of a few tokens for the H_v-row projections (beta, alpha)
     int32_t* trows = ar.take<int32_t>((size_t) (2 * T));
     int32_t* tactive = ar.take<int32_t>((size_t) T);
     int32_t* toff = ar.take<int32_t>((size_t) (T + 1));
@@ -819,43 +824,70 @@ int qwmoe_gdn_seg(void* stream, const qwmoe_gdn_layer* L, const float* h, int64_
     int vt[4] = {qw::vec_dot_type(L->type_qkv), qw::vec_dot_type(L->type_gate), qw::vec_dot_type(L->type_beta),
                  qw::vec_dot_type(L->type_alpha)};
     uint8_t* xq[4] = {nullptr, nullptr, nullptr, nullptr};
+    uint8_t *x8K = nullptr, *x80 = nullptr;
     size_t xr[4];
     for (int i = 0; i < 4; ++i) {
         xr[i] = qwmoe_row_size(vt[i], H);
-        for (int j = 0; j < i; ++j)
-            if (vt[j] == vt[i]) xq[i] = xq[j];
-        if (!xq[i] && !(xq[i] = ar.take<uint8_t>(xr[i] * (size_t) T + 64))) return QWMOE_ERR_WORKSPACE;
+        uint8_t*& x = vt[i] == qw::T_Q8_K ? x8K : x80;
+        if (!x && !(x = ar.take<uint8_t>(xr[i] * (size_t) T + 64))) return QWMOE_ERR_WORKSPACE;
+        xq[i] = x;
     }
     const int vot = qw::vec_dot_type(L->type_out);
     const size_t ro = qwmoe_row_size(vot, d_inner);
     uint8_t* yq = ar.take<uint8_t>(ro * (size_t) T + 64);
     if (!yq) return QWMOE_ERR_WORKSPACE;
-    if ((rc = qw::launch_group_dense(rows, active, active_off, n_active, T, st))) return rc;
-    if ((rc = qw::launch_gdn_group_tokens(trows, tactive, toff, tn, tslot, T, st))) return rc;
     const size_t hb = (size_t) H * 4;
-    if ((rc = qw::launch_rms_norm(h, cur, H, T, rms_eps, st, L->attn_norm))) return rc;
-    for (int i = 0; i < 4; ++i) {
-        bool done = false;
-        for (int j = 0; j < i; ++j) done = done || xq[j] == xq[i];
-        if (!done && (rc = qw::launch_quantize_act(vt[i], cur, H, 1, T, hb, hb, xq[i], st))) return rc;
-    }
-    auto proj_launch = [&](int type, const void* w, size_t nb1, int64_t K, int64_t N, const uint8_t* xb, size_t xrow,
-                           float* dst) {
+    auto proj_args = [&](int type, const void* w, size_t nb1, int64_t K, int64_t N, const uint8_t* xb, size_t xrow,
+                         float* dst) {
         const size_t ob = (size_t) N * 4;
-        qw::MmidArgs m = mmid_args(type, w, K, N, 1, nb1, nb1 * (size_t) N, xb, 1, xrow, rows, active, active_off,
-                                   n_active, 1, nullptr, 0, dst, ob, ob, T, T);
-        if (int r = mfma_f16_prep(ar, m, T, st)) return r;
-        return mmid_launch(m, st);
+        return mmid_args(type, w, K, N, 1, nb1, nb1 * (size_t) N, xb, 1, xrow, rows, active, active_off, n_active, 1,
+                         nullptr, 0, dst, ob, ob, T, T);
     };
-    if ((rc = proj_launch(L->type_qkv, L->w_qkv, L->w_qkv_nb1, H, conv_ch, xq[0], xr[0], qkv))) return rc;
-    if ((rc = proj_launch(L->type_gate, L->w_gate, L->w_gate_nb1, H, d_inner, xq[1], xr[1], z))) return rc;
-    {   // beta and alpha: a workgroup per token (and both in one launch when they share a type)
+    qw::MmidArgs mqkv = proj_args(L->type_qkv, L->w_qkv, L->w_qkv_nb1, H, conv_ch, xq[0], xr[0], qkv);
+    qw::MmidArgs mz = proj_args(L->type_gate, L->w_gate, L->w_gate_nb1, H, d_inner, xq[1], xr[1], z);
+    qw::MmidArgs mo = proj_args(L->type_out, L->w_out, L->w_out_nb1, d_inner, H, yq, ro, proj);
+    // the f16 copies the matrix cores read, written by the launches that quantize
+    mfma_f16_reserve(ar, mqkv, T);
+    if (mqkv.act_h && mz.act_q == mqkv.act_q && qw::mmid_mfma_h_ok(mz, T)) {
+        mz.act_h = mqkv.act_h;
+        mz.act_hd = mqkv.act_hd;
+    } else {
+        mfma_f16_reserve(ar, mz, T);
+    }
+    mfma_f16_reserve(ar, mo, T);
+    auto copy_of = [&](const uint8_t* x, uint16_t*& h, float*& hd) {
+        const qw::MmidArgs* m = mqkv.act_q == x && mqkv.act_h ? &mqkv : mz.act_q == x && mz.act_h ? &mz : nullptr;
+        h = m ? (uint16_t*) m->act_h : nullptr;
+        hd = m ? (float*) m->act_hd : nullptr;
+    };
+    qw::RowGroups grp{rows, active, active_off, n_active, trows, tactive, toff, tn, tslot, T >= 64 ? 4 : 1};
+    uint16_t* hx;
+    float* hxd;
+    copy_of(x80, hx, hxd);
+    if (x8K && H % 256 == 0 && !((uintptr_t) L->attn_norm & 15) && !hx) {
+        // attn_norm, both quantizations of its rows and the groupings in one launch
+        copy_of(x8K, hx, hxd);
+        if ((rc = qw::launch_rms_norm_q8K(h, H, T, rms_eps, L->attn_norm, x8K, st, hx, x80, &grp))) return rc;
+    } else {
+        if ((rc = qw::launch_row_groups(grp, T, st))) return rc;
+        if ((rc = qw::launch_rms_norm(h, cur, H, T, rms_eps, st, L->attn_norm))) return rc;
+        for (uint8_t* x : {x8K, x80}) {
+            copy_of(x, hx, hxd);
+            if (x && (rc = qw::launch_quantize_act(x == x8K ? qw::T_Q8_K : qw::T_Q8_0, cur, H, 1, T, hb, hb, x, st, hx, hxd)))
+                return rc;
+        }
+    }
+    if ((rc = mmid_launch(mqkv, st))) return rc;
+    if ((rc = mmid_launch(mz, st))) return rc;
+    {   // beta and alpha: a workgroup per bin (and both in one launch when they share a type)
+        const int64_t nb = (T + grp.tpb - 1) / grp.tpb;
         auto small = [&](int type, const void* w, size_t nb1, const uint8_t* xb, size_t xrow, float* dst) {
-            return mmid_args(type, w, H, Hv, 1, nb1, nb1 * (size_t) Hv, xb, 1, xrow, trows, tactive, toff, tn, T,
-                             tslot, T, dst, 0, (size_t) Hv * 4, 1, T);
+            return mmid_args(type, w, H, Hv, 1, nb1, nb1 * (size_t) Hv, xb, 1, xrow, trows, tactive, toff, tn, nb,
+                             tslot, nb, dst, 0, (size_t) Hv * 4, grp.tpb, T);
         };
-        const qw::MmidArgs mb = small(L->type_beta, L->w_beta, L->w_beta_nb1, xq[2], xr[2], braw);
-        const qw::MmidArgs ma = small(L->type_alpha, L->w_alpha, L->w_alpha_nb1, xq[3], xr[3], araw);
+        qw::MmidArgs mb = small(L->type_beta, L->w_beta, L->w_beta_nb1, xq[2], xr[2], braw);
+        qw::MmidArgs ma = small(L->type_alpha, L->w_alpha, L->w_alpha_nb1, xq[3], xr[3], araw);
+        mb.mfma_min_rows = ma.mfma_min_rows = 0;
         if (!(mb.type == ma.type && qw::launch_mmid_gemv2(mb, ma, st) == 0)) {
             if ((rc = mmid_launch(mb, st))) return rc;
             if ((rc = mmid_launch(ma, st))) return rc;
@@ -884,10 +916,14 @@ int qwmoe_gdn_seg(void* stream, const qwmoe_gdn_layer* L, const float* h, int64_
     a.bg = bg;
     a.o = o;
     a.y = y;
+    a.y_q8K = vot == qw::T_Q8_K ? yq : nullptr;   // the gated norm quantizes its rows
+    a.y_h = vot == qw::T_Q8_K ? (uint16_t*) mo.act_h : nullptr;
     if ((rc = qw::launch_gdn_core(a, st))) return rc == -2 ? QWMOE_ERR_UNSUPPORTED : QWMOE_ERR_HIP;
     const size_t yb = (size_t) d_inner * 4;
-    if ((rc = qw::launch_quantize_act(vot, y, d_inner, 1, T, yb, yb, yq, st))) return rc;
-    if ((rc = proj_launch(L->type_out, L->w_out, L->w_out_nb1, d_inner, H, yq, ro, proj))) return rc;
+    if (vot != qw::T_Q8_K && (rc = qw::launch_quantize_act(vot, y, d_inner, 1, T, yb, yb, yq, st, (uint16_t*) mo.act_h,
+                                                           (float*) mo.act_hd)))
+        return rc;
+    if ((rc = mmid_launch(mo, st))) return rc;
     return qw::launch_add_rms_norm_mul(proj, h, attn_resid, ffn_in, H, T, rms_eps, L->ffn_norm, st);
 }
 

@@ -427,14 +427,48 @@ __global__ void __launch_bounds__(256) k_add_rms_norm_mul(const float* __restric
     for (int64_t i = threadIdx.x; i < n; i += 256) out[o + i] = (resid[o + i] * scale) * w[i];
 }
 
+// Row t's part of the groupings (one thread per row).
+__device__ __forceinline__ void row_groups(const RowGroups& g, int t, int T) {
+    if (g.rows) {
+        g.rows[2 * t] = 0;
+        g.rows[2 * t + 1] = t;
+        if (t == 0) {
+            g.active[0] = 0;
+            g.active_off[0] = 0;
+            g.active_off[1] = T;
+            *g.n_active = 1;
+        }
+    }
+    if (g.trows) {
+        g.trows[2 * t] = 0;
+        g.trows[2 * t + 1] = t;
+        const int nb = (T + g.tpb - 1) / g.tpb;
+        if (t % g.tpb == 0) {
+            g.tactive[t / g.tpb] = t / g.tpb;
+            g.toff[t / g.tpb] = t;
+            g.tslot[t / g.tpb] = 0;
+        }
+        if (t == 0) {
+            g.toff[nb] = T;
+            *g.tn = nb;
+        }
+    }
+}
+__global__ void k_row_groups(RowGroups g, int T) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < T) row_groups(g, t, T);
+}
+
 // attn_norm and the Q8_K quantisation of its output in one launch, one
 // 256-thread block per row of n (a multiple of 256): the sum of squares and
 // scale exactly as k_rms_norm, each value (x * scale) * w as it writes them, and
 // each 256-value block quantized by one wave as k_quant_q8K does.
 __global__ void __launch_bounds__(256) k_rms_norm_q8K(const float* __restrict__ x, int64_t n, float eps,
                                                       const float* __restrict__ w, BlockQ8_K* __restrict__ dst,
-                                                      _Float16* __restrict__ hout) {
+                                                      _Float16* __restrict__ hout, BlockQ8_0* __restrict__ dst0,
+                                                      RowGroups g) {
     __shared__ double part[4];
+    if (threadIdx.x == 0) row_groups(g, blockIdx.x, gridDim.x);
     const float* xr = x + (int64_t) blockIdx.x * n;
     double s = 0.0;
     for (int64_t i = threadIdx.x; i < n; i += 256) {
@@ -456,6 +490,8 @@ __global__ void __launch_bounds__(256) k_rms_norm_q8K(const float* __restrict__ 
         const int64_t blk = (int64_t) blockIdx.x * nb + ib;
         quant_q8K_wave(v, lane, dst + blk, hout ? hout + (size_t) blk * QK_K : nullptr,
                        hout ? hout + (size_t) (nb * gridDim.x) * QK_K + (size_t) blk * 16 : nullptr);
+        if (dst0)
+            quant_q80_lane8(float4{v[0], v[1], v[2], v[3]}, true, 8 * blk + (lane >> 3), lane & 7, dst0, nullptr, nullptr);
     }
 }
 
@@ -499,11 +535,17 @@ int launch_attn_core(const AttnArgs& a, hipStream_t st) {
 }
 
 int launch_rms_norm_q8K(const float* x, int64_t n, int64_t rows, float eps, const float* w, void* dst,
-                        hipStream_t st, uint16_t* h_out) {
+                        hipStream_t st, uint16_t* h_out, void* dst0, const RowGroups* g) {
     if (n % QK_K || !w || (((uintptr_t) x | (uintptr_t) w) & 15)) return -2;
     if (rows == 0) return 0;
     hipLaunchKernelGGL(k_rms_norm_q8K, dim3((unsigned) rows), dim3(256), 0, st, x, n, eps, w, (BlockQ8_K*) dst,
-                       (_Float16*) h_out);
+                       (_Float16*) h_out, (BlockQ8_0*) dst0, g ? *g : RowGroups{});
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+int launch_row_groups(const RowGroups& g, int64_t T, hipStream_t st) {
+    if (T <= 0 || T >= (int64_t(1) << 30)) return -2;
+    hipLaunchKernelGGL(k_row_groups, dim3((unsigned) ((T + 255) / 256)), dim3(256), 0, st, g, (int) T);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

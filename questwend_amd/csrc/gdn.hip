@@ -28,31 +28,52 @@ namespace qw {
 namespace {
 
 constexpr int GS = 128;        // state size S (ssm.state_size of the Qwen3-Next family)
-constexpr int GJB = 32;        // state rows j per workgroup of the recurrence (8 lanes per row)
+constexpr int GJB = 16;        // state rows j per workgroup of the recurrence (16 lanes per row)
 
-// Thread (channel c, token t): the d_conv-tap window over [conv_state | qkv
-// rows] ending at token t, then SiLU.  The inputs x_0 .. x_{d_conv-2} are the
-// state, x_{d_conv-1+t} = qkv[t][c].
+// Four channels and CT tokens per thread: the DC-tap windows over [conv_state |
+// qkv rows] ending at each token (x_0 .. x_{DC-2} are the state, x_{DC-1+t} =
+// qkv[t]), then SiLU.  A row of x is loaded once for the DC tokens it reaches.
+// T = 300, 8192 channels: 14.7 (a thread per output) -> 10.5 us.
+constexpr int CT = 4;
+template <int DC>
 __global__ void __launch_bounds__(256) k_gdn_conv(GdnArgs a) {
-    const int64_t c = (int64_t) blockIdx.x * 256 + threadIdx.x;
-    const int t = blockIdx.y, dc = a.d_conv;
-    if (c >= a.conv_ch) return;
-    float s = 0.0f;
+    const int64_t c = ((int64_t) blockIdx.x * 64 + (threadIdx.x & 63)) * 4;
+    const int t0 = ((int) blockIdx.y * 4 + (int) (threadIdx.x >> 6)) * CT;
+    if (c >= a.conv_ch || t0 >= a.T) return;
+    float4 x[CT + DC - 1];
 #pragma unroll
-    for (int j = 0; j < GDN_MAX_CONV; ++j)
-        if (j < dc) {
-            const int xi = t + j;   // window element j is x_{t + j}
-            const float x = xi < dc - 1 ? a.conv_state[c * (dc - 1) + xi]
-                                        : a.qkv[(int64_t) (xi - (dc - 1)) * a.conv_ch + c];
-            s = __builtin_fmaf(x, a.conv1d[c * dc + j], s);
+    for (int i = 0; i < CT + DC - 1; ++i) {
+        const int xi = t0 + i;
+        if (xi < DC - 1) {
+            const float* s = a.conv_state + c * (DC - 1) + xi;
+            x[i] = float4{s[0], s[DC - 1], s[2 * (DC - 1)], s[3 * (DC - 1)]};
+        } else {
+            x[i] = *(const float4*) (a.qkv + (int64_t) min(xi - (DC - 1), a.T - 1) * a.conv_ch + c);
         }
-    a.conv[(int64_t) t * a.conv_ch + c] = v_silu(s);
+    }
+    float w[4][DC];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < DC; ++j) w[q][j] = a.conv1d[(c + q) * DC + j];
+#pragma unroll
+    for (int k = 0; k < CT; ++k) {
+        if (t0 + k >= a.T) break;
+        float4 s = float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < DC; ++j) {
+            s.x = __builtin_fmaf(x[k + j].x, w[0][j], s.x);
+            s.y = __builtin_fmaf(x[k + j].y, w[1][j], s.y);
+            s.z = __builtin_fmaf(x[k + j].z, w[2][j], s.z);
+            s.w = __builtin_fmaf(x[k + j].w, w[3][j], s.w);
+        }
+        *(float4*) (a.conv + (int64_t) (t0 + k) * a.conv_ch + c) = float4{v_silu(s.x), v_silu(s.y), v_silu(s.z), v_silu(s.w)};
+    }
 }
 
 // The conv state after the call: x_T .. x_{T+d_conv-2}, one thread per channel
-// (after k_gdn_conv, which reads the old state).
-__global__ void __launch_bounds__(256) k_gdn_conv_state(GdnArgs a) {
-    const int64_t c = (int64_t) blockIdx.x * 256 + threadIdx.x;
+// (in the launch after k_gdn_conv, which reads the old state).
+__device__ __forceinline__ void gdn_conv_state(const GdnArgs& a, int64_t c) {
     if (c >= a.conv_ch) return;
     const int dc = a.d_conv, T = a.T;
     float nw[GDN_MAX_CONV];
@@ -67,11 +88,15 @@ __global__ void __launch_bounds__(256) k_gdn_conv_state(GdnArgs a) {
         if (j < dc - 1) a.conv_state[c * (dc - 1) + j] = nw[j];
 }
 
-// Block (t, key head): q and k of that head divided by max(||.||, eps) (the
-// sum of squares in double, as ggml_l2_norm); block (t, H_k) instead forms
-// beta and g of every value head.
+// Block t (H_k + 1) + hk: q and k of token t's key head hk divided by max(||.||,
+// eps) (the sum of squares in double, as ggml_l2_norm); with hk = H_k instead beta
+// and g of every value head; the blocks past the tokens' the conv state.
 __global__ void __launch_bounds__(GS) k_gdn_prep(GdnArgs a) {
-    const int t = blockIdx.x, hk = blockIdx.y, i = threadIdx.x;
+    const int per = a.H_k + 1, t = blockIdx.x / per, hk = blockIdx.x % per, i = threadIdx.x;
+    if (t >= a.T) {
+        gdn_conv_state(a, (int64_t) ((int) blockIdx.x - a.T * per) * GS + i);
+        return;
+    }
     __shared__ double s_red[2][GS / 64];
     if (hk == a.H_k) {
         for (int hv = i; hv < a.H_v; hv += GS) {
@@ -107,154 +132,209 @@ __global__ void __launch_bounds__(GS) k_gdn_prep(GdnArgs a) {
     a.kn[((int64_t) t * a.H_k + hk) * GS + i] = k * sck;
 }
 
-// The recurrence.  Workgroup (value head hv, rows j0 .. j0 + 31 of its state
-// M = S^T): 8 lanes per row, each holding 16 of its 128 columns in registers
-// for all tokens.  Per token, as ggml: M *= exp(g); delta_j = (v_j - M_j . k) beta;
-// M_j += delta_j k; o_j = (M_j . q) / sqrt(S).  A row's dots are reduced over
-// its 8 lanes by DPP (quad xor 1, xor 2, half-row mirror).  Rows are
-// independent, so the 4 row blocks of a head run in parallel.  Tokens go in
-// blocks of GTB: the block's q, k (its key head), v (the workgroup's rows), beta
-// and g sit in LDS, and the next block's are loaded into registers while the
-// current block is applied, so the chain over the tokens waits on LDS, not on
-// a memory round trip per token.
+// The recurrence, four tokens at a time.  Workgroup (value head hv, rows j0 .. j0 +
+// GJB - 1 of its state M = S^T): 16 lanes per row, each holding 8 of its 128 columns
+// in registers for all tokens.  Per token ggml has M *= e (e = exp(g)); delta_j =
+// (v_j - M_j . k) beta; M_j += delta_j k; o_j = (M_j . q) / sqrt(S).  Token by token
+// that is one row reduction after another, 740 cycles each with a wave per SIMD.  From
+// the state M before tokens 1 .. 4 (E_b = e_1 .. e_b, E_{a,b} = e_{a+1} .. e_b),
+//     M k at token b       = E_b (M . k_b) + sum_{a < b}  E_{a,b} delta_a (k_a . k_b)
+//     o at token b sqrt(S) = E_b (M . q_b) + sum_{a <= b} E_{a,b} delta_a (k_a . q_b)
+//     M after              = E_4 M + sum_a E_{a,4} delta_a k_a
+// so the eight reductions over the row's 16 lanes are independent, and what depends
+// token on token is a few scalar steps.  The products P = E_{a,b} (k_a . k_b) and Q =
+// E_{a,b} (k_a . q_b) are the same for every row: formed once per workgroup and block
+// of GTB tokens, in LDS.  All in fp32 (the reference's sums in another order).
+//
+// Tokens go in blocks of GTB: q, k (the key head), v (the workgroup's rows), beta and
+// g sit in LDS, the next block's are loaded into registers while the current block
+// is applied.  Tokens past T have k = 0, e = 1 and delta = 0: they change nothing.
+// H_v = 32, T = 300: 101 us (8 lanes per row, token by token) -> 74 us (what is left: LDS reads, 24 of 16 bytes per
+// lane and step with one workgroup per CU; reading a step ahead changed nothing).
+typedef float fx4 __attribute__((ext_vector_type(4)));   // (arrays of it stay in registers)
 constexpr int GTB = 32;   // tokens per staged block
+constexpr int GC = 4;     // tokens per step
 __global__ void __launch_bounds__(256) k_gdn_delta(GdnArgs a) {
-    const int hv = blockIdx.x, tid = threadIdx.x, r = tid >> 3, l = tid & 7;
+    const int hv = blockIdx.x, tid = threadIdx.x, r = tid >> 4, l = tid & 15;
     const int j0 = blockIdx.y * GJB, j = j0 + r, hk = hv % a.H_k;
     __shared__ __align__(16) float s_q[GTB][GS];
     __shared__ __align__(16) float s_k[GTB][GS];
-    __shared__ float s_v[GTB][GJB];
-    __shared__ float s_b[GTB], s_g[GTB];
-    float* st = a.state + ((int64_t) hv * GS + j) * GS + 16 * l;
-    float4 m0 = *(const float4*) st, m1 = *(const float4*) (st + 4), m2 = *(const float4*) (st + 8),
-           m3 = *(const float4*) (st + 12);
+    __shared__ __align__(16) float s_v[GJB][GTB];              // [row][token]
+    __shared__ __align__(16) float s_b[GTB], s_e[GTB];
+    __shared__ __align__(16) float s_S[GTB / GC][24];          // per step: P (6), Q (10), E_b (4), E_{a,4} (4)
+    static_assert(GJB * 16 == 256 && GTB * GS / 4 == 4 * 256 && GTB * GJB == 2 * 256, "the loads' split over 256 threads");
+    float* st = a.state + ((int64_t) hv * GS + j) * GS + 4 * l;   // columns 4 l .. + 3 and 64 + 4 l .. + 3
+    fx4 m0 = *(const fx4*) st, m1 = *(const fx4*) (st + 64);
     const float scale = 1.0f / sqrtf((float) GS);
     const int64_t vbase = 2 * (int64_t) a.H_k * GS + (int64_t) hv * GS + j0;
-    // this thread's share of a block: float4 f = tid + 256 u of q and of k
-    // (token f / 32, columns 4 (f % 32) ..), v of (token f / 32, row f % 32) for
-    // f = tid + 256 u, and beta or g (tid < 2 GTB); named registers, not
-    // arrays, so that nothing lands in scratch
-    static_assert(GTB * GS / 4 == 4 * 256 && GTB * GJB == 4 * 256, "four float4 of q, k and four v per thread");
-    float4 rq0, rq1, rq2, rq3, rk0, rk1, rk2, rk3;
-    float rv0, rv1, rv2, rv3, rbg = 0.0f;
+    fx4 rq[4], rk[4];
+    float rv[2], rbg = 0.0f;
     const int64_t qcol = 4 * (tid % (GS / 4));
-    auto tok = [&](int t) { return (int64_t) (t < a.T ? t : a.T - 1); };
-#define GDN_LOAD(tb_)                                                                                          \
-    do {                                                                                                     \
-        const int t0_ = (tb_) + tid / (GS / 4);                                                              \
-        rq0 = *(const float4*) (a.qn + (tok(t0_) * a.H_k + hk) * GS + qcol);                                 \
-        rq1 = *(const float4*) (a.qn + (tok(t0_ + 8) * a.H_k + hk) * GS + qcol);                             \
-        rq2 = *(const float4*) (a.qn + (tok(t0_ + 16) * a.H_k + hk) * GS + qcol);                            \
-        rq3 = *(const float4*) (a.qn + (tok(t0_ + 24) * a.H_k + hk) * GS + qcol);                            \
-        rk0 = *(const float4*) (a.kn + (tok(t0_) * a.H_k + hk) * GS + qcol);                                 \
-        rk1 = *(const float4*) (a.kn + (tok(t0_ + 8) * a.H_k + hk) * GS + qcol);                             \
-        rk2 = *(const float4*) (a.kn + (tok(t0_ + 16) * a.H_k + hk) * GS + qcol);                            \
-        rk3 = *(const float4*) (a.kn + (tok(t0_ + 24) * a.H_k + hk) * GS + qcol);                            \
-        const int tv_ = (tb_) + tid / GJB;                                                                   \
-        rv0 = a.conv[tok(tv_) * a.conv_ch + vbase + tid % GJB];                                              \
-        rv1 = a.conv[tok(tv_ + 8) * a.conv_ch + vbase + tid % GJB];                                          \
-        rv2 = a.conv[tok(tv_ + 16) * a.conv_ch + vbase + tid % GJB];                                         \
-        rv3 = a.conv[tok(tv_ + 24) * a.conv_ch + vbase + tid % GJB];                                         \
-        if (tid < 2 * GTB) rbg = a.bg[(tok((tb_) + (tid >> 1)) * a.H_v + hv) * 2 + (tid & 1)];               \
-    } while (0)
-    auto red8 = [](float x) __attribute__((always_inline)) {
-        x = x + dpp_f<DPP_XOR1>(x);
-        x = x + dpp_f<DPP_XOR2>(x);
-        return x + dpp_f<DPP_HALF_MIRROR>(x);
+    auto load = [&](int tb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t t = min(tb + tid / (GS / 4) + 8 * u, a.T - 1);
+            rq[u] = *(const fx4*) (a.qn + (t * a.H_k + hk) * GS + qcol);
+            rk[u] = *(const fx4*) (a.kn + (t * a.H_k + hk) * GS + qcol);
+            if (tb + tid / (GS / 4) + 8 * u >= a.T) rk[u] = fx4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            rv[u] = a.conv[(int64_t) min(tb + tid / GJB + 16 * u, a.T - 1) * a.conv_ch + vbase + tid % GJB];
+        if (tid < 2 * GTB) {
+            const int t = tb + (tid >> 1);
+            rbg = t < a.T ? a.bg[((int64_t) t * a.H_v + hv) * 2 + (tid & 1)] : 0.0f;
+        }
     };
-    GDN_LOAD(0);
+    auto dot4 = [](fx4 x, fx4 y, float s) __attribute__((always_inline)) {
+        s = __builtin_fmaf(x.x, y.x, s);
+        s = __builtin_fmaf(x.y, y.y, s);
+        s = __builtin_fmaf(x.z, y.z, s);
+        return __builtin_fmaf(x.w, y.w, s);
+    };
+    load(0);
     for (int tb = 0; tb < a.T; tb += GTB) {
         __syncthreads();   // the previous block is consumed
-        {
-            const int tq = tid / (GS / 4), tv = tid / GJB;
-            *(float4*) &s_q[tq][qcol] = rq0;
-            *(float4*) &s_q[tq + 8][qcol] = rq1;
-            *(float4*) &s_q[tq + 16][qcol] = rq2;
-            *(float4*) &s_q[tq + 24][qcol] = rq3;
-            *(float4*) &s_k[tq][qcol] = rk0;
-            *(float4*) &s_k[tq + 8][qcol] = rk1;
-            *(float4*) &s_k[tq + 16][qcol] = rk2;
-            *(float4*) &s_k[tq + 24][qcol] = rk3;
-            s_v[tv][tid % GJB] = rv0;
-            s_v[tv + 8][tid % GJB] = rv1;
-            s_v[tv + 16][tid % GJB] = rv2;
-            s_v[tv + 24][tid % GJB] = rv3;
-            if (tid < 2 * GTB) {
-                if (tid & 1) s_g[tid >> 1] = rbg;
-                else s_b[tid >> 1] = rbg;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            *(fx4*) &s_q[tid / (GS / 4) + 8 * u][qcol] = rq[u];
+            *(fx4*) &s_k[tid / (GS / 4) + 8 * u][qcol] = rk[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) s_v[tid % GJB][tid / GJB + 16 * u] = rv[u];
+        if (tid < 2 * GTB) {
+            if (tid & 1) s_e[tid >> 1] = expf(rbg);
+            else s_b[tid >> 1] = rbg;
+        }
+        __syncthreads();
+        if (tb + GTB < a.T) load(tb + GTB);
+        {   // P and Q: 8 lanes per token b of a step, lane p its columns 4 p + 32 i .. + 3
+            const int grp = tid >> 3, p = tid & 7, c = grp >> 2, b = grp & 3, t0 = GC * c;
+            float dk[GC], dq[GC];
+            fx4 kb[4], qb[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                kb[i] = *(const fx4*) &s_k[t0 + b][4 * p + 32 * i];
+                qb[i] = *(const fx4*) &s_q[t0 + b][4 * p + 32 * i];
+            }
+#pragma unroll
+            for (int x = 0; x < GC; ++x) {
+                dk[x] = dq[x] = 0.0f;
+                if (x <= b) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const fx4 ka = *(const fx4*) &s_k[t0 + x][4 * p + 32 * i];
+                        dk[x] = dot4(ka, kb[i], dk[x]);
+                        dq[x] = dot4(ka, qb[i], dq[x]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < GC; ++x) {
+                dk[x] += dpp_f<DPP_XOR1>(dk[x]);
+                dq[x] += dpp_f<DPP_XOR1>(dq[x]);
+                dk[x] += dpp_f<DPP_XOR2>(dk[x]);
+                dq[x] += dpp_f<DPP_XOR2>(dq[x]);
+                dk[x] += dpp_f<DPP_HALF_MIRROR>(dk[x]);
+                dq[x] += dpp_f<DPP_HALF_MIRROR>(dq[x]);
+            }
+            // E_{x,b} as the product of the decays between
+            float E[GC], Eb = 1.0f, E4 = 1.0f;
+#pragma unroll
+            for (int x = 0; x < GC; ++x) {
+                E[x] = 1.0f;
+#pragma unroll
+                for (int y = 1; y < GC; ++y) {
+                    if (y > x && y <= b) E[x] *= s_e[t0 + y];
+                }
+                if (x <= b) Eb *= s_e[t0 + x];
+                if (x > b) E4 *= s_e[t0 + x];
+            }
+            if (p == 0) {
+#pragma unroll
+                for (int x = 0; x < GC; ++x) {   // P of (a, b) at b (b - 1) / 2 + a, Q of (a, b) at 6 + b (b + 1) / 2 + a
+                    if (x < b) s_S[c][b * (b - 1) / 2 + x] = E[x] * dk[x];
+                    if (x <= b) s_S[c][6 + b * (b + 1) / 2 + x] = E[x] * dq[x];
+                }
+                s_S[c][16 + b] = Eb;
+                s_S[c][20 + b] = E4;
             }
         }
         __syncthreads();
-        if (tb + GTB < a.T) GDN_LOAD(tb + GTB);
         const int nt = a.T - tb < GTB ? a.T - tb : GTB;
-        for (int tt = 0; tt < nt; ++tt) {
-            const float e = expf(s_g[tt]);
-            const float* qp = &s_q[tt][16 * l];
-            const float* kp = &s_k[tt][16 * l];
-            const float4 q0 = *(const float4*) qp, q1 = *(const float4*) (qp + 4), q2 = *(const float4*) (qp + 8),
-                         q3 = *(const float4*) (qp + 12);
-            const float4 k0 = *(const float4*) kp, k1 = *(const float4*) (kp + 4), k2 = *(const float4*) (kp + 8),
-                         k3 = *(const float4*) (kp + 12);
-            auto decay_dot = [&](float4& mm, const float4& kk, float& d0, float& d1) __attribute__((always_inline)) {
-                mm.x *= e;
-                mm.y *= e;
-                mm.z *= e;
-                mm.w *= e;
-                d0 = __builtin_fmaf(mm.x, kk.x, d0);
-                d1 = __builtin_fmaf(mm.y, kk.y, d1);
-                d0 = __builtin_fmaf(mm.z, kk.z, d0);
-                d1 = __builtin_fmaf(mm.w, kk.w, d1);
-            };
-            float d0 = 0.0f, d1 = 0.0f;
-            decay_dot(m0, k0, d0, d1);
-            decay_dot(m1, k1, d0, d1);
-            decay_dot(m2, k2, d0, d1);
-            decay_dot(m3, k3, d0, d1);
-            const float delta = (s_v[tt][r] - red8(d0 + d1)) * s_b[tt];
-            auto upd_dot = [&](float4& mm, const float4& kk, const float4& qq, float& o0, float& o1)
-                __attribute__((always_inline)) {
-                mm.x = __builtin_fmaf(kk.x, delta, mm.x);
-                mm.y = __builtin_fmaf(kk.y, delta, mm.y);
-                mm.z = __builtin_fmaf(kk.z, delta, mm.z);
-                mm.w = __builtin_fmaf(kk.w, delta, mm.w);
-                o0 = __builtin_fmaf(mm.x, qq.x, o0);
-                o1 = __builtin_fmaf(mm.y, qq.y, o1);
-                o0 = __builtin_fmaf(mm.z, qq.z, o0);
-                o1 = __builtin_fmaf(mm.w, qq.w, o1);
-            };
-            float o0 = 0.0f, o1 = 0.0f;
-            upd_dot(m0, k0, q0, o0, o1);
-            upd_dot(m1, k1, q1, o0, o1);
-            upd_dot(m2, k2, q2, o0, o1);
-            upd_dot(m3, k3, q3, o0, o1);
-            const float o = red8(o0 + o1);
-            if (l == 0) a.o[((int64_t) (tb + tt) * a.H_v + hv) * GS + j] = o * scale;
+#pragma unroll 1
+        for (int tt = 0; tt < nt; tt += GC) {
+            fx4 k0[GC], k1[GC], q0[GC], q1[GC], s6[6];
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                k0[b] = *(const fx4*) &s_k[tt + b][4 * l];
+                k1[b] = *(const fx4*) &s_k[tt + b][64 + 4 * l];
+                q0[b] = *(const fx4*) &s_q[tt + b][4 * l];
+                q1[b] = *(const fx4*) &s_q[tt + b][64 + 4 * l];
+            }
+#pragma unroll
+            for (int i = 0; i < 6; ++i) s6[i] = *(const fx4*) &s_S[tt / GC][4 * i];
+            const fx4 v = *(const fx4*) &s_v[r][tt], bt = *(const fx4*) &s_b[tt];
+            auto S = [&](int i) __attribute__((always_inline)) { return s6[i >> 2][i & 3]; };
+            float xk[GC], xq[GC];
+#pragma unroll
+            for (int b = 0; b < GC; ++b) xk[b] = dot4(m0, k0[b], 0.0f) + dot4(m1, k1[b], 0.0f);
+#pragma unroll
+            for (int b = 0; b < GC; ++b) xq[b] = dot4(m0, q0[b], 0.0f) + dot4(m1, q1[b], 0.0f);
+            // the row's 16 lanes
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                xk[b] += dpp_f<DPP_XOR1>(xk[b]);
+                xq[b] += dpp_f<DPP_XOR1>(xq[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                xk[b] += dpp_f<DPP_XOR2>(xk[b]);
+                xq[b] += dpp_f<DPP_XOR2>(xq[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                xk[b] += dpp_f<DPP_HALF_MIRROR>(xk[b]);
+                xq[b] += dpp_f<DPP_HALF_MIRROR>(xq[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                xk[b] += dpp_f<DPP_MIRROR>(xk[b]);
+                xq[b] += dpp_f<DPP_MIRROR>(xq[b]);
+            }
+            float dl[GC], oo[GC];
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                float x = S(16 + b) * xk[b];
+#pragma unroll
+                for (int y = 0; y < b; ++y) x = __builtin_fmaf(dl[y], S(b * (b - 1) / 2 + y), x);
+                dl[b] = tt + b < nt ? (v[b] - x) * bt[b] : 0.0f;
+            }
+            m0 *= S(19);
+            m1 *= S(19);
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                const float f = S(20 + b) * dl[b];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    m0[i] = __builtin_fmaf(k0[b][i], f, m0[i]);
+                    m1[i] = __builtin_fmaf(k1[b][i], f, m1[i]);
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < GC; ++b) {
+                float s = S(16 + b) * xq[b];
+#pragma unroll
+                for (int y = 0; y <= b; ++y) s = __builtin_fmaf(dl[y], S(6 + b * (b + 1) / 2 + y), s);
+                oo[b] = s * scale;
+            }
+            // lane b of the row writes token tt + b
+            const float ov = l == 0 ? oo[0] : l == 1 ? oo[1] : l == 2 ? oo[2] : oo[3];
+            if (l < GC && tt + l < nt) a.o[((int64_t) (tb + tt + l) * a.H_v + hv) * GS + j] = ov;
         }
     }
-#undef GDN_LOAD
-    *(float4*) st = m0;
-    *(float4*) (st + 4) = m1;
-    *(float4*) (st + 8) = m2;
-    *(float4*) (st + 12) = m3;
-}
-
-// Grouping that gives every token its own bin (all bins the one matrix, through
-// the slot rows): the small projections (ssm_beta, ssm_alpha: H_v rows) then
-// spread over T workgroups of the GEMV instead of one.
-__global__ void k_gdn_group_tokens(int32_t* rows, int32_t* active, int32_t* active_off, int32_t* n_active,
-                                   int32_t* slot, int64_t T) {
-    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
-    if (i < T) {
-        rows[2 * i] = (int32_t) i;
-        rows[2 * i + 1] = (int32_t) i;
-        active[i] = (int32_t) i;
-        active_off[i] = (int32_t) i;
-        slot[i] = 0;
-    }
-    if (i == 0) {
-        active_off[T] = (int32_t) T;
-        *n_active = (int32_t) T;
-    }
+    *(fx4*) st = m0;
+    *(fx4*) (st + 64) = m1;
 }
 
 // Block (t, value head): rms_norm of the head's 128 outputs (double sum) times
@@ -278,6 +358,26 @@ __global__ void __launch_bounds__(GS) k_gdn_gate_norm(GdnArgs a) {
     a.y[e] = zn * v_silu(a.z[e]);
 }
 
+// The same, two heads (256 values) per wave and straight into Q8_K (and its f16
+// copy): the output projection's input.
+__global__ void __launch_bounds__(256) k_gdn_gate_norm_q8K(GdnArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int64_t nblk = (int64_t) a.T * a.H_v / 2, blk = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (blk >= nblk) return;
+    const int64_t e = blk * 256 + 4 * lane;
+    const float4 x = *(const float4*) (a.o + e), z = *(const float4*) (a.z + e);
+    const float4 nw = *(const float4*) (a.ssm_norm + 4 * (lane & 31));
+    double s = ((double) (x.x * x.x) + (double) (x.y * x.y)) + ((double) (x.z * x.z) + (double) (x.w * x.w));
+    for (int off = 16; off >= 1; off >>= 1) s += __shfl_xor(s, off);   // the head's 32 lanes
+    const float mean = (float) (s / (double) GS);
+    const float sc = 1.0f / sqrtf(mean + a.eps);
+    const float v[4] = {((x.x * sc) * nw.x) * v_silu(z.x), ((x.y * sc) * nw.y) * v_silu(z.y),
+                        ((x.z * sc) * nw.z) * v_silu(z.z), ((x.w * sc) * nw.w) * v_silu(z.w)};
+    _Float16* h = (_Float16*) a.y_h;
+    quant_q8K_wave(v, lane, (BlockQ8_K*) a.y_q8K + blk, h ? h + (size_t) blk * QK_K : nullptr,
+                   h ? h + (size_t) nblk * QK_K + (size_t) blk * 16 : nullptr);
+}
+
 }  // namespace
 
 bool gdn_shape_ok(int64_t S, int64_t H_k, int64_t H_v, int64_t d_conv) {
@@ -285,20 +385,26 @@ bool gdn_shape_ok(int64_t S, int64_t H_k, int64_t H_v, int64_t d_conv) {
 }
 
 int launch_gdn_core(const GdnArgs& a, hipStream_t stream) {
-    if (!gdn_shape_ok(GS, a.H_k, a.H_v, a.d_conv) || a.T <= 0) return -2;
-    hipLaunchKernelGGL(k_gdn_conv, dim3((unsigned) ((a.conv_ch + 255) / 256), (unsigned) a.T), dim3(256), 0, stream, a);
-    hipLaunchKernelGGL(k_gdn_conv_state, dim3((unsigned) ((a.conv_ch + 255) / 256)), dim3(256), 0, stream, a);
-    hipLaunchKernelGGL(k_gdn_prep, dim3((unsigned) a.T, (unsigned) (a.H_k + 1)), dim3(GS), 0, stream, a);
+    if (!gdn_shape_ok(GS, a.H_k, a.H_v, a.d_conv) || a.T <= 0 || (a.y_q8K && a.H_v % 2)) return -2;
+    const int64_t prep = (int64_t) a.T * (a.H_k + 1) + (a.conv_ch + GS - 1) / GS;
+    if (prep > INT32_MAX) return -2;
+    const dim3 gc((unsigned) ((a.conv_ch + 255) / 256), (unsigned) ((a.T + 4 * CT - 1) / (4 * CT)));
+    switch (a.d_conv) {
+        case 2: hipLaunchKernelGGL(k_gdn_conv<2>, gc, dim3(256), 0, stream, a); break;
+        case 3: hipLaunchKernelGGL(k_gdn_conv<3>, gc, dim3(256), 0, stream, a); break;
+        case 4: hipLaunchKernelGGL(k_gdn_conv<4>, gc, dim3(256), 0, stream, a); break;
+        case 5: hipLaunchKernelGGL(k_gdn_conv<5>, gc, dim3(256), 0, stream, a); break;
+        case 6: hipLaunchKernelGGL(k_gdn_conv<6>, gc, dim3(256), 0, stream, a); break;
+        case 7: hipLaunchKernelGGL(k_gdn_conv<7>, gc, dim3(256), 0, stream, a); break;
+        default: hipLaunchKernelGGL(k_gdn_conv<8>, gc, dim3(256), 0, stream, a); break;
+    }
+    hipLaunchKernelGGL(k_gdn_prep, dim3((unsigned) prep), dim3(GS), 0, stream, a);
     hipLaunchKernelGGL(k_gdn_delta, dim3((unsigned) a.H_v, (unsigned) (GS / GJB)), dim3(256), 0, stream, a);
-    hipLaunchKernelGGL(k_gdn_gate_norm, dim3((unsigned) a.T, (unsigned) a.H_v), dim3(GS), 0, stream, a);
-    return hipGetLastError() == hipSuccess ? 0 : -3;
-}
-
-int launch_gdn_group_tokens(int32_t* rows, int32_t* active, int32_t* active_off, int32_t* n_active, int32_t* slot,
-                            int64_t T, hipStream_t stream) {
-    if (T <= 0) return -2;
-    hipLaunchKernelGGL(k_gdn_group_tokens, dim3((unsigned) ((T + 255) / 256)), dim3(256), 0, stream, rows, active,
-                       active_off, n_active, slot, T);
+    if (a.y_q8K)
+        hipLaunchKernelGGL(k_gdn_gate_norm_q8K, dim3((unsigned) (((int64_t) a.T * a.H_v / 2 + 3) / 4)), dim3(256), 0,
+                           stream, a);
+    else
+        hipLaunchKernelGGL(k_gdn_gate_norm, dim3((unsigned) a.T, (unsigned) a.H_v), dim3(GS), 0, stream, a);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

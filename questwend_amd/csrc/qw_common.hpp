@@ -204,4 +204,35 @@ __device__ __forceinline__ void quant_q8K_wave(const float* v, int lane, BlockQ8
     }
 }
 
+// Activation Q8_0 (x86 AVX2 branch): one 32-value block per 8 lanes, 4 per lane.
+// With h set, each lane also writes its four quants as f16 and the block's d as
+// f32 in launch_q80_to_f16's layout.
+__device__ __forceinline__ void quant_q80_lane8(const float4 q, bool valid, int64_t blk, int sub, BlockQ8_0* dst,
+                                                _Float16* h, float* hd) {
+    float m = fmaxf(fmaxf(__builtin_fabsf(q.x), __builtin_fabsf(q.y)), fmaxf(__builtin_fabsf(q.z), __builtin_fabsf(q.w)));
+    m = fmaxf(m, __shfl_xor(m, 1));
+    m = fmaxf(m, __shfl_xor(m, 2));
+    m = fmaxf(m, __shfl_xor(m, 4));
+    if (!valid) return;
+    const float d = m / 127.f;
+    const float id = (m != 0.0f) ? 127.f / m : 0.0f;
+    BlockQ8_0* y = dst + blk;
+    const int q0 = (int) __builtin_rintf(q.x * id), q1 = (int) __builtin_rintf(q.y * id);
+    const int q2 = (int) __builtin_rintf(q.z * id), q3 = (int) __builtin_rintf(q.w * id);
+    const uint32_t packed = (uint32_t) (q0 & 0xff) | ((uint32_t) (q1 & 0xff) << 8) | ((uint32_t) (q2 & 0xff) << 16) |
+                            ((uint32_t) (q3 & 0xff) << 24);
+    // qs starts at byte 2 of the 34-byte block: write as two 16-bit halves
+    uint16_t* qs16 = (uint16_t*) ((char*) y + 2 + 4 * sub);
+    qs16[0] = (uint16_t) (packed & 0xffff);
+    qs16[1] = (uint16_t) (packed >> 16);
+    const uint16_t dh = f2h(d);
+    if (sub == 0) y->d = dh;
+    if (h) {
+        typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+        auto b = [&](int k) { return (_Float16) (float) (int8_t) (packed >> (8 * k)); };
+        *(h4v*) (h + 32 * (size_t) blk + 8 * (sub & 3) + 4 * (sub >> 2)) = h4v{b(0), b(1), b(2), b(3)};
+        if (sub == 0) hd[blk] = h2f(dh);
+    }
+}
+
 }  // namespace qw

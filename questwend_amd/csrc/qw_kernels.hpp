@@ -196,9 +196,19 @@ struct AttnArgs {
 };
 int launch_attn_core(const AttnArgs& a, hipStream_t stream);
 // attn_norm and its Q8_K quantisation in one launch (n % 256 == 0, x and w 16-byte aligned);
-// h_out (optional): the rows' f16 copy (launch_q8K_to_f16's layout)
+// h_out (optional): the rows' f16 copy (launch_q8K_to_f16's layout); dst0 (optional):
+// the Q8_0 of the same values.  g (optional): the one-bin grouping of the rows
+// (launch_group_dense's) and, with g->trows, bins of tpb consecutive rows of matrix 0
+// (slot rows all 0), written by the same launch.
+struct RowGroups {
+    int32_t *rows, *active, *active_off, *n_active;           // [2 T], [1], [2], [1]
+    int32_t *trows, *tactive, *toff, *tn, *tslot;             // [2 T], [T], [T + 1], [1], [T]
+    int tpb;
+};
 int launch_rms_norm_q8K(const float* x, int64_t n, int64_t rows, float eps, const float* w, void* dst,
-                        hipStream_t stream, uint16_t* h_out = nullptr);
+                        hipStream_t stream, uint16_t* h_out = nullptr, void* dst0 = nullptr,
+                        const RowGroups* g = nullptr);
+int launch_row_groups(const RowGroups& g, int64_t T, hipStream_t stream);
 // resid = x + y; out = rms_norm(resid) * w (rows of n, dense), out may be null
 int launch_add_rms_norm_mul(const float* x, const float* y, float* resid, float* out, int64_t n, int64_t rows,
                             float eps, const float* w, hipStream_t stream);
@@ -225,14 +235,11 @@ struct GdnArgs {
     float* kn;                    // [T][H_k][S] l2-normed k
     float* bg;                    // [T][H_v][2] beta, g
     float* o;                     // [T][H_v][S] the recurrence's outputs
-    float* y;                     // [T][H_v S] the gated norm's outputs
+    float* y;                     // [T][H_v S] the gated norm's outputs (without y_q8K)
+    void* y_q8K;                  // optional: Q8_K rows of y, written in its place (H_v even)
+    uint16_t* y_h;                // optional, with y_q8K: its f16 copy (launch_q8K_to_f16's layout)
 };
 // S = 128, H_v a multiple of H_k, 2 <= d_conv <= GDN_MAX_CONV
 bool gdn_shape_ok(int64_t S, int64_t H_k, int64_t H_v, int64_t d_conv);
 int launch_gdn_core(const GdnArgs& a, hipStream_t stream);
-// one bin per token (bin i = token i, slot rows all 0): rows[2 T], active[T],
-// active_off[T + 1], n_active[1], slot[T]
-int launch_gdn_group_tokens(int32_t* rows, int32_t* active, int32_t* active_off, int32_t* n_active, int32_t* slot,
-                            int64_t T, hipStream_t stream);
-
 }  // namespace qw
