@@ -172,11 +172,12 @@ int mfma_f16_prep_pair(Arena& ar, qw::MmidArgs& mu, qw::MmidArgs& mg, int64_t n_
 //  - Where every form gives ggml's bits (all but the block sums), a batch dense
 //    enough sends its light bins there too, in one launch in place of two: a
 //    16-row tile costs about what reading its weights does, the GEMV a pass per
-//    few rows.  The line is pairs per bin (128 experts, 8 per token, us per layer,
-//    light bins on the GEMV / everything on the matrix cores): Q4_K at the 30B
-//    shape 86.7 / 93.3 at T = 10, 119.5 / 113.4 at T = 16 (1 pair per bin),
-//    181.6 / 146.1 at T = 33, 312.5 / 267.4 at T = 512; Q8_0 123.9 / 125.1,
-//    161.9 / 156.4, 242.0 / 207.3, 466.7 / 418.7.  Q6_K forms more integers per tile:
+//    few rows.  The line is half a pair per bin (128 experts, 8 per token, us per
+//    layer, light bins on the GEMV / everything on the matrix cores): Q4_K at the 30B
+//    shape 43.9 / 35.4 at T = 8 (512 x 256 experts), 86.0 / 85.5 at T = 10 (55.4 / 50.6 with
+//    every token routed alike), 119.5 / 113.4 at T = 16, 181.6 / 146.1 at T = 33,
+//    312.5 / 267.4 at T = 512; Q8_0 124.2 / 124.9 at T = 10, 161.9 / 156.4, 242.0 / 207.3,
+//    466.7 / 418.7.  Q6_K forms more integers per tile: 109.6 / 125.8 at T = 10,
 //    142.0 / 157.6 at T = 16, 214.5 / 203.9 at T = 33, 230.7 / 205.3 at T = 64 (4 pairs
 //    per bin), but as the down projection at H = 4096 459.7 / 510.6 at T = 33,
 //    490.8 / 508.1 at T = 64, 539.5 / 551.2 at T = 128.
@@ -185,9 +186,9 @@ qw::MmidArgs mfma_bins(const qw::MmidArgs& m) {
     if (c.type == qw::T_Q8_0 && !c.act_h) c.mfma_min_rows = 0;
     if (c.mfma_min_rows <= 1) return c;
     const int64_t bins = c.slot_of ? c.n_slot_of : c.n_as;
-    const bool all = c.type == qw::T_Q8_0 ? c.n_pairs >= bins
+    const bool all = c.type == qw::T_Q8_0 ? 2 * c.n_pairs >= bins
                                           : c.mfma_exact && (c.type == qw::T_Q6_K ? c.act_h && c.n_pairs >= 4 * bins
-                                                                                  : c.act_h && c.n_pairs >= bins);
+                                                                                  : c.act_h && 2 * c.n_pairs >= bins);
     if (all) c.mfma_min_rows = 1;
     return c;
 }
@@ -1009,18 +1010,8 @@ int qwmoe_ffn_layer(void* stream, const qwmoe_layer* L, const float* x, int64_t 
     ra.xq = xq_fused ? xg : nullptr;
     // grouping by logical expert (slot rows are injective for resident layers)
     Grouping G{};
-    if (T <= qw::GROUP_WAVES && E <= 128) {
-        // small batch: logits (+ Q8_K of x), then top-k and grouping in one launch
-        qw::GroupArgs g;
-        if ((rc = group_args(ar, ids, k, T, (size_t) k * 4, E, nullptr, nullptr, nullptr, G, g))) return rc;
-        qw::RouterArgs rl = ra;
-        rl.ids = nullptr;
-        if ((rc = qw::launch_router(rl, logits, st))) return rc;
-        if ((rc = qw::launch_topk_group(ra, logits, g, st))) return rc;
-    } else {
-        if ((rc = qw::launch_router(ra, logits, st))) return rc;
-        if ((rc = group(st, ar, ids, k, T, (size_t) k * 4, E, nullptr, nullptr, nullptr, G))) return rc;
-    }
+    qw::GroupArgs g;
+    if ((rc = group_args(ar, ids, k, T, (size_t) k * 4, E, nullptr, nullptr, nullptr, G, g))) return rc;
     const size_t dnb1 = (size_t) F * 4, dnb2 = (size_t) F * 4 * (size_t) k;
     qw::MmidArgs mu = mmid_args(L->type_up, L->up, H, F, L->n_slots_up, L->up_nb1, L->up_nb2, xu, 1, qu, G.rows,
                                       G.active, G.active_off, G.n_active, G.max_active, L->slot_up,
@@ -1036,7 +1027,7 @@ int qwmoe_ffn_layer(void* stream, const qwmoe_layer* L, const float* x, int64_t 
     // (gate and up share it when they read one buffer)
     uint16_t* hx = nullptr;
     float* hxd = nullptr;
-    if (!xq_fused && xu == xg && mfma_f16_reserve(ar, mu, T)) {
+    if (xu == xg && mfma_f16_reserve(ar, mu, T)) {
         if (L->type_gate == L->type_up && qw::mmid_mfma_h_ok(mg, T)) {
             mg.act_h = mu.act_h;
             mg.act_hd = mu.act_hd;
@@ -1046,6 +1037,17 @@ int qwmoe_ffn_layer(void* stream, const qwmoe_layer* L, const float* x, int64_t 
             mu.act_h = nullptr;
             mu.act_hd = nullptr;
         }
+    }
+    ra.xh = xq_fused ? hx : nullptr;
+    if (T <= qw::GROUP_WAVES && E <= 128) {
+        // small batch: logits (+ Q8_K of x), then top-k and grouping in one launch
+        qw::RouterArgs rl = ra;
+        rl.ids = nullptr;
+        if ((rc = qw::launch_router(rl, logits, st))) return rc;
+        if ((rc = qw::launch_topk_group(ra, logits, g, st))) return rc;
+    } else {
+        if ((rc = qw::launch_router(ra, logits, st))) return rc;
+        if ((rc = qw::launch_group(g, st))) return rc;
     }
     if (!xq_fused &&
         (rc = qw::launch_quantize_act(vg, x, H, 1, T, (size_t) H * 4, (size_t) H * 4, xg, st, hx, hxd)))

@@ -202,23 +202,33 @@ __device__ __forceinline__ void group_body(const GroupArgs& g, int32_t* s_hist, 
     }
 }
 
-// The same grouping by one wave when there are at most 64 pairs and 128 bins:
-// lane p holds pair p; in-bin ranks from the ballots of chunk_rank; the bins'
-// counts (two bins per lane) are scanned across the wave for the offsets and the
-// active list.  cnt: 128 LDS words.
+// The same grouping by one wave when there are at most 128 pairs and 128 bins:
+// lane p holds pairs p and 64 + p; in-bin ranks from the ballots of chunk_rank, the
+// second chunk's behind the first one's counts; the bins' counts (two bins per lane)
+// are scanned across the wave for the offsets and the active list.  cnt: 128 LDS words.
 __device__ __forceinline__ void group_wave(const GroupArgs& g, int32_t* cnt) {
     const int lane = threadIdx.x & 63;
     const int P = (int) (g.T * g.n_ids);
     const int nb = (int) g.n_bins;
-    int t, e;
+    int t, e, t2 = 0, e2 = 0, key2 = -1;
     const int key = pair_key(g, lane, P, t, e, true);
     const int nbits = nb > 1 ? 32 - __clz(nb - 1) : 0;
     const ChunkRank r = chunk_rank(key, nbits);
+    int rank2 = 0;
     cnt[lane] = 0;
     cnt[lane + 64] = 0;
     wave_sync();
     if (key >= 0 && r.rank == 0) cnt[key] = r.cnt;
     wave_sync();
+    if (P > 64) {   // uniform
+        key2 = pair_key(g, 64 + lane, P, t2, e2, true);
+        const ChunkRank r2 = chunk_rank(key2, nbits);
+        const int before = key2 >= 0 ? cnt[key2] : 0;
+        rank2 = before + r2.rank;
+        wave_sync();
+        if (key2 >= 0 && r2.rank == 0) cnt[key2] = before + r2.cnt;
+        wave_sync();
+    }
     const int b0 = 2 * lane, b1 = 2 * lane + 1;
     const int c0 = b0 < nb ? cnt[b0] : 0, c1 = b1 < nb ? cnt[b1] : 0;
     int ic = c0 + c1, ia = (c0 > 0) + (c1 > 0);
@@ -264,6 +274,11 @@ __device__ __forceinline__ void group_wave(const GroupArgs& g, int32_t* cnt) {
         g.rows[2 * pos] = e;
         g.rows[2 * pos + 1] = t;
     }
+    if (key2 >= 0) {
+        const int pos = cnt[key2] + rank2;
+        g.rows[2 * pos] = e2;
+        g.rows[2 * pos + 1] = t2;
+    }
 }
 
 template <bool IN_LDS>
@@ -276,28 +291,26 @@ __global__ void __launch_bounds__(GROUP_WAVES * 64) k_group(GroupArgs g) {
 // Small batches (T <= GROUP_WAVES tokens, E <= 128): the router's softmax /
 // top-k / weights for token t on wave t (the k_router_topk steps, with wave
 // barriers), then the grouping of all tokens' ids by the whole workgroup, in one
-// launch.  Dynamic LDS: per wave p[E], order[E], gsum[E / 8], the sort stack and
-// a flag; then the GROUP_WAVES * E counters.
+// launch.  Dynamic LDS: per wave p[E], order[E] and the sort stack; then the
+// GROUP_WAVES * E counters.
 __global__ void __launch_bounds__(GROUP_WAVES * 64) k_topk_group(RouterArgs ra, const float* __restrict__ logits,
                                                                  GroupArgs g) {
     extern __shared__ uint32_t dyn[];
     __shared__ int32_t s_wsum[2][GROUP_WAVES];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int E = (int) ra.E;
-    const uint32_t per_wave = (uint32_t) (2 * E + E / 8 + 1) * 4u + (uint32_t) sizeof(SortRange) * SORT_STACK;
+    const uint32_t per_wave = (uint32_t) (2 * E) * 4u + (uint32_t) sizeof(SortRange) * SORT_STACK;
     uint8_t* mine = (uint8_t*) dyn + (size_t) w * ((per_wave + 15u) & ~15u);
     float* p = (float*) mine;
     int32_t* order = (int32_t*) (p + E);
-    float* gsum = (float*) (order + E);
-    int* need_sort = (int*) (gsum + E / 8);
-    SortRange* stack = (SortRange*) (need_sort + 1);
-    // up to 64 pairs: the ids go to LDS, the one-wave grouping reads them there
+    SortRange* stack = (SortRange*) (order + E);
+    // up to 128 pairs: the ids go to LDS, the one-wave grouping reads them there
     // while the next wave copies them out to the caller's buffer
-    __shared__ int32_t s_ids[64];
-    const bool small = ra.T * ra.k <= 64;
+    __shared__ int32_t s_ids[128];
+    const bool small = ra.T * ra.k <= 128;
     if (w < ra.T)
         topk_token<true>(logits, ra.E, ra.k, w, ra.clamp_min, ra.scale, small ? s_ids : ra.ids, ra.weights, ra.probs,
-                         ra.status, p, gsum, order, stack, need_sort, lane, ra.mask, ra.want);
+                         ra.status, p, order, stack, lane, ra.mask, ra.want);
     __syncthreads();   // every token's ids are written
     int32_t* hist = (int32_t*) ((uint8_t*) dyn + (size_t) GROUP_WAVES * ((per_wave + 15u) & ~15u));
     if (small) {
@@ -305,8 +318,8 @@ __global__ void __launch_bounds__(GROUP_WAVES * 64) k_topk_group(RouterArgs ra, 
             GroupArgs gl = g;
             gl.ids = s_ids;
             group_wave(gl, hist);
-        } else if (w == 1 && lane < ra.T * ra.k) {
-            ra.ids[lane] = s_ids[lane];
+        } else if (w <= 2 && 64 * (w - 1) + lane < ra.T * ra.k) {
+            ra.ids[64 * (w - 1) + lane] = s_ids[64 * (w - 1) + lane];
         }
     } else {
         group_body<true>(g, hist, s_wsum);
@@ -317,7 +330,7 @@ int launch_topk_group(const RouterArgs& ra, const float* logits, const GroupArgs
     if (ra.T < 1 || ra.T > GROUP_WAVES || ra.E % 8 || ra.E > 128 || ra.k < 1 || ra.k > ra.E || !ra.ids || !ra.weights)
         return -2;
     if (g.n_bins != ra.E || g.ids != ra.ids || g.n_ids != ra.k || g.T != ra.T || g.ids_stride != ra.k) return -2;
-    const uint32_t per_wave = (uint32_t) (2 * ra.E + ra.E / 8 + 1) * 4u + (uint32_t) sizeof(SortRange) * SORT_STACK;
+    const uint32_t per_wave = (uint32_t) (2 * ra.E) * 4u + (uint32_t) sizeof(SortRange) * SORT_STACK;
     const size_t lds = (size_t) GROUP_WAVES * ((per_wave + 15u) & ~15u) + (size_t) GROUP_WAVES * ra.E * 4;
     hipLaunchKernelGGL(k_topk_group, dim3(1), dim3(GROUP_WAVES * 64), lds, stream, ra, logits, g);
     return hipGetLastError() == hipSuccess ? 0 : -3;

@@ -26,13 +26,16 @@ namespace qw {
 template <int ROUTER_TT, int EPW, int ROUTER_STEPS>
 __global__ void __launch_bounds__(32 * EPW) k_router_logits(const float* __restrict__ W, const float* __restrict__ x,
                                                             int64_t x_stride, int64_t H, int64_t E, int64_t T,
-                                                            float* __restrict__ logits, BlockQ8_K* __restrict__ xq) {
+                                                            float* __restrict__ logits, BlockQ8_K* __restrict__ xq,
+                                                            _Float16* __restrict__ xh) {
     if (EPW == 2 && blockIdx.x >= (E + 1) / 2) {
         const int64_t ib = blockIdx.x - (E + 1) / 2, t = blockIdx.y;
         if (ib >= H / QK_K) return;
         const float4 q = *(const float4*) (x + t * x_stride + ib * QK_K + 4 * threadIdx.x);
         const float v[4] = {q.x, q.y, q.z, q.w};
-        quant_q8K_wave(v, threadIdx.x, xq + t * (H / QK_K) + ib);
+        const int64_t blk = t * (H / QK_K) + ib;
+        quant_q8K_wave(v, threadIdx.x, xq + blk, xh ? xh + (size_t) blk * QK_K : nullptr,
+                       xh ? xh + (size_t) (T * H) + (size_t) blk * 16 : nullptr);
         return;
     }
     const int c = threadIdx.x & 31;
@@ -304,12 +307,10 @@ __global__ void __launch_bounds__(64) k_router_topk(const float* __restrict__ lo
                                                     int32_t* __restrict__ status, const float* __restrict__ mask,
                                                     int32_t* __restrict__ want) {
     __shared__ __align__(16) float p[64 * ROUTER_EPL];
-    __shared__ float gsum[64 * ROUTER_EPL / 8];
     __shared__ int32_t order[64 * ROUTER_EPL];
     __shared__ SortRange sort_stack[SORT_STACK];
-    __shared__ int need_sort;
-    topk_token<false>(logits, E, k, blockIdx.x, clamp_min, scale, ids, weights, probs_out, status, p, gsum, order,
-                      sort_stack, &need_sort, threadIdx.x, mask, want);
+    topk_token<false>(logits, E, k, blockIdx.x, clamp_min, scale, ids, weights, probs_out, status, p, order, sort_stack,
+                      threadIdx.x, mask, want);
 }
 
 int launch_router(const RouterArgs& a, float* logits_ws, hipStream_t stream) {
@@ -321,7 +322,7 @@ int launch_router(const RouterArgs& a, float* logits_ws, hipStream_t stream) {
         const int64_t nq = a.xq ? a.H / QK_K : 0;
         dim3 g1((unsigned) ((a.E + 1) / 2 + nq), (unsigned) a.T);
         hipLaunchKernelGGL((k_router_logits<1, 2, 32>), g1, dim3(64), 0, stream, a.W, a.x, a.x_stride, a.H, a.E, a.T,
-                           logits, (BlockQ8_K*) a.xq);
+                           logits, (BlockQ8_K*) a.xq, (_Float16*) a.xh);
     } else if (a.H % (2 * RL_CH) == 0 && a.E % 16 == 0 && a.x_stride % 4 == 0 && ((uintptr_t) a.x & 15) == 0 &&
                ((uintptr_t) a.W & 15) == 0) {
         dim3 g1((unsigned) (a.E / 16), (unsigned) ((a.T + 15) / 16));
