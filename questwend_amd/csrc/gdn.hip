@@ -146,13 +146,12 @@ __global__ void __launch_bounds__(GS) k_gdn_prep(GdnArgs a) {
 // E_{a,b} (k_a . q_b) are the same for every row: formed once per workgroup and block
 // of GTB tokens, in LDS.  All in fp32 (the reference's sums in another order).
 //
-// Tokens go in blocks of GTB: q, k (the key head), v (the workgroup's rows), beta and
-// g sit in LDS, the next block's are loaded into registers while the current block
-// is applied.  Tokens past T have k = 0, e = 1 and delta = 0: they change nothing.
-// H_v = 32, T = 300: 101 us (8 lanes per row, token by token) -> 74 us (what is left: LDS reads, 24 of 16 bytes per
-// lane and step with one workgroup per CU; reading a step ahead changed nothing).
+// Up to GTB tokens: q, k (the key head), v (the workgroup's rows), beta and g sit in LDS.
+// Tokens past T have k = 0, e = 1 and delta = 0: they change nothing.  About 1 us per step
+// (LDS reads, 24 of 16 bytes per lane and step with one workgroup per CU); token by token
+// 1.35 us per four.
 typedef float fx4 __attribute__((ext_vector_type(4)));   // (arrays of it stay in registers)
-constexpr int GTB = 32;   // tokens per staged block
+constexpr int GTB = 32;   // tokens staged
 constexpr int GC = 4;     // tokens per step
 __global__ void __launch_bounds__(256) k_gdn_delta(GdnArgs a) {
     const int hv = blockIdx.x, tid = threadIdx.x, r = tid >> 4, l = tid & 15;
@@ -167,47 +166,34 @@ __global__ void __launch_bounds__(256) k_gdn_delta(GdnArgs a) {
     fx4 m0 = *(const fx4*) st, m1 = *(const fx4*) (st + 64);
     const float scale = 1.0f / sqrtf((float) GS);
     const int64_t vbase = 2 * (int64_t) a.H_k * GS + (int64_t) hv * GS + j0;
-    fx4 rq[4], rk[4];
-    float rv[2], rbg = 0.0f;
-    const int64_t qcol = 4 * (tid % (GS / 4));
-    auto load = [&](int tb) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t t = min(tb + tid / (GS / 4) + 8 * u, a.T - 1);
-            rq[u] = *(const fx4*) (a.qn + (t * a.H_k + hk) * GS + qcol);
-            rk[u] = *(const fx4*) (a.kn + (t * a.H_k + hk) * GS + qcol);
-            if (tb + tid / (GS / 4) + 8 * u >= a.T) rk[u] = fx4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-            rv[u] = a.conv[(int64_t) min(tb + tid / GJB + 16 * u, a.T - 1) * a.conv_ch + vbase + tid % GJB];
-        if (tid < 2 * GTB) {
-            const int t = tb + (tid >> 1);
-            rbg = t < a.T ? a.bg[((int64_t) t * a.H_v + hv) * 2 + (tid & 1)] : 0.0f;
-        }
-    };
     auto dot4 = [](fx4 x, fx4 y, float s) __attribute__((always_inline)) {
         s = __builtin_fmaf(x.x, y.x, s);
         s = __builtin_fmaf(x.y, y.y, s);
         s = __builtin_fmaf(x.z, y.z, s);
         return __builtin_fmaf(x.w, y.w, s);
     };
-    load(0);
-    for (int tb = 0; tb < a.T; tb += GTB) {
-        __syncthreads();   // the previous block is consumed
+    {
+        const int qcol = 4 * (tid % (GS / 4));
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            *(fx4*) &s_q[tid / (GS / 4) + 8 * u][qcol] = rq[u];
-            *(fx4*) &s_k[tid / (GS / 4) + 8 * u][qcol] = rk[u];
+            const int tt = tid / (GS / 4) + 8 * u;
+            const int64_t row = ((int64_t) min(tt, a.T - 1) * a.H_k + hk) * GS + qcol;
+            *(fx4*) &s_q[tt][qcol] = *(const fx4*) (a.qn + row);
+            const fx4 k = *(const fx4*) (a.kn + row);
+            *(fx4*) &s_k[tt][qcol] = tt < a.T ? k : fx4{0.0f, 0.0f, 0.0f, 0.0f};
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) s_v[tid % GJB][tid / GJB + 16 * u] = rv[u];
+        for (int u = 0; u < 2; ++u) {
+            const int tt = tid / GJB + 16 * u;
+            s_v[tid % GJB][tt] = a.conv[(int64_t) min(tt, a.T - 1) * a.conv_ch + vbase + tid % GJB];
+        }
         if (tid < 2 * GTB) {
-            if (tid & 1) s_e[tid >> 1] = expf(rbg);
-            else s_b[tid >> 1] = rbg;
+            const int t = tid >> 1;
+            const float bg = t < a.T ? a.bg[((int64_t) t * a.H_v + hv) * 2 + (tid & 1)] : 0.0f;
+            if (tid & 1) s_e[t] = expf(bg);
+            else s_b[t] = bg;
         }
         __syncthreads();
-        if (tb + GTB < a.T) load(tb + GTB);
         {   // P and Q: 8 lanes per token b of a step, lane p its columns 4 p + 32 i .. + 3
             const int grp = tid >> 3, p = tid & 7, c = grp >> 2, b = grp & 3, t0 = GC * c;
             float dk[GC], dq[GC];
@@ -261,7 +247,7 @@ __global__ void __launch_bounds__(256) k_gdn_delta(GdnArgs a) {
             }
         }
         __syncthreads();
-        const int nt = a.T - tb < GTB ? a.T - tb : GTB;
+        const int nt = a.T;
 #pragma unroll 1
         for (int tt = 0; tt < nt; tt += GC) {
             fx4 k0[GC], k1[GC], q0[GC], q1[GC], s6[6];
@@ -330,11 +316,292 @@ __global__ void __launch_bounds__(256) k_gdn_delta(GdnArgs a) {
             }
             // lane b of the row writes token tt + b
             const float ov = l == 0 ? oo[0] : l == 1 ? oo[1] : l == 2 ? oo[2] : oo[3];
-            if (l < GC && tt + l < nt) a.o[((int64_t) (tb + tt + l) * a.H_v + hv) * GS + j] = ov;
+            if (l < GC && tt + l < nt) a.o[((int64_t) (tt + l) * a.H_v + hv) * GS + j] = ov;
         }
     }
     *(fx4*) st = m0;
     *(fx4*) (st + 64) = m1;
+}
+
+// ---- batches of GCHUNK_MIN tokens and more: sixteen tokens per step, on the matrix cores ----
+//
+// With D the deltas of a chunk's 16 tokens (a row per token), V, K, Q its rows, M the
+// state before it and E_b, E_{a,b} as above, the four-token form's equations read
+//     (I + A) D = R = beta (V - E K M^T),     A[b][a] = beta_b E_{a,b} (k_a . k_b), a < b
+//     O sqrt(S) = E Q M^T + P D,              P[b][a] = E_{a,b} (k_a . q_b),        a <= b
+//     M^T after = E_16 M^T + K^T (E_{a,16} D)
+// A and P hold nothing of the state: k_gdn_chunk forms P and T = (I + A)^-1 (16 x 16,
+// forward substitution) for every chunk and head at once, and the serial kernel is left
+// with five small fp32 matrix products per chunk.
+// From 32 tokens on (us per call, H_v = 32, four tokens a step / chunks): 86.7 / 87.3 at T = 16,
+// 88.1 / 88.9 at 24, 91.1 / 89.9 at 32, 97.6 / 93.2 at 48, 105.8 / 100.4 at 64, 220 / 181 at 300,
+// 546 / 417 at 1000.
+constexpr int GCHUNK_MIN = 32;
+constexpr int GCK = 16;              // tokens per chunk
+constexpr int GCK_P = 256, GCK_E = 512, GCK_E2 = 528, GCK_B = 544;   // record: T, P / sqrt(S), E_b, E_{a,16}, beta
+constexpr int GCK_REC = 576;         // floats per record (chunk, value head), in the y rows, written only later
+static_assert(GCHUNK_MIN - 1 <= GTB, "the four-token form stages one block of tokens");
+static_assert(GCHUNK_MIN >= GCK && 2 * GCK_REC <= (GCK + 1) * GS, "the records of ceil(T / 16) chunks fit T rows of y");
+
+__device__ __forceinline__ fx4 mfma_f32(float x, float y, fx4 c) {   // D[16][16] += A[16][4] B[4][16]
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
+}
+
+// Block c H_k + hk: k_gdn_prep's norms for chunk c of key head hk, and the records of the
+// value heads that read it; the blocks past the chunks' the conv state.
+__global__ void __launch_bounds__(256) k_gdn_chunk(GdnArgs a) {
+    const int n_ch = (a.T + GCK - 1) / GCK, c = blockIdx.x / a.H_k, hk = blockIdx.x % a.H_k, tid = threadIdx.x;
+    if (c >= n_ch) {
+        gdn_conv_state(a, (int64_t) ((int) blockIdx.x - n_ch * a.H_k) * 256 + tid);
+        return;
+    }
+    constexpr int HS = 16;   // value heads at a time
+    __shared__ __align__(16) float s_q[GCK][GS + 4], s_k[GCK][GS + 4];
+    __shared__ float s_p[2][4][256];
+    __shared__ __align__(16) float s_e[HS][GCK], s_b[HS][GCK];
+    __shared__ __align__(16) float s_A[HS][GCK * GCK + 4];
+    const int t0 = c * GCK, w = tid >> 6, lane = tid & 63;
+    const int64_t key_dim = (int64_t) a.H_k * GS;
+    {   // 32 lanes per token, two rounds
+        const int col = 4 * (lane & 31);
+        fx4 q[2], k[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const float* row = a.conv + (int64_t) min(t0 + 4 * w + 2 * u + (lane >> 5), a.T - 1) * a.conv_ch + hk * GS + col;
+            q[u] = *(const fx4*) row;
+            k[u] = *(const fx4*) (row + key_dim);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int b = 4 * w + 2 * u + (lane >> 5);
+            double sq = 0.0, sk = 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sq += (double) (q[u][i] * q[u][i]);
+                sk += (double) (k[u][i] * k[u][i]);
+            }
+            for (int off = 16; off >= 1; off >>= 1) {
+                sq += __shfl_xor(sq, off);
+                sk += __shfl_xor(sk, off);
+            }
+            const float scq = 1.0f / fmaxf(sqrtf((float) sq), a.eps), sck = 1.0f / fmaxf(sqrtf((float) sk), a.eps);
+            const fx4 qn = q[u] * scq, kn = k[u] * sck;
+            *(fx4*) &s_q[b][col] = qn;
+            *(fx4*) &s_k[b][col] = kn;
+            if (t0 + b < a.T) {
+                *(fx4*) (a.qn + ((int64_t) (t0 + b) * a.H_k + hk) * GS + col) = qn;
+                *(fx4*) (a.kn + ((int64_t) (t0 + b) * a.H_k + hk) * GS + col) = kn;
+            }
+        }
+    }
+    __syncthreads();
+    {   // k_b . k_a and q_b . k_a over the wave's 32 columns; the contraction takes them in any order
+        const int n = lane & 15, g = lane >> 4;
+        fx4 gk = fx4{0.0f, 0.0f, 0.0f, 0.0f}, gq = gk;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const fx4 kf = *(const fx4*) &s_k[n][32 * w + 16 * u + 4 * g], qf = *(const fx4*) &s_q[n][32 * w + 16 * u + 4 * g];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                gk = mfma_f32(kf[r], kf[r], gk);
+                gq = mfma_f32(qf[r], kf[r], gq);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s_p[0][w][(4 * g + r) * GCK + n] = gk[r];
+            s_p[1][w][(4 * g + r) * GCK + n] = gq[r];
+        }
+    }
+    __syncthreads();
+    const int hi = tid >> 4, lo = tid & 15;
+    const float gk = (s_p[0][0][tid] + s_p[0][1][tid]) + (s_p[0][2][tid] + s_p[0][3][tid]);
+    const float gq = (s_p[1][0][tid] + s_p[1][1][tid]) + (s_p[1][2][tid] + s_p[1][3][tid]);
+    const float scale = 1.0f / sqrtf((float) GS);
+    const int rep = a.H_v / a.H_k;
+    for (int m0 = 0; m0 < rep; m0 += HS) {
+        const int nm = rep - m0 < HS ? rep - m0 : HS;
+        if (hi < nm) {   // head m0 + hi, token lo
+            const int hv = hk + (m0 + hi) * a.H_k, t = t0 + lo;
+            float e = 1.0f, be = 0.0f;
+            if (t < a.T) {
+                const float al = a.araw[(int64_t) t * a.H_v + hv] + a.dt_bias[hv];
+                const float sp = al > 20.0f ? al : logf(1.0f + expf(al));
+                e = expf(sp * a.ssm_a[hv]);
+                be = 1.0f / (1.0f + expf(-a.braw[(int64_t) t * a.H_v + hv]));
+            }
+            s_e[hi][lo] = e;
+            s_b[hi][lo] = be;
+        }
+        __syncthreads();
+        for (int m = 0; m < nm; ++m) {   // token hi against token lo
+            float* rec = a.y + ((int64_t) c * a.H_v + hk + (m0 + m) * a.H_k) * GCK_REC;
+            float ev[GCK], E = 1.0f;
+#pragma unroll
+            for (int y = 0; y < GCK; y += 4) *(fx4*) &ev[y] = *(const fx4*) &s_e[m][y];
+#pragma unroll
+            for (int y = 1; y < GCK; ++y) E = y > lo && y <= hi ? E * ev[y] : E;
+            const float be = s_b[m][hi];
+            s_A[m][tid] = lo < hi && t0 + hi < a.T ? (be * E) * gk : 0.0f;
+            rec[GCK_P + tid] = lo <= hi ? (E * gq) * scale : 0.0f;
+            if (lo == 0) {
+                rec[GCK_E + hi] = ev[0] * E;
+                rec[GCK_B + hi] = be;
+            }
+            if (hi == GCK - 1) rec[GCK_E2 + lo] = E;
+        }
+        __syncthreads();
+        if (hi < nm) {   // head m0 + hi, column lo of T
+            float* rec = a.y + ((int64_t) c * a.H_v + hk + (m0 + hi) * a.H_k) * GCK_REC;
+            float tc[GCK];
+#pragma unroll
+            for (int b = 0; b < GCK; ++b) {
+                float s = b == lo ? 1.0f : 0.0f;
+#pragma unroll
+                for (int y = 0; y < b; ++y) s = __builtin_fmaf(-s_A[hi][b * GCK + y], tc[y], s);
+                tc[b] = lo > b ? 0.0f : s;
+                rec[b * GCK + lo] = tc[b];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// C[b][j] += sum_{a <= b} L[b][a] x[a][j] for values that are not all finite: the product over
+// whole rows would carry a token's infinity or NaN to the tokens before it as 0 * inf.
+__device__ __forceinline__ fx4 gdn_tri(const float* __restrict__ L, fx4 x, fx4 acc) {
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+#pragma unroll 1
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const float xa = __shfl(x[y], h * 16 + n);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (4 * h + y <= 4 * g + r) acc[r] = __builtin_fmaf(L[(4 * g + r) * GCK + 4 * h + y], xa, acc[r]);
+        }
+    return acc;
+}
+
+// Workgroup (value head hv, rows j0 .. j0 + 15 of M), wave w its columns 32 w .. + 31 as two
+// accumulator tiles of M^T: lane (g, n) = (lane / 16, lane % 16) holds M[j0 + n][i0 + 4 g + r]
+// in register r.  Register r is at once the operand B of a product that contracts the
+// columns 4 g + r of step r, so the state never changes its layout; nor do X = K M^T, R
+// and D, which come out as [token 4 g + r][row n] and are contracted over the tokens the
+// same way.  K M^T and Q M^T are summed over the four waves through LDS (one barrier per
+// chunk); R and D are formed by every wave, O by one of them in turn.  Operands are
+// loaded two chunks ahead.  H_v = 32, T = 300, with k_gdn_chunk (7.4) in place of k_gdn_prep
+// (6.0): 74 us four tokens a step, 39 loading one chunk ahead, 32 now: 1.3 us a chunk, the
+// chain of products, exchange and elementwise steps with one wave per SIMD (26 us without
+// any load).  Buffer loads with scalar bases, O split over all waves and loads placed
+// between the products: 33 each.
+__global__ void __launch_bounds__(256) k_gdn_delta_chunk(GdnArgs a) {
+    const int hv = blockIdx.x, j0 = blockIdx.y * 16, hk = hv % a.H_k;
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
+    const int n_ch = (a.T + GCK - 1) / GCK;
+    __shared__ fx4 s_x[2][2][4][64];
+    float* st = a.state + ((int64_t) hv * GS + j0 + n) * GS + 32 * w + 4 * g;
+    fx4 m[2] = {*(const fx4*) st, *(const fx4*) (st + 16)};
+    const float scale = 1.0f / sqrtf((float) GS);
+    const int64_t vcol = 2 * (int64_t) a.H_k * GS + (int64_t) hv * GS + j0 + n;
+    struct Chunk {
+        fx4 kf[2], qf[2], kt[2], v, T, P, E, E2, b;
+        float e;
+    };
+    auto load = [&](int c) __attribute__((always_inline)) {
+        Chunk x;
+        const int t0 = c * GCK, last = a.T - 1;
+        const int64_t row = ((int64_t) min(t0 + n, last) * a.H_k + hk) * GS + 32 * w + 4 * g;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            x.kf[u] = *(const fx4*) (a.kn + row + 16 * u);
+            x.qf[u] = *(const fx4*) (a.qn + row + 16 * u);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t t = min(t0 + 4 * g + r, last);
+            x.v[r] = a.conv[t * a.conv_ch + vcol];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) x.kt[u][r] = a.kn[(t * a.H_k + hk) * GS + 32 * w + 16 * u + n];
+        }
+        const float* rec = a.y + ((int64_t) c * a.H_v + hv) * GCK_REC;
+        x.T = *(const fx4*) (rec + n * GCK + 4 * g);
+        x.P = *(const fx4*) (rec + GCK_P + n * GCK + 4 * g);
+        x.E = *(const fx4*) (rec + GCK_E + 4 * g);
+        x.E2 = *(const fx4*) (rec + GCK_E2 + 4 * g);
+        x.b = *(const fx4*) (rec + GCK_B + 4 * g);
+        x.e = rec[GCK_E + GCK - 1];
+        return x;
+    };
+    auto finite = [](fx4 x) __attribute__((always_inline)) {
+        bool f = true;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f = f && __builtin_fabsf(x[r]) < INFINITY;
+        return (bool) __all(f);
+    };
+    const fx4 zero = fx4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto step = [&](int c, const Chunk& x) __attribute__((always_inline)) {
+        const float* rec = a.y + ((int64_t) c * a.H_v + hv) * GCK_REC;
+        fx4 X[2] = {zero, zero}, Y[2] = {zero, zero};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                X[u] = mfma_f32(x.kf[u][r], m[u][r], X[u]);
+                Y[u] = mfma_f32(x.qf[u][r], m[u][r], Y[u]);
+            }
+        s_x[c & 1][0][w][lane] = X[0] + X[1];
+        s_x[c & 1][1][w][lane] = Y[0] + Y[1];
+        __syncthreads();   // (a wave that writes these words again has passed the next barrier)
+        const fx4(*sx)[64] = s_x[c & 1][0];
+        const fx4 Xs = (sx[0][lane] + sx[1][lane]) + (sx[2][lane] + sx[3][lane]);
+        fx4 R, D = zero;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            R[r] = c * GCK + 4 * g + r < a.T ? (x.v[r] - x.E[r] * Xs[r]) * x.b[r] : 0.0f;
+        if (finite(R)) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) D = mfma_f32(x.T[r], R[r], D);
+        } else {
+            D = gdn_tri(rec, R, D);
+        }
+        const fx4 De = D * x.E2;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) m[u] *= x.e;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) m[u] = mfma_f32(x.kt[u][r], De[r], m[u]);
+        if ((c & 3) == w) {
+            const fx4(*sy)[64] = s_x[c & 1][1];
+            fx4 O = ((sy[0][lane] + sy[1][lane]) + (sy[2][lane] + sy[3][lane])) * x.E * scale;
+            if (finite(D)) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) O = mfma_f32(x.P[r], D[r], O);
+            } else {
+                O = gdn_tri(rec + GCK_P, D, O);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = c * GCK + 4 * g + r;
+                if (t < a.T) a.o[((int64_t) t * a.H_v + hv) * GS + j0 + n] = O[r];
+            }
+        }
+    };
+    Chunk x0 = load(0), x1 = load(min(1, n_ch - 1)), x2;
+#pragma unroll 1
+    for (int c = 0; c < n_ch; c += 3) {
+        x2 = load(min(c + 2, n_ch - 1));
+        step(c, x0);
+        if (c + 1 >= n_ch) break;
+        x0 = load(min(c + 3, n_ch - 1));
+        step(c + 1, x1);
+        if (c + 2 >= n_ch) break;
+        x1 = load(min(c + 4, n_ch - 1));
+        step(c + 2, x2);
+    }
+    *(fx4*) st = m[0];
+    *(fx4*) (st + 16) = m[1];
 }
 
 // Block (t, value head): rms_norm of the head's 128 outputs (double sum) times
@@ -398,8 +665,14 @@ int launch_gdn_core(const GdnArgs& a, hipStream_t stream) {
         case 7: hipLaunchKernelGGL(k_gdn_conv<7>, gc, dim3(256), 0, stream, a); break;
         default: hipLaunchKernelGGL(k_gdn_conv<8>, gc, dim3(256), 0, stream, a); break;
     }
-    hipLaunchKernelGGL(k_gdn_prep, dim3((unsigned) prep), dim3(GS), 0, stream, a);
-    hipLaunchKernelGGL(k_gdn_delta, dim3((unsigned) a.H_v, (unsigned) (GS / GJB)), dim3(256), 0, stream, a);
+    if (a.T >= GCHUNK_MIN) {
+        const int64_t chunks = (int64_t) ((a.T + GCK - 1) / GCK) * a.H_k + (a.conv_ch + 255) / 256;
+        hipLaunchKernelGGL(k_gdn_chunk, dim3((unsigned) chunks), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL(k_gdn_delta_chunk, dim3((unsigned) a.H_v, (unsigned) (GS / 16)), dim3(256), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL(k_gdn_prep, dim3((unsigned) prep), dim3(GS), 0, stream, a);
+        hipLaunchKernelGGL(k_gdn_delta, dim3((unsigned) a.H_v, (unsigned) (GS / GJB)), dim3(256), 0, stream, a);
+    }
     if (a.y_q8K)
         hipLaunchKernelGGL(k_gdn_gate_norm_q8K, dim3((unsigned) (((int64_t) a.T * a.H_v / 2 + 3) / 4)), dim3(256), 0,
                            stream, a);

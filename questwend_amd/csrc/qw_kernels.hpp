@@ -236,7 +236,7 @@ struct GdnArgs {
     float* kn;                    // [T][H_k][S] l2-normed k
     float* bg;                    // [T][H_v][2] beta, g
     float* o;                     // [T][H_v][S] the recurrence's outputs
-    float* y;                     // [T][H_v S] the gated norm's outputs (without y_q8K)
+    float* y;                     // [T][H_v S] the gated norm's outputs (without y_q8K); before them the chunks' records
     void* y_q8K;                  // optional: Q8_K rows of y, written in its place (H_v even)
     uint16_t* y_h;                // optional, with y_q8K: its f16 copy (launch_q8K_to_f16's layout)
 };
