@@ -32,9 +32,12 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 // Head rows of one token: Q and K heads get ggml_rms_norm (sum of squares in
 // double) * norm weight and NEOX RoPE; K and V heads go to the caches at row
 // n_past + t.  A wave per head row, lane i holds elements i and i + 64: NEOX's
-// pair.  Block (t, y) takes head rows y * HPB ..; its cosines and sines (the same
-// for every head) are formed once, in LDS.  T = 512, 40 head rows: 14.3 us with
-// one row per block -> 13.2 us.
+// pair.  Block (t, y) takes head rows y * hpb ..; its cosines and sines (the same
+// for every head) are formed once, in LDS.  A wave takes RB rows at a time, whose
+// loads and double sums overlap: a row alone is a load and six dependent shuffles of
+// a double.  T = 512, 40 head rows: 13.2 us a row at a time, a block per
+// token -> 8.8, five rows at a time, two blocks.  Few tokens take a row per wave.
+template <int RB>
 __global__ void __launch_bounds__(256) k_attn_qk_rope(AttnArgs a, int hpb) {
     __shared__ float s_c[AD / 2], s_s[AD / 2];
     const int t = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -49,29 +52,44 @@ __global__ void __launch_bounds__(256) k_attn_qk_rope(AttnArgs a, int hpb) {
         s_s[lane] = sinf(th);
     }
     __syncthreads();
-    for (int r = r0 + w; r < r1; r += 4) {
-        if (r >= nq + nk) {
-            const int g = r - nq - nk;
-            const float* src = a.v + (int64_t) t * gqa + g * AD;
-            __half* dst = (__half*) a.vc + pos * gqa + g * AD;
-            dst[lane] = __float2half_rn(src[lane]);
-            dst[lane + 64] = __float2half_rn(src[lane + 64]);
-            continue;
+    const float wq0 = a.q_norm[lane], wq1 = a.q_norm[lane + 64], wk0 = a.k_norm[lane], wk1 = a.k_norm[lane + 64];
+    for (int rb = r0 + w; rb < r1; rb += 4 * RB) {
+        float x0[RB], x1[RB];
+        double s[RB];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const int r = min(rb + 4 * i, r1 - 1);
+            const float* src = r < nq        ? a.q + ((int64_t) t * nq + r) * AD
+                               : r < nq + nk ? a.k + (int64_t) t * gqa + (r - nq) * AD
+                                             : a.v + (int64_t) t * gqa + (r - nq - nk) * AD;
+            x0[i] = src[lane];
+            x1[i] = src[lane + 64];
         }
-        const bool is_q = r < nq;
-        const float* src = is_q ? a.q + ((int64_t) t * nq + r) * AD : a.k + (int64_t) t * gqa + (r - nq) * AD;
-        const float* wn = is_q ? a.q_norm : a.k_norm;
-        const float x0 = src[lane], x1 = src[lane + 64];
-        double s = (double) (x0 * x0) + (double) (x1 * x1);
-        for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
-        const float mean = (float) (s / (double) AD);
-        const float scale = 1.0f / sqrtf(mean + a.eps);
-        const float y0 = (x0 * scale) * wn[lane], y1 = (x1 * scale) * wn[lane + 64];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) s[i] = (double) (x0[i] * x0[i]) + (double) (x1[i] * x1[i]);
+        for (int off = 32; off >= 1; off >>= 1) {
+#pragma unroll
+            for (int i = 0; i < RB; ++i) s[i] += __shfl_xor(s[i], off);
+        }
         const float c = s_c[lane], sn = s_s[lane];
-        const float o0 = y0 * c - y1 * sn, o1 = y0 * sn + y1 * c;
-        __half* dst = is_q ? (__half*) a.qr + ((int64_t) t * nq + r) * AD : (__half*) a.kc + pos * gqa + (r - nq) * AD;
-        dst[lane] = __float2half_rn(o0);
-        dst[lane + 64] = __float2half_rn(o1);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const int r = rb + 4 * i;
+            if (r >= r1) break;
+            float o0 = x0[i], o1 = x1[i];
+            if (r < nq + nk) {
+                const float mean = (float) (s[i] / (double) AD);
+                const float scale = 1.0f / sqrtf(mean + a.eps);
+                const float y0 = (o0 * scale) * (r < nq ? wq0 : wk0), y1 = (o1 * scale) * (r < nq ? wq1 : wk1);
+                o0 = y0 * c - y1 * sn;
+                o1 = y0 * sn + y1 * c;
+            }
+            __half* dst = r < nq        ? (__half*) a.qr + ((int64_t) t * nq + r) * AD
+                          : r < nq + nk ? (__half*) a.kc + pos * gqa + (r - nq) * AD
+                                        : (__half*) a.vc + pos * gqa + (r - nq - nk) * AD;
+            dst[lane] = __float2half_rn(o0);
+            dst[lane + 64] = __float2half_rn(o1);
+        }
     }
 }
 
@@ -511,10 +529,11 @@ int launch_attn_core(const AttnArgs& a, hipStream_t st) {
     if (n_split <= 0 || n_split > 65535 || n_pv <= 0 || a.split % FK || !a.stat || !a.part || (a.att_q8K && n % QK_K) ||
         (!a.att_q8K && !a.att) || a.split * a.merge * (int64_t) nk * AD * 2 >= (int64_t(1) << 31))
         return -2;
-    // head rows per block: all of a token's for many tokens, four (one per wave) for few
-    const int hpb = a.T >= 128 ? nq + 2 * nk : 4;
-    hipLaunchKernelGGL(k_attn_qk_rope, dim3((unsigned) a.T, (unsigned) ((nq + 2 * nk + hpb - 1) / hpb)), dim3(256), 0, st,
-                       a, hpb);
+    // head rows per block: five per wave for many tokens, one for few (T = 1: 4.8 us)
+    const int hpb = a.T >= 128 ? 20 : 4;
+    const dim3 gr((unsigned) a.T, (unsigned) ((nq + 2 * nk + hpb - 1) / hpb));
+    if (hpb == 4) hipLaunchKernelGGL(k_attn_qk_rope<1>, gr, dim3(256), 0, st, a, hpb);
+    else hipLaunchKernelGGL(k_attn_qk_rope<5>, gr, dim3(256), 0, st, a, hpb);
     const int nw = attn_waves(rows);
     const unsigned rb = (unsigned) ((rows + 32 * nw - 1) / (32 * nw));
     const dim3 gs((unsigned) nk, rb, (unsigned) n_split), gp((unsigned) nk, rb, (unsigned) n_pv);
