@@ -861,7 +861,12 @@ int qwmoe_gdn_seg(void* stream, const qwmoe_gdn_layer* L, const float* h, int64_
         h = m ? (uint16_t*) m->act_h : nullptr;
         hd = m ? (float*) m->act_hd : nullptr;
     };
-    qw::RowGroups grp{rows, active, active_off, n_active, trows, tactive, toff, tn, tslot, T >= 64 ? 4 : 1};
+    // tokens per bin of beta and alpha: more share a weight row's load, fewer give more workgroups (us
+    // per call, H_v = 32, both Q8_0, one / two / four: 98.4 / 98.7 / 101.7 at T = 64, 110.9 / 111.4 /
+    // 114.3 at 128, 142.4 / 138.3 / 141.8 at 200, 182.8 / 177.6 / 182.7 at 300, 223.8 / 219.3 / 218.3 at
+    // 420, 427.8 / 416.0 / 416.5 at 1000)
+    const int tpb = T >= 400 ? 4 : T >= 128 ? 2 : 1;
+    qw::RowGroups grp{rows, active, active_off, n_active, trows, tactive, toff, tn, tslot, tpb};
     uint16_t* hx;
     float* hxd;
     copy_of(x80, hx, hxd);

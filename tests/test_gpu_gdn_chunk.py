@@ -1,9 +1,10 @@
 """GPU parity of the delta net's 16-token chunks (k_gdn_chunk, k_gdn_delta_chunk) at the
 edges of a chunk, of the batches that take them and of the 16 value heads one block
-takes at a time, and with a token whose values are not finite: nothing of it reaches the tokens before it or other rows of
-the state.  Against the CPU restatement, within the 1e-3 of the reference's magnitude
-that one rounding step of a re-quantized activation moves an output by; the state, that
-no quantization follows, within 2e-5: 128 products of sums of up to 33 fp32 terms (n eps
+takes at a time, with the last bin of beta and alpha part full, and with a token whose
+values are not finite: nothing of it reaches the tokens before it or other rows of the
+state.  Against the CPU restatement, within the 1e-3 of the reference's magnitude that
+one rounding step of a re-quantized activation moves an output by; the state, that no
+quantization follows, within 2e-5: 128 products of sums of up to 33 fp32 terms (n eps
 = 2e-6 each) over the restatement's float32 inputs."""
 from __future__ import annotations
 
@@ -34,7 +35,7 @@ def orc():
 
 
 @pytest.mark.parametrize("H_k,H_v,types", [(2, 4, (Q4_K, Q6_K, Q8_0, Q8_0, Q4_K)), (1, 17, (Q8_0,) * 5)])
-@pytest.mark.parametrize("T", [31, 32, 33, 47, 64, 65, 130])
+@pytest.mark.parametrize("T", [31, 32, 33, 47, 64, 65, 129, 402])
 def test_chunks(orc, H_k, H_v, types, T):
     gw = GdnWeights(512, 128, H_k, H_v, 4, types, 7 + T, orc)
     h = np.random.default_rng(T).standard_normal((T, 512)).astype(np.float32)

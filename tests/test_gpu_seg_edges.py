@@ -3,8 +3,8 @@
 Attention (attn.hip): query rows around 32 and 64 (one, two and four waves), chunks
 and splits of 64 keys around their ends, a first token without a past, heads per kv
 head that do not divide 32, an odd number of heads (f32 attention output), one and
-several PV splits.  Delta net (gdn.hip): tokens around the 4-token step, the 32-token
-block and the 64 tokens from which beta and alpha take four tokens per bin, every
+several PV splits.  Delta net (gdn.hip): tokens around the 4-token step, the 32
+tokens from which it takes 16 at a time and the ends of those chunks, every
 number of conv taps, an odd number of value heads, Q8_0 throughout.
 
 Against the CPU restatements (oracle_lib, pinned to ggml), within the 1e-3 of the
