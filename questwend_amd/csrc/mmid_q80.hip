@@ -36,19 +36,23 @@ typedef float q80_f16 __attribute__((ext_vector_type(16)));
 // one weight row, whose block scale it converts once for all its activation rows;
 // those rows' scales are one 16-byte LDS read.
 //
-// Workgroup: 64 weight rows (a wave per 16) x one item of up to 32 routed rows
-// (two tiles; an item of at most 16 rows computes one, as separate straight-line
-// code).  Eight blocks (272 weight bytes, 17 x 16) per step are copied straight
-// into LDS one step ahead (two buffers, 70 KB: two workgroups per CU).  The LDS
-// strides (272 and 1040 bytes) put the 16 rows of a tile on distinct banks.
+// Workgroup: 64 weight rows (a wave per 16) x one item of up to 16 routed rows.
+// Eight blocks (272 weight bytes, 17 x 16) per step are copied straight into LDS one
+// step ahead (two buffers).  52.7 KB and 112 VGPRs: three workgroups per CU, whose
+// products and fp32 steps cover each other's waits for copies.  Items of 32 rows (two
+// tiles share each weight operand, but 70 KB and 177 VGPRs leave two per CU) were slower
+// up to 32 rows per bin and no faster at 64; us per 30B layer, 32 / 16 rows per item: 97.5 /
+// 86.6 at T = 8, 207 / 184 at 33, 244 / 217 at 128, 308 / 282 at 251 (Zipf-skewed), 426 / 424 at
+// 512, 702 / 707 and 713 / 709 at 1024 (skewed, not); H = 1024, 64 experts: 99.1 / 88.5 at 400.
+// Weight rows sit 272 bytes apart, activation rows in pairs 1040 bytes apart, the odd
+// row's 16-byte chunk c at position c ^ 8: 16 rows read at one chunk hit distinct banks.
 //
-// Bound: VALU issue (41 instructions per tile and block against 64 cycles of
-// matrix core).  T = 251, 30B layer, Zipf-skewed: gate + up and down 124 us each
-// beside 113 us of GEMV for the light bins, the layer 2509 -> 393 us; the GEMV
-// alone took 1.8 ms per launch.
+// Bound: VALU issue (about 46 instructions per tile and block against 64 cycles of
+// matrix core) and the weights' bytes (T = 251: 430 MB of gate and up).  The GEMV alone
+// took 1.8 ms per launch at T = 251, the layer 2509 us.
 constexpr uint32_t Q80_WS = 272;     // LDS bytes of a staged weight row (8 blocks)
-constexpr uint32_t Q80_HS = 1040;    // LDS bytes of an activation copy instruction (rows i, i + 16, pad)
-constexpr int Q80_NR = 32;           // activation rows per item
+constexpr uint32_t Q80_HS = 1040;    // LDS bytes of an activation copy instruction (rows 2 i, 2 i + 1, pad)
+constexpr int Q80_NR = 16;           // activation rows per item
 constexpr int Q80_WDMA = MF_M * 17 / 64;   // weight copy instructions per step
 
 __device__ __forceinline__ q80_h4 q80_to_h4(uint32_t q) {
@@ -58,14 +62,14 @@ __device__ __forceinline__ q80_h4 q80_to_h4(uint32_t q) {
     return q80_h4{lo.x, lo.y, hi.x, hi.y};
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) k_mmid_mfma_q80(MfLaunch lp) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) k_mmid_mfma_q80(MfLaunch lp) {
     const uint32_t zm = blockIdx.x >= lp.groups ? 1u : 0u;   // uniform: which matrix
     const MmidArgs& m = lp.m[zm];
     const uint32_t bid = blockIdx.x - zm * lp.groups;
     __shared__ __align__(16) uint8_t s_w0[MF_M * Q80_WS];
     __shared__ __align__(16) uint8_t s_w1[MF_M * Q80_WS];
-    __shared__ __align__(16) uint8_t s_h0[16 * Q80_HS];
-    __shared__ __align__(16) uint8_t s_h1[16 * Q80_HS];
+    __shared__ __align__(16) uint8_t s_h0[8 * Q80_HS];
+    __shared__ __align__(16) uint8_t s_h1[8 * Q80_HS];
     __shared__ __align__(16) float s_d0[8 * Q80_NR];   // activation block scales [block][row]
     __shared__ __align__(16) float s_d1[8 * Q80_NR];
     __shared__ int32_t s_arow[Q80_NR];
@@ -102,7 +106,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         s_arow[tid] = (int) ((int64_t) (e % m.b_ne1) + (int64_t) t * m.b_ne1);
     }
     lds_barrier();
-    uint32_t woff[5], hoff[4];
+    uint32_t woff[5], hoff[2];
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
         const int q = 64 * (wave + 4 * k) + lane;
@@ -110,12 +114,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         woff[k] = (uint32_t) (qc / 17) * (uint32_t) m.nb1 + 16u * (uint32_t) (qc % 17);
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int n = wave + 4 * k + 16 * (lane >> 5);
-        hoff[k] = (uint32_t) s_arow[n] * (uint32_t) (2 * m.K) + 16u * (uint32_t) (lane & 31);
+    for (int k = 0; k < 2; ++k) {
+        const int up = lane >> 5, n = 2 * (wave + 4 * k) + up;
+        hoff[k] = (uint32_t) s_arow[n] * (uint32_t) (2 * m.K) + 16u * (uint32_t) ((lane & 31) ^ (8 * up));
     }
-    // block scales: instruction w brings blocks 2 w, 2 w + 1 of the step, all 32 rows
-    const uint32_t doff = (uint32_t) s_arow[lane & 31] * (uint32_t) (m.K / 8) + 4u * (uint32_t) (2 * wave + (lane >> 5));
+    // block scales: instruction w (of two) brings blocks 4 w .. 4 w + 3 of the step, all rows
+    const uint32_t doff = (uint32_t) s_arow[lr] * (uint32_t) (m.K / 8) + 4u * (uint32_t) (4 * wave + gq);
     auto issue = [&](uint8_t* sw, uint8_t* sh, float* sd, int i) __attribute__((always_inline)) {
         uint32_t lw = (uint32_t) (uintptr_t) sw, lh = (uint32_t) (uintptr_t) sh, ld = (uint32_t) (uintptr_t) sd;
         asm volatile("" : "+s"(lw), "+s"(lh), "+s"(ld));
@@ -123,85 +127,74 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int k = 0; k < 5; ++k)
             if (wv + 4 * k < Q80_WDMA) dma_b128(wrsrc, lw + 1024u * (uint32_t) (wv + 4 * k), woff[k], 272u * (uint32_t) i);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) dma_b128(hrsrc, lh + Q80_HS * (uint32_t) (wv + 4 * k), hoff[k], 512u * (uint32_t) i);
-        dma_b32(drsrc, ld + 256u * (uint32_t) wv, doff, 32u * (uint32_t) i);
+        for (int k = 0; k < 2; ++k) dma_b128(hrsrc, lh + Q80_HS * (uint32_t) (wv + 4 * k), hoff[k], 512u * (uint32_t) i);
+        if (wv < 2) dma_b32(drsrc, ld + 256u * (uint32_t) wv, doff, 32u * (uint32_t) i);
     };
-    auto run = [&](auto nbt_c) __attribute__((always_inline)) {
-        constexpr int NBT = decltype(nbt_c)::value;
-        float acc[NBT][4][8];
+    float acc[4][8];
 #pragma unroll
-        for (int t = 0; t < NBT; ++t)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+        for (int L = 0; L < 8; ++L) acc[r][L] = 0.0f;
+    auto compute = [&](const uint8_t* sw, const uint8_t* sh, const float* sd) __attribute__((always_inline)) {
+        const uint32_t* wr = (const uint32_t*) (sw + (16 * wave + lr) * Q80_WS);
+        const uint8_t* ah = sh + Q80_HS * (uint32_t) (lr >> 1) + 512 * (lr & 1) + 16 * gq;
+        const int odd = 128 * (lr & 1);   // (chunk 4 i + gq at position ^ 8)
 #pragma unroll
-                for (int L = 0; L < 8; ++L) acc[t][r][L] = 0.0f;
-        auto compute = [&](const uint8_t* sw, const uint8_t* sh, const float* sd) __attribute__((always_inline)) {
-            const uint32_t* wr = (const uint32_t*) (sw + (16 * wave + lr) * Q80_WS);
-            const uint8_t* ah = sh + Q80_HS * (uint32_t) lr + 16 * gq;
+        for (int p = 0; p < 4; ++p) {
+            // two blocks, 17 dwords: the even block's quants start 2 bytes into a dword
+            const uint32_t e0 = wr[17 * p + gq], e1 = wr[17 * p + gq + 1];
+            const uint32_t e2 = wr[17 * p + gq + 4], e3 = wr[17 * p + gq + 5];
+            const uint32_t o0 = wr[17 * p + gq + 9], o1 = wr[17 * p + gq + 13];
+            const uint32_t dd[2] = {wr[17 * p], wr[17 * p + 8]};
+            const uint32_t q0[2] = {__builtin_amdgcn_alignbyte(e1, e0, 2), o0};
+            const uint32_t q1[2] = {__builtin_amdgcn_alignbyte(e3, e2, 2), o1};
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                // two blocks, 17 dwords: the even block's quants start 2 bytes into a dword
-                const uint32_t e0 = wr[17 * p + gq], e1 = wr[17 * p + gq + 1];
-                const uint32_t e2 = wr[17 * p + gq + 4], e3 = wr[17 * p + gq + 5];
-                const uint32_t o0 = wr[17 * p + gq + 9], o1 = wr[17 * p + gq + 13];
-                const uint32_t dd[2] = {wr[17 * p], wr[17 * p + 8]};
-                const uint32_t q0[2] = {__builtin_amdgcn_alignbyte(e1, e0, 2), o0};
-                const uint32_t q1[2] = {__builtin_amdgcn_alignbyte(e3, e2, 2), o1};
+            for (int h = 0; h < 2; ++h) {
+                const int i = 2 * p + h;
+                const float dx = h2f((uint16_t) (h ? dd[h] >> 16 : dd[h] & 0xffffu));
+                const q80_h4 b0 = q80_to_h4(q0[h]), b1 = q80_to_h4(q1[h]);
+                const q80_h8 a = *(const q80_h8*) (ah + (i & 2 ? -odd : odd) + 64 * i);
+                const float4 dy = *(const float4*) (sd + Q80_NR * i + 4 * gq);
+                const q80_h4 a0 = {a[0], a[1], a[2], a[3]}, a1 = {a[4], a[5], a[6], a[7]};
+                q80_f16 z;
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int i = 2 * p + h;
-                    const float dx = h2f((uint16_t) (h ? dd[h] >> 16 : dd[h] & 0xffffu));
-                    const q80_h4 b0 = q80_to_h4(q0[h]), b1 = q80_to_h4(q1[h]);
+                for (int k = 0; k < 16; ++k) z[k] = 0.0f;
+                const q80_f16 s0 = __builtin_amdgcn_mfma_f32_16x16x4f16(a0, b0, z, 0, 0, 0);
+                const q80_f16 s1 = __builtin_amdgcn_mfma_f32_16x16x4f16(a1, b1, z, 0, 0, 0);
+                const float d[4] = {dx * dy.x, dx * dy.y, dx * dy.z, dx * dy.w};
 #pragma unroll
-                    for (int t = 0; t < NBT; ++t) {
-                        const q80_h8 a = *(const q80_h8*) (ah + 512 * t + 64 * i);
-                        const float4 dy = *(const float4*) (sd + Q80_NR * i + 16 * t + 4 * gq);
-                        const q80_h4 a0 = {a[0], a[1], a[2], a[3]}, a1 = {a[4], a[5], a[6], a[7]};
-                        q80_f16 z;
+                for (int r = 0; r < 4; ++r)
 #pragma unroll
-                        for (int k = 0; k < 16; ++k) z[k] = 0.0f;
-                        const q80_f16 s0 = __builtin_amdgcn_mfma_f32_16x16x4f16(a0, b0, z, 0, 0, 0);
-                        const q80_f16 s1 = __builtin_amdgcn_mfma_f32_16x16x4f16(a1, b1, z, 0, 0, 0);
-                        const float d[4] = {dx * dy.x, dx * dy.y, dx * dy.z, dx * dy.w};
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-#pragma unroll
-                            for (int L = 0; L < 4; ++L) {
-                                acc[t][r][L] = __builtin_fmaf(d[r], s0[4 * L + r], acc[t][r][L]);
-                                acc[t][r][4 + L] = __builtin_fmaf(d[r], s1[4 * L + r], acc[t][r][4 + L]);
-                            }
+                    for (int L = 0; L < 4; ++L) {
+                        acc[r][L] = __builtin_fmaf(d[r], s0[4 * L + r], acc[r][L]);
+                        acc[r][4 + L] = __builtin_fmaf(d[r], s1[4 * L + r], acc[r][4 + L]);
                     }
-                }
             }
-        };
-        issue(s_w0, s_h0, s_d0, 0);
-        for (int i = 0; i < steps; i += 2) {
-            vm_wait<0>();
-            lds_barrier();
-            if (i + 1 < steps) issue(s_w1, s_h1, s_d1, i + 1);
-            compute(s_w0, s_h0, s_d0);
-            if (i + 1 >= steps) break;
-            vm_wait<0>();
-            lds_barrier();
-            if (i + 2 < steps) issue(s_w0, s_h0, s_d0, i + 2);
-            compute(s_w1, s_h1, s_d1);
         }
-#pragma unroll
-        for (int t = 0; t < NBT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * t + 4 * gq + r;
-                const float* a = acc[t][r];
-                const float o = ((a[4] + a[0]) + (a[6] + a[2])) + ((a[5] + a[1]) + (a[7] + a[3]));
-                if (row < ntok) {
-                    const int e = s_et[row][0], tt = s_et[row][1];
-                    float* dp = (float*) ((char*) m.dst + (size_t) e * m.dst_nb1 + (size_t) tt * m.dst_nb2);
-                    dp[r0 + 16 * wave + lr] = o;
-                }
-            }
     };
-    if (__builtin_amdgcn_readfirstlane(ntok) > 16) run(std::integral_constant<int, 2>{});
-    else run(std::integral_constant<int, 1>{});
+    issue(s_w0, s_h0, s_d0, 0);
+    for (int i = 0; i < steps; i += 2) {
+        vm_wait<0>();
+        lds_barrier();
+        if (i + 1 < steps) issue(s_w1, s_h1, s_d1, i + 1);
+        compute(s_w0, s_h0, s_d0);
+        if (i + 1 >= steps) break;
+        vm_wait<0>();
+        lds_barrier();
+        if (i + 2 < steps) issue(s_w0, s_h0, s_d0, i + 2);
+        compute(s_w1, s_h1, s_d1);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int row = 4 * gq + r;
+        const float* a = acc[r];
+        const float o = ((a[4] + a[0]) + (a[6] + a[2])) + ((a[5] + a[1]) + (a[7] + a[3]));
+        if (row < ntok) {
+            const int e = s_et[row][0], tt = s_et[row][1];
+            float* dp = (float*) ((char*) m.dst + (size_t) e * m.dst_nb1 + (size_t) tt * m.dst_nb2);
+            dp[r0 + 16 * wave + lr] = o;
+        }
+    }
 }
 
 // Rows of 16-byte aligned groups of eight blocks; 64-row tiles.

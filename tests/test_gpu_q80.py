@@ -1,6 +1,6 @@
 """GPU parity of the Q8_0 mul_mat_id kernels (mmid_q80.hip): the matrix-core form
 and the row-copying GEMV, bit for bit against the CPU oracle, at the edges of
-their tiles: one row and full / partial 16- and 32-row items, weight rows that do
+their tiles: one row and full / partial 16-row items, weight rows that do
 not fill a 16-row workgroup, the smallest and larger row lengths, each activation
 row of a pass (1 to 4), the weights' extreme quants (-128), a workspace without
 room for the f16 copy, and the SwiGLU launch that writes Q8_0 rows directly."""
