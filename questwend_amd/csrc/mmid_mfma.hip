@@ -630,16 +630,16 @@ int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t row
 // k_mmid_mfma_hp computes what k_mmid_mfma_q4k_h computes -- the same A and
 // B operands, one v_mfma_f32_16x16x32_f16 per AVX lane and tile, the same fp32
 // steps in the same order, so the same bits -- with another schedule:
-//  - a grid of two workgroups per CU walks the work units u = b, b + grid, ...
+//  - a grid of two workgroups per CU (NT = 2; three with NT = 1) walks the work units u = b, b + grid, ...
 //    A unit is (item, 64-row weight tile) of one of the launch's one or two
-//    matrices; an item is up to 32 routed rows of one heavy expert.  Each
+//    matrices; an item is up to 16 NT routed rows of one heavy expert.  Each
 //    workgroup builds the item table (first item of each active expert) once in
 //    LDS; a unit's expert is a count over that table.
 //  - the copy pipeline (two stage buffers, one super-block ahead) runs on across
 //    units: while the last super-block of a unit is computed, the first one of the
 //    next unit is being copied.  The next unit's (e, t) pairs are copied into LDS by
 //    the same DMA path two super-blocks ahead.
-//  - two 16-row activation tiles per item: each A operand (sc * q4 of 16 weight
+//  - NT = 2, two 16-row activation tiles per item: each A operand (sc * q4 of 16 weight
 //    rows) serves 32 activation rows.  A last item of at most 16 rows computes
 //    one tile; those items are numbered after all others, so a workgroup runs
 //    its two-tile units, then its one-tile units, each as straight-line code
@@ -649,13 +649,16 @@ int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t row
 //  - activation rows i and i + 16 share one DMA instruction and sit 1040 bytes
 //    per pair apart (16 bytes of pad): the 16 rows a tile reads at one chunk
 //    offset fall on distinct LDS banks, and every B read is the lane's base plus
-//    a constant.
+//    a constant.  NT = 1: rows 2 i and 2 i + 1, the odd row's chunk c at position c ^ 8.
+//  - NT = 1, items of one tile, for light bins and small launches (the line: launch_mf):
+//    half the accumulators leave 134 (Q4_K) or 163 (Q6_K) registers and 40 or 53 KB, so
+//    three workgroups per CU cover each other's LDS and barrier waits.
 //  - the min lanes from the Q8_K blocks' bsums (an f16 copy behind the quants' one):
 //    prod_m is mins 2m, 2m, 2m + 1, 2m + 1 against bsums 4m .. 4m + 3, so one
 //    v_mfma_f32_16x16x4_4b_f16 forms all four min lanes of a tile from 8 bytes per
 //    lane, in place of eight 32-deep products over the quants read from LDS a
 //    second time (half of the kernel's LDS reads).
-// ~57 KB of LDS, 248 VGPRs: two workgroups per CU.  Needs K >= 768 (three
+// NT = 2: ~57 KB of LDS, 247 VGPRs, two workgroups per CU.  Needs K >= 768 (three
 // super-blocks: the next unit's pairs land before they are used) and at most
 // MP_MAXG active bins.  Bound: VALU issue (about 258 instructions per wave and
 // super-block, 96 of them ggml's own fma) with two waves per SIMD to hide each
@@ -688,10 +691,10 @@ struct MpUnit {
     i32x4 wrsrc;
 };
 
-template <int TYPE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
-    constexpr bool Q6 = TYPE == T_Q6_K;
+template <int TYPE, int NT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4 - NT, 4 - NT)))
+k_mmid_mfma_hp(MfLaunch lp, uint32_t nz) {
+    constexpr bool Q6 = TYPE == T_Q6_K, one_tile = NT == 1;
     // 16-byte chunks of a staged weight row: Q4_K the block's nine; Q6_K the 212 bytes
     // from the dword at or below the block's start (210-byte blocks start 2 bytes past
     // a dword in every other row or super-block) as chunks 0 .. 12, chunk 13 bytes
@@ -700,7 +703,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
     constexpr uint32_t WST = 16u * WCH;                   // LDS stride of a staged row
     constexpr int WDMA = MF_M * WCH / 64, WDW = (WDMA + 3) / 4;   // copy instructions per stage, per wave
     __shared__ __align__(16) uint8_t s_w[MP_ST][MF_M * WST];
-    __shared__ __align__(16) uint8_t s_h[MP_ST][16 * MP_HS];
+    __shared__ __align__(16) uint8_t s_h[MP_ST][8 * NT * MP_HS];
     __shared__ __align__(16) uint8_t s_b[MP_ST][MP_NR * 32];   // bsums (f16)
     __shared__ __align__(16) float s_d[MP_ST][MP_NR];
     __shared__ __align__(16) int32_t s_meta[2][2 * MP_NR];   // (e, t) of a unit's 32 rows
@@ -814,6 +817,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
             woff[k] = (uint32_t) (qc / WCH) * (uint32_t) m0.nb1 + 16u * (uint32_t) c;
         }
     }
+    constexpr int HC = 2 * NT;   // activation copy instructions per wave
     auto arow = [&](int mb, int nn) __attribute__((always_inline)) {
         // (32-bit: slot e >= 0 and 1 <= b_ne1 <= 65535 -- mp_ok -- give e % b_ne1 without
         // the 64-bit division's ~130 instructions per call)
@@ -822,17 +826,18 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
         const uint32_t er = bn == 1u ? 0u : e < bn ? e : e % bn;
         return er + t * bn;
     };
-    auto lane_offs = [&](int mb, int ntok, uint32_t (&ho)[4], uint32_t& dof, uint32_t& bof) __attribute__((always_inline)) {
+    auto lane_offs = [&](int mb, int ntok, uint32_t (&ho)[HC], uint32_t& dof, uint32_t& bof) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int nrow = wave + 4 * k + 16 * (lane >> 5);
-            ho[k] = arow(mb, nrow < ntok ? nrow : 0) * (uint32_t) (2 * m0.K) + 16u * (uint32_t) (lane & 31);
+        for (int k = 0; k < HC; ++k) {
+            const int up = lane >> 5, nrow = NT == 2 ? wave + 4 * k + 16 * up : 2 * (wave + 4 * k) + up;
+            ho[k] = arow(mb, nrow < ntok ? nrow : 0) * (uint32_t) (2 * m0.K) +
+                    16u * (uint32_t) (NT == 2 ? lane & 31 : (lane & 31) ^ (8 * up));
         }
         dof = arow(mb, lane < ntok && lane < MP_NR ? lane : 0) * (uint32_t) m0.act_row_bytes;
         bof = arow(mb, (lane >> 1) < ntok ? lane >> 1 : 0) * (uint32_t) (m0.K / 8) + 16u * (uint32_t) (lane & 1);
     };
     // copies of super-block i of a unit into stage buffer sb
-    auto issue = [&](int sb, const MpUnit& U, const uint32_t (&ho)[4], uint32_t dof, uint32_t bof, int i)
+    auto issue = [&](int sb, const MpUnit& U, const uint32_t (&ho)[HC], uint32_t dof, uint32_t bof, int i)
         __attribute__((always_inline)) {
         uint32_t lw = (uint32_t) (uintptr_t) s_w[sb], lh = (uint32_t) (uintptr_t) s_h[sb];
         uint32_t ld = (uint32_t) (uintptr_t) s_d[sb], lb = (uint32_t) (uintptr_t) s_b[sb];
@@ -847,15 +852,15 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
                     dma_b128(U.wrsrc, lw + 1024u * (uint32_t) (wv + 4 * k), woff[k], 144u * (uint32_t) i);
             }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) dma_b128(hrsrc, lh + MP_HS * (uint32_t) (wv + 4 * k), ho[k], 512u * (uint32_t) i);
+        for (int k = 0; k < HC; ++k) dma_b128(hrsrc, lh + MP_HS * (uint32_t) (wv + 4 * k), ho[k], 512u * (uint32_t) i);
         if (wv == 3 && lane < MP_NR) dma_b32(arsrc, ld, dof, 292u * (uint32_t) i);
         if (wv == 2) dma_b128(brsrc, lb, bof, 32u * (uint32_t) i);   // row lane / 2, half lane % 2
     };
 
-    float acc[2][4][8], accm[Q6 ? 1 : 2][4][4];
+    float acc[NT][4][8], accm[Q6 ? 1 : NT][4][4];
     auto zero = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
 #pragma unroll
@@ -867,6 +872,9 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
     uint32_t hmag = 0x64006400u;
     asm volatile("" : "+v"(hmag));
     const int arow_l = 16 * wave + lr;
+    // this lane's activation row and 16-byte chunks 8 gq .. + 7 of it in a stage
+    const uint32_t hrow = NT == 2 ? MP_HS * (uint32_t) lr + 128u * (uint32_t) gq
+                                  : MP_HS * (uint32_t) (lr >> 1) + 512u * (uint32_t) (lr & 1) + 128u * (uint32_t) (gq ^ (lr & 1));
     // NBT activation tiles (1 or 2, a compile-time constant): straight-line code
     // from each matrix-core instruction to the reads of its result.  (With the tile
     // count tested inside the unrolled loops, the compiler put its wait states for
@@ -875,7 +883,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
     auto compute_q4k = [&](int sb, auto nbt_c) __attribute__((always_inline)) {
         constexpr int NBT = decltype(nbt_c)::value;
         const uint8_t* sw = s_w[sb];
-        const uint8_t* sh = s_h[sb] + MP_HS * (uint32_t) lr;   // this lane's rows: lr (tile 0), lr + 16 (tile 1)
+        const uint8_t* sh = s_h[sb] + hrow;   // this lane's rows: lr (tile 0), lr + 16 (tile 1)
         const float* sd = s_d[sb];
         // this lane's A row: the 6-bit scales and mins of the 8 sub-blocks (quants.c:2067-2072);
         // the fp16 d / dmin of the four rows of its D registers; the activation rows' d.
@@ -944,14 +952,14 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
         f4m Dp[NBT];
         h8m Bc[NBT];
 #pragma unroll
-        for (int t = 0; t < NBT; ++t) Bc[t] = *(const h8m*) (sh + 512 * t + 16 * (8 * gq));
+        for (int t = 0; t < NBT; ++t) Bc[t] = *(const h8m*) (sh + 512 * t);
 #pragma unroll
         for (int L = 0; L < 8; ++L) {
             const uint32_t w = wl[L];
             h8m Bn[NBT];
 #pragma unroll
             for (int t = 0; t < NBT; ++t)
-                Bn[t] = L < 7 ? *(const h8m*) (sh + 512 * t + 16 * (8 * gq + L + 1)) : Bc[t];
+                Bn[t] = L < 7 ? *(const h8m*) (sh + 512 * t + 16 * (L + 1)) : Bc[t];
             __builtin_amdgcn_sched_barrier(0);   // (keeps those reads issued here, a step ahead)
             const uint32_t v = w >> 8;
             const h2m a0 = __builtin_elementwise_fma(h2_bits((w & 0x000F000Fu) | hmag), S_lo, C_lo);
@@ -989,7 +997,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
     // Q6_K (see above): super-block i of the unit
     auto compute_q6k = [&](int sb, int i, auto nbt_c) __attribute__((always_inline)) {
         constexpr int NBT = decltype(nbt_c)::value;
-        const uint8_t* sh = s_h[sb] + MP_HS * (uint32_t) lr;
+        const uint8_t* sh = s_h[sb] + hrow;
         const float* sd = s_d[sb];
         const uint32_t nb1 = (uint32_t) m0.nb1, si = 2u * ((uint32_t) i & 1u);
         const uint32_t off = (((uint32_t) arow_l * nb1) & 2u) ^ si;   // the block's byte offset in its window
@@ -1044,7 +1052,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
         f4m Plo[NBT], Phi[NBT];
         h8m Bc[NBT];
 #pragma unroll
-        for (int t = 0; t < NBT; ++t) Bc[t] = *(const h8m*) (sh + 512 * t + 16 * (8 * gq));
+        for (int t = 0; t < NBT; ++t) Bc[t] = *(const h8m*) (sh + 512 * t);
         auto step = [&](int t, int L) __attribute__((always_inline)) {   // lane L's fp32 steps: (float) (16 hi + lo) is one rounding
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -1066,7 +1074,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
             const h8m Alo = four(S_lo, C_lo), Ahi = four(S_hi, C_hi);
             h8m Bn[NBT];
 #pragma unroll
-            for (int t = 0; t < NBT; ++t) Bn[t] = L < 7 ? *(const h8m*) (sh + 512 * t + 16 * (8 * gq + L + 1)) : Bc[t];
+            for (int t = 0; t < NBT; ++t) Bn[t] = L < 7 ? *(const h8m*) (sh + 512 * t + 16 * (L + 1)) : Bc[t];
             __builtin_amdgcn_sched_barrier(0);
             u32x4m ab = {0u, 0u, 0u, 0u};
             ab[L & 3] = gq == L >> 2 ? bp[L & 3] : 0u;
@@ -1132,10 +1140,10 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
     if (wv == 0) dma_b32(prsrc, (uint32_t) (uintptr_t) s_meta[0], 4u * (uint32_t) lane, 8u * (uint32_t) cur.p0);
     vm_wait<0>();
     lds_barrier();
-    uint32_t ho[4], dof, bof, hn[4], dn = 0, bn = 0;
+    uint32_t ho[HC], dof, bof, hn[HC], dn = 0, bn = 0;
     lane_offs(0, cur.ntok, ho, dof, bof);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) hn[k] = ho[k];
+    for (int k = 0; k < HC; ++k) hn[k] = ho[k];
     zero();
     issue(0, cur, ho, dof, bof, 0);
     const int S = my_units * nb;
@@ -1166,7 +1174,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
             zero();
             cur = nxt;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) ho[k] = hn[k];
+            for (int k = 0; k < HC; ++k) ho[k] = hn[k];
             dof = dn;
             bof = bn;
             i = 0;
@@ -1175,7 +1183,9 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz, uint32_t one_tile) {
         sb ^= 1;
         ++s;
     };
-    while (s < S && cur.ntok > 16) step(std::integral_constant<int, 2>{});
+    if constexpr (NT == 2) {
+        while (s < S && cur.ntok > 16) step(std::integral_constant<int, 2>{});
+    }
     while (s < S) step(std::integral_constant<int, 1>{});
 }
 
@@ -1692,7 +1702,7 @@ static bool mp_ok(const MfLaunch& lp, int nz) {
     return !(e && e[0] == '0');
 }
 
-// Two workgroups per CU of the current device (cached per device).
+// Two workgroups per CU of the current device (cached per device): the two-tile form's grid.
 static unsigned mp_grid() {
     static int cus[64] = {0};
     int dev = 0;
@@ -1710,19 +1720,24 @@ static int launch_mf(const MfLaunch& lp, int nz, hipStream_t stream) {
     if (lp.groups == 0) return 0;
     if (m.type == T_Q8_0) return launch_mf_q80(lp, nz, stream);
     if (mp_ok(lp, nz)) {
-        // at most (items of 32 rows) x tiles x nz units: no more workgroups than that.
-        // Units for half of the workgroups or fewer: items of 16 rows (one tile), twice
-        // the workgroups with half the work each (a 512-row Q6_K projection of 512
-        // tokens: 23.3 -> 17.9 us with the bsum form below 256 registers)
+        // at most items x tiles x nz units: no more workgroups than that.  Items of 16 rows
+        // (NT = 1) for
+        //  - units for half of the two-tile form's workgroups or fewer: twice the
+        //    workgroups with half the work each (attention half, T = 64: 107 -> 96 us);
+        //  - up to 13 rows per bin, where most items hold one tile anyway (us per layer,
+        //    NT = 2 / 1, 128 experts): Q4_K 67.6 / 60.7 at 0.5 rows per bin, 147 / 127 at 4,
+        //    153 / 138 at 8, 169 / 165 at 16, 233 / 247 at 32; Q6_K 221 / 188 at 4, 234 / 212 at
+        //    12.5, 259 / 282 at 19; Q4_K + Q6_K at H = 4096 516 / 449 at 4, 525 / 465 at 8, 582 / 619
+        //    at 16, 1467 / 1715 at 64.
         int64_t units = mf_max_items(m, MP_NR) * (m.N / MF_M) * nz;
-        const uint32_t one = 2 * units <= (int64_t) mp_grid() ? 1u : 0u;
+        const int64_t bins = std::min<int64_t>(m.max_active, m.n_pairs / std::max(m.mfma_min_rows, 1));
+        const bool one = 2 * units <= (int64_t) mp_grid() || m.n_pairs <= 13 * bins;
         if (one) units = mf_max_items(m, 16) * (m.N / MF_M) * nz;
-        const unsigned grid = (unsigned) std::min<int64_t>(units, (int64_t) mp_grid());
+        const unsigned grid = (unsigned) std::min<int64_t>(units, (int64_t) mp_grid() / 2 * (one ? 3 : 2));
         if (grid == 0) return 0;
-        if (m.type == T_Q6_K)
-            hipLaunchKernelGGL(k_mmid_mfma_hp<T_Q6_K>, dim3(grid), dim3(256), 0, stream, lp, (uint32_t) nz, one);
-        else
-            hipLaunchKernelGGL(k_mmid_mfma_hp<T_Q4_K>, dim3(grid), dim3(256), 0, stream, lp, (uint32_t) nz, one);
+        auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, stream, lp, (uint32_t) nz); };
+        if (m.type == T_Q6_K) one ? go(k_mmid_mfma_hp<T_Q6_K, 1>) : go(k_mmid_mfma_hp<T_Q6_K, 2>);
+        else one ? go(k_mmid_mfma_hp<T_Q4_K, 1>) : go(k_mmid_mfma_hp<T_Q4_K, 2>);
         return hipGetLastError() == hipSuccess ? 0 : -3;
     }
     const unsigned grid = lp.groups * (unsigned) nz;

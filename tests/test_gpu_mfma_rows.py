@@ -2,7 +2,8 @@
 of the whole range -- every quant, every 6-bit or int8 scale, extreme activations
 -- bit for bit against the CPU oracle: Q4_K and Q6_K, row lengths whose Q6_K rows
 start on and off a dword, one- and two-tile items of every remainder, launches small
-enough for 16-row items and large enough for 32-row ones, all bins on the matrix
+enough for 16-row items and large enough for 32-row ones, light bins in more 16-row
+units than workgroups, all bins on the matrix
 cores and only those of eight rows or more."""
 from __future__ import annotations
 
@@ -59,6 +60,26 @@ def test_raw_blocks(orc, t, K, N, min_rows, many):
     b = rng.standard_normal((ids.shape[0], 1, K)).astype(np.float32)
     b[0] = np.float32(3.0)               # a row of equal values: quants all -127
     b[1, 0, 256:512] = 0.0
+    prev = ops.set_mfma_min_rows(min_rows)
+    try:
+        got = host(ops.mul_mat_id(t, dev(w), K, N, n_as, dev(b), dev(ids)))
+    finally:
+        ops.set_mfma_min_rows(prev)
+    assert np.array_equal(bits(got), bits(orc.mul_mat_id(t, K, N, n_as, w, b, ids)))
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("min_rows,per_bin", [(1, 13), (1, 14), (8, 13)])
+def test_light_bins(orc, t, min_rows, per_bin):
+    """The line of the 16-row items, 13 rows per bin, with more units (16 tiles of 64 weight
+    rows per item) than the 768 workgroups, so that they walk from unit to unit."""
+    K, N, n_as = 768, 1024, 48
+    rng = np.random.default_rng(per_bin + min_rows)
+    counts = np.tile([1, 16, 17, 33, 2, 9], n_as // 6)   # 13 per bin
+    counts[0] += (per_bin - 13) * n_as
+    w = raw_blocks(rng, t, n_as * N, K)
+    ids = rng.permutation(np.repeat(np.arange(n_as), counts)).astype(np.int32).reshape(-1, 1)
+    b = rng.standard_normal((ids.shape[0], 1, K)).astype(np.float32)
     prev = ops.set_mfma_min_rows(min_rows)
     try:
         got = host(ops.mul_mat_id(t, dev(w), K, N, n_as, dev(b), dev(ids)))
