@@ -177,7 +177,8 @@ int mfma_f16_prep_pair(Arena& ar, qw::MmidArgs& mu, qw::MmidArgs& mg, int64_t n_
 //    shape 43.9 / 35.4 at T = 8 (512 x 256 experts), 86.0 / 85.5 at T = 10 (55.4 / 50.6 with
 //    every token routed alike), 119.5 / 113.4 at T = 16, 181.6 / 146.1 at T = 33,
 //    312.5 / 267.4 at T = 512; Q8_0 69.1 / 66.2 at T = 4, 82.3 / 82.4 at T = 6, 86.1 /
-//    86.4 at T = 7 (64 experts, 4 per token: 33.6 / 36.5 at T = 6, 35.5 / 37.3 at T = 7).  Q6_K forms more integers per tile: 109.6 / 125.8 at T = 10,
+//    86.4 at T = 7 (64 experts, 4 per token: 33.6 / 36.5 at T = 6, 35.5 / 37.3 at T = 7).
+//    Q6_K forms more integers per tile: 109.6 / 125.8 at T = 10,
 //    142.0 / 157.6 at T = 16, 214.5 / 203.9 at T = 33, 230.7 / 205.3 at T = 64 (4 pairs
 //    per bin), but as the down projection at H = 4096 459.7 / 510.6 at T = 33,
 //    490.8 / 508.1 at T = 64, 539.5 / 551.2 at T = 128.

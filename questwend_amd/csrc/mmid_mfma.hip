@@ -1192,8 +1192,7 @@ k_mmid_mfma_hp(MfLaunch lp, uint32_t nz) {
 
 // Q6_K x Q8_K on the matrix cores, block-sum form only: the down projections of
 // the layer entry points under QWMOE_MFMA_AUTO, every projection under
-// QWMOE_MFMA_BLOCK_SUM.  (Replaying ggml's eight float lanes for Q6_K is not
-// done on the matrix cores; the exact form keeps Q6_K on the GEMV.)
+// QWMOE_MFMA_BLOCK_SUM.  (The exact forms are k_mmid_mfma_hp and k_mmid_mfma_q6k_x.)
 //
 // Reference: ggml_vec_dot_q6_K_q8_K (ggml/src/ggml-cpu/arch/x86/quants.c:
 // 2426-2508).  Its integers, per (weight row, activation row, super-block):
