@@ -387,7 +387,9 @@ typedef struct qwmoe_gdn_layer {
  * The projections are the quantized mul_mat row dots (ggml's bits); the rest
  * agrees with the reference CPU graph within float rounding (1e-3).  Calls
  * carry the layer's states: one call of T tokens equals consecutive calls of
- * its parts.  Workspace ~4 T (3 conv_ch + 5 d_inner + 2 H) bytes plus the
+ * its parts, bit for bit while T < 32 (decode steps, a verify batch); from 32
+ * tokens on the recurrence sums sixteen tokens at a time, and a call equals
+ * its parts within fp32 rounding.  Workspace ~4 T (3 conv_ch + 5 d_inner + 2 H) bytes plus the
  * quantized activations. */
 int qwmoe_gdn_seg(void * stream, const qwmoe_gdn_layer * layer, const float * h, int64_t T, float rms_eps,
                   float * attn_resid, float * ffn_in);

@@ -28,7 +28,7 @@ namespace qw {
 namespace {
 
 constexpr int GS = 128;        // state size S (ssm.state_size of the Qwen3-Next family)
-constexpr int GJB = 16;        // state rows j per workgroup of the recurrence (16 lanes per row)
+constexpr int GJB = 32;        // state rows j per workgroup of the token-by-token recurrence (8 lanes per row)
 
 // Four channels and CT tokens per thread: the DC-tap windows over [conv_state |
 // qkv rows] ending at each token (x_0 .. x_{DC-2} are the state, x_{DC-1+t} =
@@ -132,215 +132,109 @@ __global__ void __launch_bounds__(GS) k_gdn_prep(GdnArgs a) {
     a.kn[((int64_t) t * a.H_k + hk) * GS + i] = k * sck;
 }
 
-// The recurrence, four tokens at a time.  Workgroup (value head hv, rows j0 .. j0 +
-// GJB - 1 of its state M = S^T): 16 lanes per row, each holding 8 of its 128 columns
-// in registers for all tokens.  Per token ggml has M *= e (e = exp(g)); delta_j =
-// (v_j - M_j . k) beta; M_j += delta_j k; o_j = (M_j . q) / sqrt(S).  Token by token
-// that is one row reduction after another, 740 cycles each with a wave per SIMD.  From
-// the state M before tokens 1 .. 4 (E_b = e_1 .. e_b, E_{a,b} = e_{a+1} .. e_b),
-//     M k at token b       = E_b (M . k_b) + sum_{a < b}  E_{a,b} delta_a (k_a . k_b)
-//     o at token b sqrt(S) = E_b (M . q_b) + sum_{a <= b} E_{a,b} delta_a (k_a . q_b)
-//     M after              = E_4 M + sum_a E_{a,4} delta_a k_a
-// so the eight reductions over the row's 16 lanes are independent, and what depends
-// token on token is a few scalar steps.  The products P = E_{a,b} (k_a . k_b) and Q =
-// E_{a,b} (k_a . q_b) are the same for every row: formed once per workgroup and block
-// of GTB tokens, in LDS.  All in fp32 (the reference's sums in another order).
+// The recurrence token by token, for batches of fewer than GCHUNK_MIN tokens.
+// Workgroup (value head hv, rows j0 .. j0 + GJB - 1 of its state M = S^T): 8 lanes per
+// row, each holding 16 of its 128 columns in registers for all tokens.  Per token, as
+// ggml: M *= exp(g); delta_j = (v_j - M_j . k) beta; M_j += delta_j k; o_j = (M_j . q) /
+// sqrt(S).  A row's dots are reduced over its 8 lanes by DPP (quad xor 1, xor 2, half-row
+// mirror).  Nothing of a token's steps depends on where it stands in the call, so a call
+// gives the bits that calls of its parts give (decode steps and a verify batch agree).
+// q, k (the key head), v (the workgroup's rows), beta and exp(g) sit in LDS.
 //
-// Up to GTB tokens: q, k (the key head), v (the workgroup's rows), beta and g sit in LDS.
-// Tokens past T have k = 0, e = 1 and delta = 0: they change nothing.  About 1 us per step
-// (LDS reads, 24 of 16 bytes per lane and step with one workgroup per CU); token by token
-// 1.35 us per four.
+// Bound: the chain of the two row reductions per token, with a wave per SIMD (0.34 us a
+// token).  Four tokens per step, whose reductions are independent, take 0.25 us a token
+// but round each token by its place in the call.
 typedef float fx4 __attribute__((ext_vector_type(4)));   // (arrays of it stay in registers)
 constexpr int GTB = 32;   // tokens staged
-constexpr int GC = 4;     // tokens per step
 __global__ void __launch_bounds__(256) k_gdn_delta(GdnArgs a) {
-    const int hv = blockIdx.x, tid = threadIdx.x, r = tid >> 4, l = tid & 15;
+    const int hv = blockIdx.x, tid = threadIdx.x, r = tid >> 3, l = tid & 7;
     const int j0 = blockIdx.y * GJB, j = j0 + r, hk = hv % a.H_k;
     __shared__ __align__(16) float s_q[GTB][GS];
     __shared__ __align__(16) float s_k[GTB][GS];
-    __shared__ __align__(16) float s_v[GJB][GTB];              // [row][token]
-    __shared__ __align__(16) float s_b[GTB], s_e[GTB];
-    __shared__ __align__(16) float s_S[GTB / GC][24];          // per step: P (6), Q (10), E_b (4), E_{a,4} (4)
-    static_assert(GJB * 16 == 256 && GTB * GS / 4 == 4 * 256 && GTB * GJB == 2 * 256, "the loads' split over 256 threads");
-    float* st = a.state + ((int64_t) hv * GS + j) * GS + 4 * l;   // columns 4 l .. + 3 and 64 + 4 l .. + 3
-    fx4 m0 = *(const fx4*) st, m1 = *(const fx4*) (st + 64);
+    __shared__ float s_v[GTB][GJB];
+    __shared__ float s_b[GTB], s_e[GTB];
+    static_assert(GJB * 8 == 256 && GTB * GS / 4 == 4 * 256 && GTB * GJB == 4 * 256, "the loads' split over 256 threads");
+    float* st = a.state + ((int64_t) hv * GS + j) * GS + 16 * l;
+    fx4 m[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[i] = *(const fx4*) (st + 4 * i);
     const float scale = 1.0f / sqrtf((float) GS);
     const int64_t vbase = 2 * (int64_t) a.H_k * GS + (int64_t) hv * GS + j0;
-    auto dot4 = [](fx4 x, fx4 y, float s) __attribute__((always_inline)) {
-        s = __builtin_fmaf(x.x, y.x, s);
-        s = __builtin_fmaf(x.y, y.y, s);
-        s = __builtin_fmaf(x.z, y.z, s);
-        return __builtin_fmaf(x.w, y.w, s);
-    };
-    {
-        const int qcol = 4 * (tid % (GS / 4));
+    const int qcol = 4 * (tid % (GS / 4));
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int tt = tid / (GS / 4) + 8 * u;
-            const int64_t row = ((int64_t) min(tt, a.T - 1) * a.H_k + hk) * GS + qcol;
-            *(fx4*) &s_q[tt][qcol] = *(const fx4*) (a.qn + row);
-            const fx4 k = *(const fx4*) (a.kn + row);
-            *(fx4*) &s_k[tt][qcol] = tt < a.T ? k : fx4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int tt = tid / GJB + 16 * u;
-            s_v[tid % GJB][tt] = a.conv[(int64_t) min(tt, a.T - 1) * a.conv_ch + vbase + tid % GJB];
-        }
-        if (tid < 2 * GTB) {
-            const int t = tid >> 1;
-            const float bg = t < a.T ? a.bg[((int64_t) t * a.H_v + hv) * 2 + (tid & 1)] : 0.0f;
-            if (tid & 1) s_e[t] = expf(bg);
-            else s_b[t] = bg;
-        }
-        __syncthreads();
-        {   // P and Q: 8 lanes per token b of a step, lane p its columns 4 p + 32 i .. + 3
-            const int grp = tid >> 3, p = tid & 7, c = grp >> 2, b = grp & 3, t0 = GC * c;
-            float dk[GC], dq[GC];
-            fx4 kb[4], qb[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                kb[i] = *(const fx4*) &s_k[t0 + b][4 * p + 32 * i];
-                qb[i] = *(const fx4*) &s_q[t0 + b][4 * p + 32 * i];
-            }
-#pragma unroll
-            for (int x = 0; x < GC; ++x) {
-                dk[x] = dq[x] = 0.0f;
-                if (x <= b) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const fx4 ka = *(const fx4*) &s_k[t0 + x][4 * p + 32 * i];
-                        dk[x] = dot4(ka, kb[i], dk[x]);
-                        dq[x] = dot4(ka, qb[i], dq[x]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int x = 0; x < GC; ++x) {
-                dk[x] += dpp_f<DPP_XOR1>(dk[x]);
-                dq[x] += dpp_f<DPP_XOR1>(dq[x]);
-                dk[x] += dpp_f<DPP_XOR2>(dk[x]);
-                dq[x] += dpp_f<DPP_XOR2>(dq[x]);
-                dk[x] += dpp_f<DPP_HALF_MIRROR>(dk[x]);
-                dq[x] += dpp_f<DPP_HALF_MIRROR>(dq[x]);
-            }
-            // E_{x,b} as the product of the decays between
-            float E[GC], Eb = 1.0f, E4 = 1.0f;
-#pragma unroll
-            for (int x = 0; x < GC; ++x) {
-                E[x] = 1.0f;
-#pragma unroll
-                for (int y = 1; y < GC; ++y) {
-                    if (y > x && y <= b) E[x] *= s_e[t0 + y];
-                }
-                if (x <= b) Eb *= s_e[t0 + x];
-                if (x > b) E4 *= s_e[t0 + x];
-            }
-            if (p == 0) {
-#pragma unroll
-                for (int x = 0; x < GC; ++x) {   // P of (a, b) at b (b - 1) / 2 + a, Q of (a, b) at 6 + b (b + 1) / 2 + a
-                    if (x < b) s_S[c][b * (b - 1) / 2 + x] = E[x] * dk[x];
-                    if (x <= b) s_S[c][6 + b * (b + 1) / 2 + x] = E[x] * dq[x];
-                }
-                s_S[c][16 + b] = Eb;
-                s_S[c][20 + b] = E4;
-            }
-        }
-        __syncthreads();
-        const int nt = a.T;
-#pragma unroll 1
-        for (int tt = 0; tt < nt; tt += GC) {
-            fx4 k0[GC], k1[GC], q0[GC], q1[GC], s6[6];
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                k0[b] = *(const fx4*) &s_k[tt + b][4 * l];
-                k1[b] = *(const fx4*) &s_k[tt + b][64 + 4 * l];
-                q0[b] = *(const fx4*) &s_q[tt + b][4 * l];
-                q1[b] = *(const fx4*) &s_q[tt + b][64 + 4 * l];
-            }
-#pragma unroll
-            for (int i = 0; i < 6; ++i) s6[i] = *(const fx4*) &s_S[tt / GC][4 * i];
-            const fx4 v = *(const fx4*) &s_v[r][tt], bt = *(const fx4*) &s_b[tt];
-            auto S = [&](int i) __attribute__((always_inline)) { return s6[i >> 2][i & 3]; };
-            float xk[GC], xq[GC];
-#pragma unroll
-            for (int b = 0; b < GC; ++b) xk[b] = dot4(m0, k0[b], 0.0f) + dot4(m1, k1[b], 0.0f);
-#pragma unroll
-            for (int b = 0; b < GC; ++b) xq[b] = dot4(m0, q0[b], 0.0f) + dot4(m1, q1[b], 0.0f);
-            // the row's 16 lanes
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                xk[b] += dpp_f<DPP_XOR1>(xk[b]);
-                xq[b] += dpp_f<DPP_XOR1>(xq[b]);
-            }
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                xk[b] += dpp_f<DPP_XOR2>(xk[b]);
-                xq[b] += dpp_f<DPP_XOR2>(xq[b]);
-            }
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                xk[b] += dpp_f<DPP_HALF_MIRROR>(xk[b]);
-                xq[b] += dpp_f<DPP_HALF_MIRROR>(xq[b]);
-            }
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                xk[b] += dpp_f<DPP_MIRROR>(xk[b]);
-                xq[b] += dpp_f<DPP_MIRROR>(xq[b]);
-            }
-            float dl[GC], oo[GC];
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                float x = S(16 + b) * xk[b];
-#pragma unroll
-                for (int y = 0; y < b; ++y) x = __builtin_fmaf(dl[y], S(b * (b - 1) / 2 + y), x);
-                dl[b] = tt + b < nt ? (v[b] - x) * bt[b] : 0.0f;
-            }
-            m0 *= S(19);
-            m1 *= S(19);
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                const float f = S(20 + b) * dl[b];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    m0[i] = __builtin_fmaf(k0[b][i], f, m0[i]);
-                    m1[i] = __builtin_fmaf(k1[b][i], f, m1[i]);
-                }
-            }
-#pragma unroll
-            for (int b = 0; b < GC; ++b) {
-                float s = S(16 + b) * xq[b];
-#pragma unroll
-                for (int y = 0; y <= b; ++y) s = __builtin_fmaf(dl[y], S(6 + b * (b + 1) / 2 + y), s);
-                oo[b] = s * scale;
-            }
-            // lane b of the row writes token tt + b
-            const float ov = l == 0 ? oo[0] : l == 1 ? oo[1] : l == 2 ? oo[2] : oo[3];
-            if (l < GC && tt + l < nt) a.o[((int64_t) (tt + l) * a.H_v + hv) * GS + j] = ov;
-        }
+    for (int u = 0; u < 4; ++u) {
+        const int tq = tid / (GS / 4) + 8 * u, tv = tid / GJB + 8 * u;
+        const int64_t row = ((int64_t) min(tq, a.T - 1) * a.H_k + hk) * GS + qcol;
+        *(fx4*) &s_q[tq][qcol] = *(const fx4*) (a.qn + row);
+        *(fx4*) &s_k[tq][qcol] = *(const fx4*) (a.kn + row);
+        s_v[tv][tid % GJB] = a.conv[(int64_t) min(tv, a.T - 1) * a.conv_ch + vbase + tid % GJB];
     }
-    *(fx4*) st = m0;
-    *(fx4*) (st + 64) = m1;
+    if (tid < 2 * GTB) {
+        const float bg = a.bg[((int64_t) min(tid >> 1, a.T - 1) * a.H_v + hv) * 2 + (tid & 1)];
+        if (tid & 1) s_e[tid >> 1] = expf(bg);
+        else s_b[tid >> 1] = bg;
+    }
+    auto red8 = [](float x) __attribute__((always_inline)) {
+        x = x + dpp_f<DPP_XOR1>(x);
+        x = x + dpp_f<DPP_XOR2>(x);
+        return x + dpp_f<DPP_HALF_MIRROR>(x);
+    };
+    __syncthreads();
+#pragma unroll 1
+    for (int t = 0; t < a.T; ++t) {
+        const float e = s_e[t];
+        fx4 q[4], k[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            q[i] = *(const fx4*) &s_q[t][16 * l + 4 * i];
+            k[i] = *(const fx4*) &s_k[t][16 * l + 4 * i];
+        }
+        float d0 = 0.0f, d1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            m[i] *= e;
+            d0 = __builtin_fmaf(m[i].x, k[i].x, d0);
+            d1 = __builtin_fmaf(m[i].y, k[i].y, d1);
+            d0 = __builtin_fmaf(m[i].z, k[i].z, d0);
+            d1 = __builtin_fmaf(m[i].w, k[i].w, d1);
+        }
+        const float delta = (s_v[t][r] - red8(d0 + d1)) * s_b[t];
+        float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) m[i][c] = __builtin_fmaf(k[i][c], delta, m[i][c]);
+            o0 = __builtin_fmaf(m[i].x, q[i].x, o0);
+            o1 = __builtin_fmaf(m[i].y, q[i].y, o1);
+            o0 = __builtin_fmaf(m[i].z, q[i].z, o0);
+            o1 = __builtin_fmaf(m[i].w, q[i].w, o1);
+        }
+        const float o = red8(o0 + o1);
+        if (l == 0) a.o[((int64_t) t * a.H_v + hv) * GS + j] = o * scale;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(fx4*) (st + 4 * i) = m[i];
 }
 
 // ---- batches of GCHUNK_MIN tokens and more: sixteen tokens per step, on the matrix cores ----
 //
 // With D the deltas of a chunk's 16 tokens (a row per token), V, K, Q its rows, M the
-// state before it and E_b, E_{a,b} as above, the four-token form's equations read
+// state before it, E_b = e_1 .. e_b and E_{a,b} = e_{a+1} .. e_b, the recurrence reads
 //     (I + A) D = R = beta (V - E K M^T),     A[b][a] = beta_b E_{a,b} (k_a . k_b), a < b
 //     O sqrt(S) = E Q M^T + P D,              P[b][a] = E_{a,b} (k_a . q_b),        a <= b
 //     M^T after = E_16 M^T + K^T (E_{a,16} D)
 // A and P hold nothing of the state: k_gdn_chunk forms P and T = (I + A)^-1 (16 x 16,
 // forward substitution) for every chunk and head at once, and the serial kernel is left
 // with five small fp32 matrix products per chunk.
-// From 32 tokens on (us per call, H_v = 32, four tokens a step / chunks): 86.7 / 87.3 at T = 16,
-// 88.1 / 88.9 at 24, 91.1 / 89.9 at 32, 97.6 / 93.2 at 48, 105.8 / 100.4 at 64, 220 / 181 at 300,
-// 546 / 417 at 1000.
+// The same sums in another order, all in fp32: a call of 32 tokens and more equals calls
+// of its parts to fp32 rounding.  From 32 tokens on (us per call, token by token / chunks,
+// H_v = 32): 81.4 / 83.1 at T = 16, 84.9 / 85.4 at 24, 87.2 / 86.2 at 31; H_v = 16: 74.2 /
+// 75.2, 76.8 / 76.7, 78.9 / 77.1.
 constexpr int GCHUNK_MIN = 32;
 constexpr int GCK = 16;              // tokens per chunk
 constexpr int GCK_P = 256, GCK_E = 512, GCK_E2 = 528, GCK_B = 544;   // record: T, P / sqrt(S), E_b, E_{a,16}, beta
 constexpr int GCK_REC = 576;         // floats per record (chunk, value head), in the y rows, written only later
-static_assert(GCHUNK_MIN - 1 <= GTB, "the four-token form stages one block of tokens");
+static_assert(GCHUNK_MIN - 1 <= GTB, "the token-by-token form stages one block of tokens");
 static_assert(GCHUNK_MIN >= GCK && 2 * GCK_REC <= (GCK + 1) * GS, "the records of ceil(T / 16) chunks fit T rows of y");
 
 __device__ __forceinline__ fx4 mfma_f32(float x, float y, fx4 c) {   // D[16][16] += A[16][4] B[4][16]

@@ -49,6 +49,22 @@ def test_chunks(orc, H_k, H_v, types, T):
     assert rel(gss, ss) < STATE_TOL
 
 
+@pytest.mark.parametrize("types", [(Q4_K, Q6_K, Q8_0, Q8_0, Q4_K), (Q8_0,) * 5])
+@pytest.mark.parametrize("parts", [(1,) * 9, (1, 3, 8, 19), (4, 27), (7, 8, 9), (2, 29)])
+def test_parts_give_the_same_bits(orc, types, parts):
+    """Calls of fewer than 32 tokens: outputs and states bit for bit those of any parts."""
+    T = sum(parts)
+    gw = GdnWeights(512, 128, 2, 4, 4, types, 11, orc)
+    h = np.random.default_rng(T).standard_normal((T, 512)).astype(np.float32)
+    cs, ss = gw.fresh_state(np.random.default_rng(5))
+    whole, split = GpuGdn(gw, cs, ss), GpuGdn(gw, cs, ss)
+    want = whole.run(h)
+    got = [split.run(p) for p in np.split(h, np.cumsum(parts)[:-1])]
+    for i in range(2):
+        assert np.array_equal(np.concatenate([g[i] for g in got]), want[i])
+        assert np.array_equal(split.states()[i], whole.states()[i])
+
+
 @pytest.mark.parametrize("T,p", [(40, 21), (32, 9), (37, 36)])
 def test_overflow_stays_with_its_token(orc, T, p):
     """Value channel 3 of head 1: its projection reads only columns that are zero before
