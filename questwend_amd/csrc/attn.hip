@@ -117,13 +117,15 @@ __global__ void __launch_bounds__(256) k_attn_qk_rope(AttnArgs a, int hpb) {
 // stored transposed, four keys of a dim as one 8-byte store at quad position
 // q ^ (dim / 2 % 16).
 //
-// The exponent is the hardware's exp2 of (score - maximum) / sqrt(D) * log2 e: its
-// error (~1e-6 of p) moves a probability across an f16 step in about one of 500.
+// The probabilities are ggml's: ggml_v_expf of score / sqrt(D) less the row's maximum,
+// times 1 / S, S in double over the splits (k_attn_stat).
 //
 // Bound: latency and VALU (the exponentials), not memory or matrix cores.  30B
 // heads, T = 512 behind 1037 keys: 233 us (16-row tiles of v_mfma_f32_16x16x16_f16 and
-// one workgroup per CU) -> 52 us for the three; T = 1 at 3000 keys: 34.1 us
-// (dot products on the VALU, scores through memory) -> 19.1 us.
+// one workgroup per CU) -> 61 us for the three (15.7, 36.0, 9.4; 52 with the hardware's
+// exp2 of a fused product for ggml_v_expf, which moved one probability in 500 by an f16
+// step); T = 1 at 3000 keys: 34.1 us (dot products on the VALU, scores through memory) ->
+// 18.8 us (5.0, 9.4, 4.4).
 constexpr int FK = 64;   // keys per chunk
 
 // What both kernels know of a wave's rows and its workgroup's keys.
@@ -133,6 +135,7 @@ struct AttnTile {
     int nkeys;         // keys of the split some row of the workgroup sees (<= 0: none)
     int vis;           // this lane's row: the last key it sees, relative to k0 (rows past the end: -1)
     int vis_all;       // keys up to here are visible to every row of the workgroup
+    int wrows;         // rows of this wave (<= 0: none)
     bool row_ok;
 };
 template <int NW>
@@ -141,6 +144,7 @@ __device__ __forceinline__ AttnTile attn_tile(const AttnArgs& a, int w, int li, 
     const int64_t rows = (int64_t) a.T * R, row0 = (int64_t) blockIdx.y * (32 * NW), r = row0 + 32 * w + li;
     AttnTile x;
     x.row_ok = r < rows;
+    x.wrows = (int) min(rows - row0 - 32 * w, (int64_t) 32);
     const int t = x.row_ok ? (int) (r / R) : 0, hd = x.row_ok ? g * R + (int) (r % R) : 0;
     x.row_id = (int64_t) t * nq + hd;
     const int t_last = (int) ((min(rows, row0 + 32 * NW) - 1) / R);
@@ -204,62 +208,91 @@ __device__ __forceinline__ f16v attn_scores(const uint8_t* sk, int kk, int li, i
     return s;
 }
 
-constexpr float LOG2E = 1.4426950408889634f;
+// v_expf for -80 <= x <= 0, its bits without its branches.  Scores further below the
+// maximum are raised to -80: 0 as an f16 probability, and nothing beside a double sum
+// of at least 1.
+__device__ __forceinline__ float exp_score(float x) {
+    const float z = __builtin_fmaf(x, 0x1.715476p+0f, 0x1.8p23f);
+    const float n = z - 0x1.8p23f;
+    const float b = __builtin_fmaf(-n, 0x1.7f7d1cp-20f, __builtin_fmaf(-n, 0x1.62e4p-1f, x));
+    const float k = bitsf((fbits(z) << 23) + 0x3f800000u);
+    const float u = b * b;
+    const float j = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(0x1.0e4020p-7f, b, 0x1.573e2ep-5f), u,
+                                                  __builtin_fmaf(0x1.555e66p-3f, b, 0x1.fffdb6p-2f)),
+                                   u, 0x1.ffffecp-1f * b);
+    return __builtin_fmaf(k, j, k);
+}
 
-// Per row and split of a.split keys: the maximum (in log2 units) and sum of
-// exponentials, -inf and 0 where the row sees none of its keys.
+// Per row and split of a.split keys: the maximum of its scores and, in double, the sum
+// of exponentials (stored as a float); a maximum of -inf where the row sees none of its keys.
+// Up to 64 rows (decode, verify) the exponentials are ggml_v_expf's, each added in
+// double; more rows form them with the hardware's exp and add sixteen in fp32 first
+// (they only normalize: S moves by ~1e-7 of itself, far below the f16 step of p).
 template <int NW>
 __global__ void __launch_bounds__(64 * NW) k_attn_stat(AttnArgs a) {
+    constexpr bool EXACT = NW <= 2;
     __shared__ __align__(16) uint8_t s_k[2][FK * 2 * AD];
     const int l = threadIdx.x & 63, li = l & 31, h = l >> 5;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const AttnTile x = attn_tile<NW>(a, w, li, (int64_t) blockIdx.z * a.split, a.split);
     float* stat = a.stat + 2 * ((int64_t) blockIdx.z * a.T * a.n_head + x.row_id);
-    float m = -INFINITY, lsum = 0.0f;   // over this lane's keys
+    float m = -INFINITY;   // the row's maximum so far (both lanes that hold it)
+    double lsum = 0.0;     // over this lane's keys
     if (x.nkeys > 0) {
         h8 qb[8];
         attn_load_q(a, x, h, qb);
         AttnKCopy<NW> kc;
         kc.init(a, x, w, l);
-        const float sc2 = a.kq_scale * LOG2E;
         kc.issue(s_k[0], 0);
         int buf = 0;
         for (int c0 = 0; c0 < x.nkeys; c0 += FK) {
             vm_wait<0>();
             lds_barrier();   // this chunk's copies are there; the other buffer's readers are done
             if (c0 + FK < x.nkeys) kc.issue(s_k[buf ^ 1], c0 + FK);
+            f16v s[2];
+            float mc = -INFINITY;
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
-                f16v s = attn_scores(s_k[buf], kk, li, h, qb);
+                s[kk] = attn_scores(s_k[buf], kk, li, h, qb);
+#pragma unroll
+                for (int i = 0; i < 16 && EXACT; ++i) s[kk][i] *= a.kq_scale;
                 if (c0 + FK - 1 > x.vis_all) {   // uniform
 #pragma unroll
                     for (int i = 0; i < 16; ++i)
-                        s[i] = c0 + 32 * kk + 8 * (i >> 2) + 4 * h + (i & 3) <= x.vis ? s[i] : -INFINITY;
+                        s[kk][i] = c0 + 32 * kk + 8 * (i >> 2) + 4 * h + (i & 3) <= x.vis ? s[kk][i] : -INFINITY;
                 }
-                float mc = s[0];
 #pragma unroll
-                for (int i = 1; i < 16; ++i) mc = fmaxf(mc, s[i]);
-                const float mn = fmaxf(m, mc * sc2);
-                const float mu = mn == -INFINITY ? 0.0f : mn;   // (no key yet: every exponential is 0)
-                lsum *= __builtin_amdgcn_exp2f(m - mu);
-                m = mn;
-                float e0 = 0.0f, e1 = 0.0f;
+                for (int i = 0; i < 16; ++i) mc = fmaxf(mc, s[kk][i]);
+            }
+            if constexpr (!EXACT) mc *= a.kq_scale;
+            mc = fmaxf(mc, __shfl_xor(mc, 32));   // (lane l ^ 32 holds the row's other keys)
+            const float mn = fmaxf(m, mc), mu = mn == -INFINITY ? 0.0f : mn;   // (no key yet: every exponential is 0)
+            if (__any(mn > m && m != -INFINITY))
+                lsum *= m == -INFINITY ? 0.0 : EXACT ? exp((double) m - (double) mn) : (double) __expf(m - mn);
+            m = mn;
 #pragma unroll
-                for (int i = 0; i < 16; i += 2) {
-                    e0 += __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sc2, -mu));
-                    e1 += __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], sc2, -mu));
+            for (int kk = 0; kk < 2; ++kk) {
+                if constexpr (EXACT) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const float d = s[kk][i] - mu;
+                        lsum += (double) exp_score(d < -80.0f ? -80.0f : d);   // (a NaN stays)
+                    }
+                } else {
+                    float e0 = 0.0f, e1 = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 16; i += 2) {
+                        e0 += __expf(__builtin_fmaf(s[kk][i], a.kq_scale, -mu));
+                        e1 += __expf(__builtin_fmaf(s[kk][i + 1], a.kq_scale, -mu));
+                    }
+                    lsum += (double) (e0 + e1);
                 }
-                lsum += e0 + e1;
             }
             buf ^= 1;
         }
-        // lane l ^ 32 holds the row's other keys
-        const float mo = __shfl_xor(m, 32), lo = __shfl_xor(lsum, 32);
-        const float mn = fmaxf(m, mo), mu = mn == -INFINITY ? 0.0f : mn;
-        lsum = lsum * __builtin_amdgcn_exp2f(m - mu) + lo * __builtin_amdgcn_exp2f(mo - mu);
-        m = mn;
+        lsum += __shfl_xor(lsum, 32);
     }
-    if (x.row_ok && h == 0) *(float2*) stat = float2{m, lsum};
+    if (x.row_ok && h == 0) *(float2*) stat = float2{m, (float) lsum};
 }
 
 // P.V sums over a PV split (merge statistics splits of a.split keys each).
@@ -315,22 +348,28 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
         load_v(0);
         h8 qb[8];
         attn_load_q(a, x, h, qb);
-        // the row's maximum M and 1 / S, S = sum_s exp2(m_s - M) l_s (in double), over
-        // the splits (lane half h those of its parity)
+        // each row's maximum M and 1 / S, S = sum_s exp(m_s - M) l_s in double over the
+        // splits: 64 / p2 lanes per row, p2 the power of two that holds the wave's rows
+        int p2 = 32;
+        while (p2 / 2 >= x.wrows && p2 > 1) p2 /= 2;   // uniform
+        const int mine = l & (p2 - 1);
+        const int64_t rid = __shfl(x.row_id, mine);
+        const float2* st = (const float2*) a.stat + rid;
         float M = -INFINITY;
-        const float2* st = (const float2*) a.stat + x.row_id;
 #pragma unroll 4
-        for (int s = h; s < n_split; s += 2) M = fmaxf(M, st[s * heads].x);
-        M = fmaxf(M, __shfl_xor(M, 32));
+        for (int s = l / p2; s < n_split; s += 64 / p2) M = fmaxf(M, st[s * heads].x);
+        for (int off = p2; off < 64; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
         double S = 0.0;
-#pragma unroll 4
-        for (int s = h; s < n_split; s += 2) {
+#pragma unroll 1
+        for (int s = l / p2; s < n_split; s += 64 / p2) {
             const float2 v = st[s * heads];
-            S += (double) __builtin_amdgcn_exp2f(v.x - M) * (double) v.y;
+            if (v.x != -INFINITY) S += exp((double) v.x - (double) M) * (double) v.y;
         }
-        S += __shfl_xor(S, 32);
-        const float inv = x.row_ok ? (float) (1.0 / S) : 0.0f;
-        const float sc2 = a.kq_scale * LOG2E;
+        for (int off = p2; off < 64; off <<= 1) S += __shfl_xor(S, off);
+        // (every score -inf: probabilities 0)
+        const float inv1 = __shfl(S == 0.0 ? 0.0f : (float) (1.0 / S), li & (p2 - 1));
+        M = __shfl(M == -INFINITY ? 0.0f : M, li & (p2 - 1));
+        const float inv = x.row_ok ? inv1 : 0.0f;
         int buf = 0;
         for (int c0 = 0; c0 < x.nkeys; c0 += FK) {
             vm_wait<0>();      // this chunk's K copies and V rows
@@ -345,7 +384,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW
             for (int kk = 0; kk < 2; ++kk) {
                 f16v s = attn_scores(s_k[buf], kk, li, h, qb);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sc2, -M)) * inv;
+                for (int i = 0; i < 16; ++i) 
+                    s[i] = exp_score(fmaxf(s[i] * a.kq_scale - M, -80.0f)) * inv;   // (a NaN: inv is one too)
                 if (c0 + FK - 1 > x.vis_all) {   // uniform
 #pragma unroll
                     for (int i = 0; i < 16; ++i)

@@ -190,7 +190,7 @@ struct AttnArgs {
     int64_t split;                // keys per split of the statistics (attn_split)
     int merge;                    // statistics splits per PV split
     float* part;                  // [PV splits][T][n_head][128] each PV split's sums
-    float* stat;                  // [splits][T][n_head][2] each split's maximum (log2 units) and sum
+    float* stat;                  // [splits][T][n_head][2] each split's maximum and sum of exponentials
     float* att;                   // [T][n_head * 128] (without att_q8K; may be part when there is one split)
     void* att_q8K;                // optional: Q8_K rows of att, written in its place (n_head * 128 a multiple of 256)
     uint16_t* att_h;              // optional, with att_q8K: its f16 copy (launch_q8K_to_f16's layout)

@@ -68,6 +68,37 @@ def test_attention_odd_heads(orc, T, n_past):
     attn_case(orc, (3, 1), (Q8_0,) * 4, T, n_past)
 
 
+@pytest.mark.parametrize("T", [4096, 4])
+def test_attention_long_sum(orc, T):
+    """The softmax's sum over 100 k keys of which one holds nearly everything: each of the
+    others adds 0.9 * 2^-28, a group of sixteen less than half a step of a 32-bit 1.0.  All
+    together they take that one's probability below 1 - 2^-12, the middle between the f16s 1
+    and 1 - 2^-11; with those beside the largest key lost, it is above.  T = 4096: one split
+    over all keys.  The query turns with its position in a pair of dims that the rotary
+    base leaves still, so every row has the same result: that of the CPU restatement, whose
+    sum is in double, within 1e-5 (a step of p is 5e-4)."""
+    n = 100096
+    aw = AttnWeights(512, 16, 1, 128, (Q4_K, Q4_K, Q8_0, Q4_K), seed=3, oracle=orc, freq_base=1e38)
+    aw.wq = np.ascontiguousarray(np.tile(aw.wq.reshape(16, -1)[:1], (16, 1)).reshape(-1))   # every head the same query
+    aw.k_norm[:] = 0.0                                                                      # new keys: score 0
+    keep = aw.q_norm[[63, 127]].copy()
+    aw.q_norm[:] = 0.0
+    aw.q_norm[[63, 127]] = 10.0 * keep
+    h = np.random.default_rng(8).standard_normal((1, 512)).astype(np.float32)
+    kc, vc = np.zeros((n, 128), np.uint16), np.zeros((n, 128), np.uint16)
+    q = attn_seg_restated(aw, h, 1, kc[:2].copy(), vc[:2].copy(), orc)[2][0, :128].astype(np.float16).astype(np.float64)
+    s = 28.0 * np.log(2.0) - np.log(0.9)
+    kc[0] = (q * (s * np.sqrt(128.0) / (q @ q))).astype(np.float16).view(np.uint16)
+    vc[0] = np.random.default_rng(9).standard_normal(128).astype(np.float16).view(np.uint16)
+    g = GpuAttn(aw, n, kc, vc)
+    res, _ = ops.attn_seg(g.layer, dev(np.repeat(h, T, 0)), n - T)
+    want, _, _, att = attn_seg_restated(aw, h, n - 1, kc.copy(), vc.copy(), orc)
+    v0 = vc[0].view(np.float16).astype(np.float32)
+    assert np.allclose(att.reshape(16, 128), (1.0 - 2.0 ** -11) * v0, rtol=1e-6, atol=0)   # (p is where it should be)
+    got = res.cpu().numpy() - h
+    assert rel(got, np.repeat(want - h, T, 0)) < 1e-5
+
+
 def gdn_case(orc, H_k, H_v, d_conv, types, T):
     gw = GdnWeights(512, 128, H_k, H_v, d_conv, types, 7 + T, orc)
     h = np.random.default_rng(T).standard_normal((T, 512)).astype(np.float32)
