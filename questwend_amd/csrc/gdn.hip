@@ -527,13 +527,13 @@ __global__ void __launch_bounds__(256) k_gdn_gate_norm_q8K(GdnArgs a) {
     if (blk >= nblk) return;
     const int64_t e = blk * 256 + 4 * lane;
     const float4 x = *(const float4*) (a.o + e), z = *(const float4*) (a.z + e);
-    const float4 nw = *(const float4*) (a.ssm_norm + 4 * (lane & 31));
+    const float* nw = a.ssm_norm + 4 * (lane & 31);   // (the caller's: any alignment)
     double s = ((double) (x.x * x.x) + (double) (x.y * x.y)) + ((double) (x.z * x.z) + (double) (x.w * x.w));
     for (int off = 16; off >= 1; off >>= 1) s += __shfl_xor(s, off);   // the head's 32 lanes
     const float mean = (float) (s / (double) GS);
     const float sc = 1.0f / sqrtf(mean + a.eps);
-    const float v[4] = {((x.x * sc) * nw.x) * v_silu(z.x), ((x.y * sc) * nw.y) * v_silu(z.y),
-                        ((x.z * sc) * nw.z) * v_silu(z.z), ((x.w * sc) * nw.w) * v_silu(z.w)};
+    const float v[4] = {((x.x * sc) * nw[0]) * v_silu(z.x), ((x.y * sc) * nw[1]) * v_silu(z.y),
+                        ((x.z * sc) * nw[2]) * v_silu(z.z), ((x.w * sc) * nw[3]) * v_silu(z.w)};
     _Float16* h = (_Float16*) a.y_h;
     quant_q8K_wave(v, lane, (BlockQ8_K*) a.y_q8K + blk, h ? h + (size_t) blk * QK_K : nullptr,
                    h ? h + (size_t) nblk * QK_K + (size_t) blk * 16 : nullptr);

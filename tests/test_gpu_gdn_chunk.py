@@ -65,6 +65,20 @@ def test_parts_give_the_same_bits(orc, types, parts):
         assert np.array_equal(split.states()[i], whole.states()[i])
 
 
+def test_ssm_norm_at_any_address(orc):
+    gw = GdnWeights(512, 128, 2, 4, 4, (Q4_K, Q6_K, Q8_0, Q8_0, Q4_K), 12, orc)
+    h = np.random.default_rng(1).standard_normal((5, 512)).astype(np.float32)
+    cs, ss = gw.fresh_state(np.random.default_rng(5))
+    want = GpuGdn(gw, cs, ss).run(h)
+    g = GpuGdn(gw, cs, ss)
+    off = torch.zeros(131, dtype=torch.float32, device="cuda:0")
+    off[3:] = g.t[9]
+    g.t[9] = off
+    g.layer.ssm_norm = off.data_ptr() + 12
+    got = g.run(h)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("T,p", [(40, 21), (32, 9), (37, 36)])
 def test_overflow_stays_with_its_token(orc, T, p):
     """Value channel 3 of head 1: its projection reads only columns that are zero before
