@@ -142,8 +142,23 @@ bool mfma_f16_reserve(Arena& ar, qw::MmidArgs& m, int64_t n_rows) {
     return h != nullptr;
 }
 
-// The same, and the copy made from the quantized rows by a launch of its own.
+// Whether the batch holds half_pairs / 2 routed rows per bin.
+bool mfma_dense(const qw::MmidArgs& m, int half_pairs) {
+    return 2 * m.n_pairs >= half_pairs * (m.slot_of ? m.n_slot_of : m.n_as);
+}
+// Half pairs per bin from which the matrix cores take every bin (mfma_bins).
+int mfma_all_line(const qw::MmidArgs& m) { return m.type == qw::T_Q6_K ? 8 : 1; }
+
+// The same, and the copy made from the quantized rows by a launch of its own (about
+// 2 us; mul_mat_id).  For Q8_0 and Q6_K only where every bin then goes to the matrix
+// cores, which read it, and gains by more than the launch: Q6_K at its line, Q8_0 at
+// 1.5 pairs per bin (us, GEMV / copy and matrix cores: K = 768, N = 2048, 128 experts 43.5 /
+// 45.3 at 1 pair per bin, 57.2 / 54.0 at 1.5; K = 1024, N = 512, 64 experts 19.4 / 21.6,
+// 24.1 / 21.7).  A sparser call's bins are the GEMV's (Q6_K's heavy ones the int8 kernel's).
 int mfma_f16_prep(Arena& ar, qw::MmidArgs& m, int64_t n_rows, hipStream_t st) {
+    if (m.type != qw::T_Q4_K && (!qw::mmid_mfma_h_read(m) ||
+                                 (m.mfma_min_rows != 1 && !mfma_dense(m, m.type == qw::T_Q6_K ? mfma_all_line(m) : 3))))
+        return 0;
     if (!mfma_f16_reserve(ar, m, n_rows)) return 0;
     const int rc = m.type == qw::T_Q8_0
                        ? qw::launch_q80_to_f16(m.act_q, m.K, n_rows, (uint16_t*) m.act_h, (float*) m.act_hd, st)
@@ -186,11 +201,7 @@ qw::MmidArgs mfma_bins(const qw::MmidArgs& m) {
     qw::MmidArgs c = m;
     if (c.type == qw::T_Q8_0 && !c.act_h) c.mfma_min_rows = 0;
     if (c.mfma_min_rows <= 1) return c;
-    const int64_t bins = c.slot_of ? c.n_slot_of : c.n_as;
-    const bool all = c.type == qw::T_Q8_0 ? 2 * c.n_pairs >= bins
-                                          : c.mfma_exact && (c.type == qw::T_Q6_K ? c.act_h && c.n_pairs >= 4 * bins
-                                                                                  : c.act_h && 2 * c.n_pairs >= bins);
-    if (all) c.mfma_min_rows = 1;
+    if (c.act_h && mfma_dense(c, mfma_all_line(c))) c.mfma_min_rows = 1;   // (a K-quant has the copy in the exact form only)
     return c;
 }
 

@@ -1681,6 +1681,10 @@ bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows) {
            (uint64_t) n_rows * (uint64_t) m.K * 2u + 512u < (1ull << 31);
 }
 
+bool mmid_mfma_h_read(const MmidArgs& m) {
+    return m.type != T_Q6_K || (m.K >= 3 * QK_K && m.max_active <= MP_MAXG && m.b_ne1 <= 65535);
+}
+
 // Whether the persistent f16 kernel takes the launch: the exact form with the f16
 // copy, at least three super-blocks per row, at most MP_MAXG active bins, and for
 // two matrices one grouping and one activation buffer.  QWMOE_MFMA_PERSIST=0 in

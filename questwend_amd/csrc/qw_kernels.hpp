@@ -120,6 +120,8 @@ int launch_mmid_mfma2(const MmidArgs& a, const MmidArgs& b, hipStream_t stream);
 int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t n_rows, uint16_t* out, hipStream_t stream);
 // whether m (with act_q holding n_rows rows) can take such a copy as act_h
 bool mmid_mfma_h_ok(const MmidArgs& m, int64_t n_rows);
+// whether the matrix-core kernel that takes m's bins reads the copy (Q6_K's int8 kernel does not)
+bool mmid_mfma_h_read(const MmidArgs& m);
 
 // The f16 copy the Q8_0 matrix-core form reads, of n_rows dense Q8_0 rows of K
 // values: per 32-value block four 16-byte chunks, chunk c the quants of elements

@@ -3,7 +3,8 @@ and the row-copying GEMV, bit for bit against the CPU oracle, at the edges of
 their tiles: one row and full / partial 16-row items, weight rows that do
 not fill a 16-row workgroup, the smallest and larger row lengths, each activation
 row of a pass (1 to 4), the weights' extreme quants (-128), a workspace without
-room for the f16 copy, and the SwiGLU launch that writes Q8_0 rows directly."""
+room for the f16 copy, a batch too sparse for it, and the SwiGLU launch that writes Q8_0
+rows directly."""
 from __future__ import annotations
 
 import numpy as np
@@ -12,8 +13,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
-from questwend_amd import ops  # noqa: E402
-from oracle_lib import LayerWeights, Oracle, Q8_0  # noqa: E402
+from questwend_amd import lib, ops  # noqa: E402
+from oracle_lib import LayerWeights, Oracle, Q6_K, Q8_0, row_size, vec_dot_type  # noqa: E402
 from test_gpu_decode import GpuLayer  # noqa: E402
 from test_gpu_parity import bits, dev, host  # noqa: E402
 
@@ -63,6 +64,24 @@ def test_no_room_for_the_copy(orc):
     """The allocation-free call's 8 MiB hold the Q8_0 rows but not their f16 copy: the GEMV, the same bits."""
     run, want = counts_case(orc, 2048, 64, [900, 900], 1, seed=3)
     assert np.array_equal(bits(run(noalloc=True)), bits(want))
+
+
+@pytest.mark.parametrize("t", [Q6_K, Q8_0])
+def test_no_copy_that_nothing_reads(orc, t):
+    """64 tokens, two of 512 experts each: the GEMV takes the bins, so the call's workspace holds the
+    quantized rows and the grouping (under 100 KB) and no f16 copy of the rows (278 KB), nor is there a launch for it."""
+    K, N, T, E = 2048, 64, 64, 512
+    w = torch.zeros((E * N, row_size(t, K)), dtype=torch.uint8, device="cuda:0")
+    b = torch.zeros((T, 1, K), dtype=torch.float32, device="cuda:0")
+    ids = torch.arange(2 * T, dtype=torch.int32, device="cuda:0").view(T, 2)
+    ops.shutdown()
+    try:
+        ops.init(0, 64 << 20)
+        ops.mul_mat_id(t, w, K, N, E, b, ids)
+        torch.cuda.synchronize()
+        assert lib().qwmoe_workspace_high_water() < T * row_size(vec_dot_type(t), K) + 100_000
+    finally:
+        ops.init(0, 512 << 20)
 
 
 @pytest.mark.parametrize("K", [256, 768, 2048, 4096, 64, 1088])
