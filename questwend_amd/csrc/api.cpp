@@ -147,7 +147,7 @@ bool mfma_dense(const qw::MmidArgs& m, int half_pairs) {
     return 2 * m.n_pairs >= half_pairs * (m.slot_of ? m.n_slot_of : m.n_as);
 }
 // Half pairs per bin from which the matrix cores take every bin (mfma_bins).
-int mfma_all_line(const qw::MmidArgs& m) { return m.type == qw::T_Q6_K ? 8 : 1; }
+int mfma_all_line(const qw::MmidArgs& m) { return m.type == qw::T_Q6_K ? 6 : 1; }
 
 // The same, and the copy made from the quantized rows by a launch of its own (about
 // 2 us; mul_mat_id).  For Q8_0 and Q6_K only where every bin then goes to the matrix
@@ -187,16 +187,19 @@ int mfma_f16_prep_pair(Arena& ar, qw::MmidArgs& mu, qw::MmidArgs& mg, int64_t n_
 //  - Where every form gives ggml's bits (all but the block sums), a batch dense
 //    enough sends its light bins there too, in one launch in place of two: a
 //    16-row tile costs about what reading its weights does, the GEMV a pass per
-//    few rows.  The line is half a pair per bin (128 experts, 8 per token, us per
-//    layer, light bins on the GEMV / everything on the matrix cores): Q4_K at the 30B
-//    shape 43.9 / 35.4 at T = 8 (512 x 256 experts), 86.0 / 85.5 at T = 10 (55.4 / 50.6 with
-//    every token routed alike), 119.5 / 113.4 at T = 16, 181.6 / 146.1 at T = 33,
-//    312.5 / 267.4 at T = 512; Q8_0 69.1 / 66.2 at T = 4, 82.3 / 82.4 at T = 6, 86.1 /
-//    86.4 at T = 7 (64 experts, 4 per token: 33.6 / 36.5 at T = 6, 35.5 / 37.3 at T = 7).
-//    Q6_K forms more integers per tile: 109.6 / 125.8 at T = 10,
-//    142.0 / 157.6 at T = 16, 214.5 / 203.9 at T = 33, 230.7 / 205.3 at T = 64 (4 pairs
-//    per bin), but as the down projection at H = 4096 459.7 / 510.6 at T = 33,
-//    490.8 / 508.1 at T = 64, 539.5 / 551.2 at T = 128.
+//    few rows.  The line is half a pair per bin, three for Q6_K, which forms more
+//    integers per tile (us per layer, light bins on the GEMV / everything on the
+//    matrix cores; experts drawn evenly):
+//      pairs per bin                 0.5            1             2             3             16
+//      Q4_K  30B shape          69.8 / 63.5  114.4 / 91.3  181.3 / 121   223.8 / 129   178.8 / 169
+//            64 experts, top 4  37.7 / 31.4   44.9 / 36.0   66.7 / 53.5   70.1 / 53.9   95.9 / 62.4
+//      Q8_0  30B shape         101.7 / 92.4  161.8 / 146   238.7 / 182   296.0 / 192   273.0 / 261
+//            64 experts, top 4  42.0 / 37.5   51.8 / 44.9   69.1 / 61.5   78.2 / 62.4   96.4 / 71.5
+//      Q6_K  30B shape          88.3 / 90.8  142.0 / 145   209.7 / 178   253.4 / 193   258.3 / 247
+//            64 experts, top 4  38.0 / 40.8   46.2 / 48.7   67.5 / 70.1   72.9 / 70.4  109.7 / 81.4
+//            one mul_mat_id, K = 1536, N = 4096, 128 experts, with its copy's launch
+//                               72.3 / 91.0  117.5 / 133   178.3 / 187   233.0 / 211   354.9 / 273
+//    (a Zipf-skewed batch gains more: Q6_K, 64 experts, 80.2 / 60.7 at 2).
 qw::MmidArgs mfma_bins(const qw::MmidArgs& m) {
     qw::MmidArgs c = m;
     if (c.type == qw::T_Q8_0 && !c.act_h) c.mfma_min_rows = 0;
