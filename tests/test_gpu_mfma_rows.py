@@ -3,8 +3,9 @@ of the whole range -- every quant, every 6-bit or int8 scale, extreme activation
 -- bit for bit against the CPU oracle: Q4_K and Q6_K, row lengths whose Q6_K rows
 start on and off a dword, one- and two-tile items of every remainder, launches small
 enough for 16-row items and large enough for 32-row ones, light bins in more 16-row
-units than workgroups, all bins on the matrix
-cores and only those of eight rows or more."""
+units than workgroups.  The dense cases send every bin to the matrix cores whatever
+the row threshold; the sparse ones at the end split the bins between the GEMV and the
+matrix cores (mul_mat_id, and whole layers, whose quantizing launches write the f16 copy)."""
 from __future__ import annotations
 
 import numpy as np
@@ -14,8 +15,8 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 from questwend_amd import ops  # noqa: E402
-from oracle_lib import Oracle, Q4_K, Q6_K  # noqa: E402
-from test_gpu_parity import bits, dev, host  # noqa: E402
+from oracle_lib import LayerWeights, Oracle, Q4_K, Q6_K, Q8_0  # noqa: E402
+from test_gpu_parity import _layer_gpu, bits, dev, host  # noqa: E402
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -86,3 +87,64 @@ def test_light_bins(orc, t, min_rows, per_bin):
     finally:
         ops.set_mfma_min_rows(prev)
     assert np.array_equal(bits(got), bits(orc.mul_mat_id(t, K, N, n_as, w, b, ids)))
+
+
+SPARSE = [9, 17, 33, 8, 1, 2, 3, 4, 5, 6, 7]   # 95 rows: four bins for the matrix cores, the rest the GEMV's
+
+
+# bins: more than the rows' density asks for, so that the light ones stay on the GEMV
+@pytest.mark.parametrize("t,n_as", [(Q4_K, 200), (Q4_K, 256), (Q6_K, 32), (Q6_K, 200), (Q8_0, 64), (Q8_0, 200)])
+@pytest.mark.parametrize("K,N", [(768, 64), (2048, 128)])
+def test_sparse_bins(orc, t, n_as, K, N):
+    rng = np.random.default_rng(K + n_as)
+    counts = np.zeros(n_as, np.int64)
+    counts[rng.permutation(n_as)[:len(SPARSE)]] = SPARSE
+    if t == Q8_0:
+        w = orc.quantize(t, (rng.standard_normal((n_as * N, K)) * 0.02).astype(np.float32))
+    else:
+        w = raw_blocks(rng, t, n_as * N, K)
+    ids = rng.permutation(np.repeat(np.arange(n_as), counts)).astype(np.int32).reshape(-1, 1)
+    b = rng.standard_normal((ids.shape[0], 1, K)).astype(np.float32)
+    prev = ops.set_mfma_min_rows(8)
+    try:
+        got = host(ops.mul_mat_id(t, dev(w), K, N, n_as, dev(b), dev(ids)))
+    finally:
+        ops.set_mfma_min_rows(prev)
+    assert np.array_equal(bits(got), bits(orc.mul_mat_id(t, K, N, n_as, w, b, ids)))
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("permute", [False, True])
+def test_sparse_layer(orc, t, permute):
+    """36 tokens over 80 experts, one each: 17 on expert 3, 9 on expert 9, the rest as the router has it."""
+    H = F = 768
+    E, T = 80, 36
+    rng = np.random.default_rng(4)
+    lw = LayerWeights.__new__(LayerWeights)
+    lw.H, lw.E, lw.k, lw.F, lw.n_slots = H, E, 1, F, E
+    lw.type_gate = lw.type_up = lw.type_down = t
+    lw.slot_of = tuple(rng.permutation(E).astype(np.int32) for _ in range(3)) if permute else None
+    def raw():
+        if t != Q8_0:
+            return raw_blocks(rng, t, E * H, F)
+        w = rng.integers(0, 256, (E * H * F // 32, 34)).astype(np.uint8)
+        w[:, :2] = (rng.standard_normal((w.shape[0], 1)) * 1e-3).astype(np.float16).view(np.uint8)
+        return w.reshape(-1)
+    lw.gate, lw.up, lw.down = raw(), raw(), raw()
+    lw.router = (rng.standard_normal((E, H)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((T, H)).astype(np.float32)
+    x[:, :2] = 0.0
+    x[:17, 0] = x[17:26, 1] = 3.0
+    lw.router[3, 0] = lw.router[9, 1] = 20.0
+    prev, form = ops.set_mfma_min_rows(8), ops.set_mfma_form(ops.MFMA_EXACT)
+    try:
+        L, keep, _ = _layer_gpu(lw)
+        out, xn, ids, w = ops.ffn_layer(L, dev(x), 1e-6)
+        out, ids = host(out), host(ids)
+    finally:
+        ops.set_mfma_min_rows(prev)
+        ops.set_mfma_form(form)
+    r = orc.moe_layer(lw, x, rms_eps=1e-6)
+    n = np.bincount(ids.reshape(-1), minlength=E)
+    assert n[3] >= 17 and n[9] >= 9 and (n > 0).sum() > 6 and np.sort(n)[-3] < 8
+    assert np.array_equal(ids, r["ids"]) and np.array_equal(bits(out), bits(r["out"]))
