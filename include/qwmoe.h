@@ -338,12 +338,16 @@ typedef struct qwmoe_attn_layer {
  * rounded to f16 before their products as ggml's f16 mul_mat does.  Outputs
  * agree with the reference CPU graph within the fp32 rounding of the sums
  * (1e-3), not bit for bit.  Requires D = n_rot = 128, n_head / n_head_kv <= 16,
- * n_past + T <= n_ctx, h 16-byte aligned.  Workspace: ~40 T n_embd bytes of
- * projections, plus, for batches of fewer than 64 query rows per kv head
- * (T n_head / n_head_kv < 64: decode, verify), the score rows (4 n_head T
- * (n_past + T) bytes); larger chunks keep only per-512-key softmax statistics
- * and recompute the scores beside P.V (QWMOE_ERR_WORKSPACE when it does not
- * fit, nothing enqueued). */
+ * n_past + T <= n_ctx, h 16-byte aligned.  Workspace, per token: 4 (n_head D +
+ * 2 n_head_kv D + H) bytes of projections (another 4 H where one of Q, K, V is
+ * Q8_0), 2 n_head D of f16 queries, the quantized rows of the two inputs, 8 n_head
+ * of softmax statistics and 4 n_head D of P.V sums per split of the keys: at least
+ * one split (QWMOE_ERR_WORKSPACE when that does not fit, nothing enqueued), and up
+ * to one per 64 keys, as many as give the launch about 512 workgroups, where the
+ * workspace holds them and 2.125 (H + n_head D) of f16 copies.  Scores are never
+ * stored.  The order of the fp32 P.V sums, and with it the last bits, follows the
+ * number of splits: equal calls in workspaces of different sizes can differ in
+ * them when the smaller one does not hold every split. */
 int qwmoe_attn_seg(void * stream, const qwmoe_attn_layer * layer, const float * h, int64_t T, int64_t n_past,
                    float rms_eps, float * attn_resid, float * ffn_in);
 

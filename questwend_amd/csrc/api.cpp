@@ -669,12 +669,15 @@ int qwmoe_attn_seg(void* stream, const qwmoe_attn_layer* L, const float* h, int6
     const bool all_q8K = vqt == qw::T_Q8_K && xk == xq && xv == xq && H % 256 == 0 && !((uintptr_t) L->attn_norm & 15);
     float* cur = all_q8K ? nullptr : ar.take<float>((size_t) (H * T));
     if (!all_q8K && !cur) return QWMOE_ERR_WORKSPACE;
-    // PV splits: as many of the statistics' splits as the workspace holds beside the
-    // f16 copies (f32 att too where the output projection reads Q8_0 and there is
-    // more than one), the others merged
-    const int64_t split = qw::attn_split(T, nq, nk, n_kv), n_split = (n_kv + split - 1) / split;
-    float* stat = ar.take<float>((size_t) (n_split * T * nq * 2));
+    // statistics splits: fewer, larger ones where their statistics leave no room for one
+    // PV split's sums.  PV splits: as many of the statistics' splits as the workspace
+    // holds beside the f16 copies (f32 att too where the output projection reads Q8_0 and
+    // there is more than one), the others merged
     const size_t per_pv = (size_t) (T * NQ * 4);
+    int64_t split = qw::attn_split(T, nq, nk, n_kv);
+    while (split < n_kv && (size_t) ((n_kv + split - 1) / split * T * nq * 8) + per_pv + 1024 > ar.left()) split *= 2;
+    const int64_t n_split = (n_kv + split - 1) / split;
+    float* stat = ar.take<float>((size_t) (n_split * T * nq * 2));
     const size_t beside = (size_t) (T * (H + NQ) * 2) + (size_t) (T * (H + NQ) / 8) + (vot == qw::T_Q8_K ? 0 : per_pv) + 8192;
     const int64_t fit = ar.left() > beside + per_pv ? (int64_t) ((ar.left() - beside) / per_pv) : 1;
     int64_t merge = (n_split + std::min(fit, n_split) - 1) / std::min(fit, n_split);

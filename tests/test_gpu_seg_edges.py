@@ -3,7 +3,8 @@
 Attention (attn.hip): query rows around 32 and 64 (one, two and four waves), chunks
 and splits of 64 keys around their ends, a first token without a past, heads per kv
 head that do not divide 32, an odd number of heads (f32 attention output), one and
-several PV splits.  Delta net (gdn.hip): tokens around the 4-token step, the 32
+several PV splits, as a small workspace has them (merged, the last group ragged), and the
+smallest workspace that a call fits.  Delta net (gdn.hip): tokens around the 4-token step, the 32
 tokens from which it takes 16 at a time and the ends of those chunks, every
 number of conv taps, an odd number of value heads, Q8_0 throughout.
 
@@ -18,13 +19,14 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
-from questwend_amd import ops  # noqa: E402
+from questwend_amd import QwmoeError, ops, row_size, vec_dot_type  # noqa: E402
 from oracle_lib import (AttnWeights, GdnWeights, Oracle, Q4_K, Q6_K, Q8_0, attn_seg_restated,  # noqa: E402
                         gdn_seg_restated)
 from test_gpu_attn import GpuAttn, dev, rel  # noqa: E402
 from test_gpu_gdn import GpuGdn  # noqa: E402
 
 TOL = 1e-3
+ERR_WORKSPACE = -4
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -97,6 +99,58 @@ def test_attention_long_sum(orc, T):
     assert np.allclose(att.reshape(16, 128), (1.0 - 2.0 ** -11) * v0, rtol=1e-6, atol=0)   # (p is where it should be)
     got = res.cpu().numpy() - h
     assert rel(got, np.repeat(want - h, T, 0)) < 1e-5
+
+
+@pytest.mark.parametrize("heads,types,T,n_past", [((8, 2), (Q4_K, Q4_K, Q6_K, Q4_K), 3, 1000), ((3, 1), (Q8_0,) * 4, 2, 700),
+                                                  ((8, 1), (Q4_K,) * 4, 32, 16082)])
+def test_attention_workspaces(orc, heads, types, T, n_past):
+    """From the smallest workspace that the call fits (which the header states) up, one PV
+    split at a time: 1, 2, 3 ... of the statistics' splits together."""
+    nq, nk = heads
+    H, NQ, NK = 512, nq * 128, nk * 128
+    aw = AttnWeights(H, nq, nk, 128, types, seed=2, oracle=orc)
+    rng = np.random.default_rng(T + n_past)
+    kc = np.full((n_past + T, NK), 0x7e00, np.uint16)
+    vc = kc.copy()
+    for c in (kc, vc):
+        c[:n_past] = (rng.standard_normal((n_past, NK)) * 0.5).astype(np.float16).view(np.uint16)
+    h = rng.standard_normal((T, H)).astype(np.float32)
+    kr, vr = kc.copy(), vc.copy()
+    want = attn_seg_restated(aw, h, n_past, kr, vr, orc)[:2]
+    hd = dev(h)
+
+    def call(size):
+        """Whether a workspace of `size` bytes takes the call; the result checked, or that nothing was written."""
+        g = GpuAttn(aw, n_past + T, kc, vc)
+        ops.shutdown()
+        ops.init(0, size)
+        try:
+            got = ops.attn_seg(g.layer, hd, n_past)
+        except QwmoeError as e:
+            assert e.status == ERR_WORKSPACE
+            torch.cuda.synchronize()
+            assert np.array_equal(g.caches()[1], vc)
+            return False
+        torch.cuda.synchronize()
+        assert rel(got[0].cpu().numpy(), want[0]) < TOL and rel(got[1].cpu().numpy(), want[1]) < TOL
+        assert np.array_equal(g.caches()[1], vr)
+        return True
+
+    per_pv = 4 * T * NQ
+    quantized = sum(row_size(vec_dot_type(t), n) for t, n in ((types[0], H), (types[3], NQ)))
+    least = T * (4 * (NQ + 2 * NK + H) + (4 * H if Q8_0 in types else 0) + 2 * NQ + quantized + 8 * nq) + per_pv
+    try:
+        lo, hi = 4096, least + 16384   # (alignment of some twenty buffers)
+        assert call(hi) and not call(lo)
+        while hi - lo > 256:
+            mid = (lo + hi) // 512 * 256
+            lo, hi = (lo, mid) if call(mid) else (mid, hi)
+        beside = 17 * T * (H + NQ) // 8 + per_pv + 8192
+        for i in range(min(18, (n_past + T) // 64 + 2) if T < 32 else 4):
+            assert call(hi + beside + i * per_pv)
+    finally:
+        ops.shutdown()
+        ops.init(0, 512 << 20)
 
 
 def gdn_case(orc, H_k, H_v, d_conv, types, T):
