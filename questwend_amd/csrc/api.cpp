@@ -154,11 +154,13 @@ int mfma_all_line(const qw::MmidArgs& m) { return m.type == qw::T_Q6_K ? 6 : 1; 
 // cores, which read it, and gains by more than the launch: Q6_K at its line, Q8_0 at
 // 1.5 pairs per bin (us, GEMV / copy and matrix cores: K = 768, N = 2048, 128 experts 43.5 /
 // 45.3 at 1 pair per bin, 57.2 / 54.0 at 1.5; K = 1024, N = 512, 64 experts 19.4 / 21.6,
-// 24.1 / 21.7).  A sparser call's bins are the GEMV's (Q6_K's heavy ones the int8 kernel's).
+// 24.1 / 21.7), or at 12 of tensors of fewer than 2^20 weights, whose GEMV is as long as
+// its launch (K = 256, N = 64, 8 experts 16.0 / 18.6 at 2, 21.2 / 19.0 at 16).  A sparser
+// call's bins are the GEMV's (Q6_K's heavy ones the int8 kernel's).
 int mfma_f16_prep(Arena& ar, qw::MmidArgs& m, int64_t n_rows, hipStream_t st) {
-    if (m.type != qw::T_Q4_K && (!qw::mmid_mfma_h_read(m) ||
-                                 (m.mfma_min_rows != 1 && !mfma_dense(m, m.type == qw::T_Q6_K ? mfma_all_line(m) : 3))))
-        return 0;
+    const int64_t weights = m.K * m.N * (m.slot_of ? m.n_slot_of : m.n_as);
+    const int line = m.type == qw::T_Q6_K ? mfma_all_line(m) : weights < (1 << 20) ? 24 : 3;
+    if (m.type != qw::T_Q4_K && (!qw::mmid_mfma_h_read(m) || (m.mfma_min_rows != 1 && !mfma_dense(m, line)))) return 0;
     if (!mfma_f16_reserve(ar, m, n_rows)) return 0;
     const int rc = m.type == qw::T_Q8_0
                        ? qw::launch_q80_to_f16(m.act_q, m.K, n_rows, (uint16_t*) m.act_h, (float*) m.act_hd, st)
