@@ -106,7 +106,7 @@ __device__ __forceinline__ void topk_token(const float* __restrict__ logits, int
     sync();
     if (probs_out)
         for (int64_t i = lane; i < E; i += 64) probs_out[t * E + i] = p[i];
-    // the order of the probabilities.  A NaN (eq == 0) goes to the sort replay:
+    // the order of the probabilities.  NaNs go to the sort replay (they fill one place only):
     // softmax makes every probability NaN then, which std::sort treats as all
     // equivalent.
     topk_order<WAVE>(p, E, k, order, sort_stack, status, lane);
