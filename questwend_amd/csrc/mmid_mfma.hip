@@ -661,8 +661,10 @@ int launch_q8K_to_f16(const uint8_t* q, size_t row_bytes, int64_t K, int64_t row
 // NT = 2: ~57 KB of LDS, 247 VGPRs, two workgroups per CU.  Needs K >= 768 (three
 // super-blocks: the next unit's pairs land before they are used) and at most
 // MP_MAXG active bins.  Bound: VALU issue (about 258 instructions per wave and
-// super-block, 96 of them ggml's own fma) with two waves per SIMD to hide each
-// other's LDS and barrier waits.  us per launch: T = 1024 at H = 4096, gate + up
+// super-block, 96 of them ggml's own fma) in 52 to 65 % of the cycles; the two waves per
+// SIMD wait 27 to 35 % of theirs, for copies issued one super-block before and the
+// barrier of each step, hardly for LDS; the matrix cores are 10 to 21 % busy.  T = 1024 at
+// H = 4096 reads 3.9 GB past the L2s for gate + up, 5.4 TB/s.  us per launch: T = 1024 at H = 4096, gate + up
 // 894 (min lanes over the quants) -> 723; T = 512 at the 30B shape, Zipf-skewed,
 // mean of gate + up and down 129 -> 120.
 //

@@ -48,7 +48,8 @@ typedef float q80_f16 __attribute__((ext_vector_type(16)));
 // row's 16-byte chunk c at position c ^ 8: 16 rows read at one chunk hit distinct banks.
 //
 // Bound: VALU issue (about 46 instructions per tile and block against 64 cycles of
-// matrix core) and the weights' bytes (T = 251: 430 MB of gate and up).  The GEMV alone
+// matrix core), 77 % of the cycles of gate and up at T = 251 (down 68 %), with waves waiting
+// 36 % (45 %) of theirs; 607 MB read past the L2s there, of 430 MB of weights.  The GEMV alone
 // took 1.8 ms per launch at T = 251, the layer 2509 us.
 constexpr uint32_t Q80_WS = 272;     // LDS bytes of a staged weight row (8 blocks)
 constexpr uint32_t Q80_HS = 1040;    // LDS bytes of an activation copy instruction (rows 2 i, 2 i + 1, pad)

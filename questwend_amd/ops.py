@@ -48,7 +48,8 @@ def set_mfma_form(form: int) -> int:
     chains (bit-identical), MFMA_BLOCK_SUM adds exact integer block sums in one
     fp32 chain per output, MFMA_AUTO is exact except for the down projections
     of the layer entry points.  The default is MFMA_EXACT; the other two are
-    opt-in speed settings whose outputs drift from ggml's in the last bits.
+    opt-in settings, faster for large experts, whose outputs drift from ggml's in
+    the last bits.
     Returns the previous setting."""
     prev = int(lib().qwmoe_get_mfma_form())
     check(lib().qwmoe_set_mfma_form(int(form)), "set_mfma_form")
