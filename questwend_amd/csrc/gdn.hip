@@ -141,9 +141,10 @@ __global__ void __launch_bounds__(GS) k_gdn_prep(GdnArgs a) {
 // gives the bits that calls of its parts give (decode steps and a verify batch agree).
 // q, k (the key head), v (the workgroup's rows), beta and exp(g) sit in LDS.
 //
-// Bound: the chain of the two row reductions per token, with a wave per SIMD (0.34 us a
-// token).  Four tokens per step, whose reductions are independent, take 0.25 us a token
-// but round each token by its place in the call.
+// Bound: the chain of the two row reductions per token, with a wave per SIMD.  Four tokens
+// per step, whose reductions are independent, gain little at this length and round each
+// token by its place in the call (us per call, H_v = 32, token by token / four per step:
+// 49.8 / 51.0 at T = 1, 71.0 / 71.4 at 4, 81.2 / 81.3 at 16, 86.3 / 85.3 at 31).
 typedef float fx4 __attribute__((ext_vector_type(4)));   // (arrays of it stay in registers)
 constexpr int GTB = 32;   // tokens staged
 __global__ void __launch_bounds__(256) k_gdn_delta(GdnArgs a) {
